@@ -170,7 +170,7 @@ typedef struct misohip_work {
 
 /* Context: device ordinal and the HIP stream every call is ordered on
  * (NULL = the null stream).  Creates no stream at creation; the first
- * misohip_rt_solve with both multi-plane and plane rays creates one more
+ * misohip_rt_solve with rays along more than one sweep axis creates two more
  * (default priority) for the multi-plane sweeps, forked from and joined back
  * to the context's stream with events inside each iteration, and
  * misohip_destroy frees it. */
@@ -314,9 +314,9 @@ int misohip_update_noalloc(misohip_ctx *ctx, const misohip_grid *g, misohip_dtyp
  * on x and on y) keeps its field of rint y-fastest, index
  * ((k * i_total + i) * j_total + j), so the planes it sweeps are contiguous;
  * misohip_rt_ray_layout names those rays.  0: every ray x-fastest.
- * sweep_planes 2..16: a ray whose shorter transverse axis (c) has at most
- * 32 lattice nodes (the x and y rays of a thin slab) advances that many
- * planes per launch; 0 or 1: one launch per plane for every ray.  Results
+ * sweep_planes 2..16: a ray with two real transverse axes advances
+ * min(sweep_planes, 8) planes per launch; 0 or 1: one launch per plane for
+ * every ray.  Results
  * are the same bits under every setting of both. */
 typedef struct misohip_rt_config {
   int num_rays;

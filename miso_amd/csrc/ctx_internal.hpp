@@ -25,10 +25,10 @@ struct misohip_ctx {
   double *rt_kap_y = nullptr, *rt_src_y = nullptr;
   size_t rt_cells = 0;
   unsigned *rt_parts = nullptr;  // the RT change-reduction slots
-  // a second stream (default priority) and two events: an RT solve sweeps
-  // its multi-plane rays there while the plane rays sweep on `stream`
-  hipStream_t rt_side = nullptr;
-  hipEvent_t rt_fork = nullptr, rt_join = nullptr;
+  // two more streams (default priority) and their events: an RT solve's
+  // sweeps along different axes run side by side
+  hipStream_t rt_side[2] = {nullptr, nullptr};
+  hipEvent_t rt_fork = nullptr, rt_join[2] = {nullptr, nullptr};
   // two more streams (default priority) for the AV sweeps run as a pipeline
   // over z slabs (the x-y walk on the first, the z walk on the second), and
   // its events: one per slab (16), the fork and the two joins

@@ -62,7 +62,7 @@ __device__ __forceinline__ float reg_copy(float x) {
 // wave_shr:1 (0x138) gives lane i the value of lane i-1, wave_shl:1 (0x130)
 // that of lane i+1; the end lanes, which no caller stores, get 0.
 template <int CTRL> __device__ __forceinline__ int dpp_move(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false);
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true);
 }
 template <int CTRL> __device__ __forceinline__ float dpp_move(float v) {
   return __int_as_float(dpp_move<CTRL>(__float_as_int(v)));

@@ -78,13 +78,33 @@ hipError_t launch_rt_sweep_plane(hipStream_t, double *, const double *, const do
                                  const double *, const double *, const RtRays &, int, int, long,
                                  int, unsigned *);
 hipError_t launch_rt_transpose_xy(hipStream_t, const double *, double *, int, int, int);
-// several planes per launch for rays whose c axis has at most RT_MULTI_ROWS - 1 nodes
-constexpr int RT_MULTI_COLS = 32;  // b nodes a workgroup owns
-constexpr int RT_MULTI_PLANES = 16;
-constexpr int RT_MULTI_ROWS = 33;
-hipError_t launch_rt_sweep_multi(hipStream_t, double *, const double *, const double *,
+// The patched sweep: P <= RT_TILE_PLANES planes per launch (4, 6, 8 and 10
+// planes: 17.4, 17.0, 17.0, 17.3 ms for a radiative step of 256^3 and 9.2,
+// 8.6, 8.3, 8.5 ms for a cold solve of 211 x 150 x 187), in patches of 64 x
+// RT_ROWS nodes; of 64 x RT_ROWS_SMALL where a chain's launch would have
+// fewer than RT_FEW workgroups, so that a thin slab's x and y rays reach the
+// CUs that whole patches leave idle (slab solve of 384^2 x 27: 4.44 -> 3.83
+// ms; at 256^3, where the chip is full either way, the short patches'
+// repeated rows make 19.1 ms of 17.0).
+// The first patch of an axis starts on the upwind boundary and owns size - 1
+// nodes, the others start P nodes before the size - P they own.
+constexpr int RT_TILE_PLANES = 8;
+constexpr int RT_ROWS = 32, RT_ROWS_SMALL = 16, RT_FEW = 128;
+__host__ __device__ inline int rt_patches(int n, int size, int P) {
+  return n < size ? 1 : 1 + (n - (size - 1) + size - P - 1) / (size - P);
+}
+__host__ __device__ inline int rt_patch_first(int a, int size, int P) {
+  return a == 0 ? -1 : size - 1 + (a - 1) * (size - P) - P;
+}
+// the patches of a launch, by groups of `same` rays with the same planes:
+// group g has patches start[g] .. start[g + 1] - 1, per_xcd go to each XCD
+struct RtPatches {
+  int same, groups, per_xcd;
+  int start[25];
+};
+hipError_t launch_rt_sweep_tiles(hipStream_t, double *, const double *, const double *,
                                  const double *, const double *, const RtRays &, int, int, int,
-                                 long, int, unsigned *);
+                                 int, long, unsigned *);
 hipError_t launch_rt_halo(hipStream_t, double *, int, int, int, int, int, int, unsigned, unsigned,
                           long, int);
 hipError_t launch_rt_face(hipStream_t, double *, const double *, int, int, int, int, int, int,

@@ -25,7 +25,11 @@ __device__ __forceinline__ double rt_integrate(double Iu, double Su, double Sd, 
   const double eps_tau = 1.e-4;
   const double exp_dtau = exp(-dtau);
   const double u0 = 1.0 - exp_dtau;
-  const double u1 = dtau < eps_tau ? 0.5 * dtau : 1.0 - (u0 / dtau);
+  // the quotient is formed for every node (and dropped where dtau is small):
+  // without a branch the nodes of a thread interleave
+  double quot = u0 / dtau;
+  asm("" : "+v"(quot));
+  const double u1 = dtau < eps_tau ? 0.5 * dtau : 1.0 - quot;
   return Iu * exp_dtau + (u0 - u1) * Su + u1 * Sd;
 }
 
@@ -97,137 +101,187 @@ __global__ __launch_bounds__(256) void rt_sweep_plane_kernel(double *__restrict_
   rt_block_max(best, part);
 }
 
-// Planes p0 .. p0 + P - 1 of every ray of `rays` in one launch, for rays
-// whose c axis is short (nc < RT_MULTI_ROWS; a thin slab's x and y rays).
-// Node coordinates are mirrored so that upwind is always one step back:
-// u = ib (sb > 0) or nb - 1 - ib, likewise v.  A workgroup owns the
-// RT_MULTI_COLS columns u in [U0, U0 + W) of a ray over the whole c range,
-// and computes plane by plane the cone u in [U0 - P, U0 + W) of nodes
-// that its last plane depends on; the plane is kept in LDS, column u = -1
-// and row v = -1 (the upwind boundary nodes, which the sweep never writes)
-// are read from memory.  Every node is computed by rt_node from the same
-// values as in rt_sweep_plane_kernel, so the results are the same bits;
-// cone nodes outside the owned columns are recomputed, not stored, and the
-// cone's stale edge (u below U0 - P + s + 1 at step s) never reaches them.
-constexpr int RT_MULTI_THREADS = 1024;
+// Planes p0 .. p0 + P - 1 of every ray of `rays` in one launch.  Node
+// coordinates are mirrored so that upwind is always one step back: u = ib
+// (sb > 0) or nb - 1 - ib, likewise v.  A workgroup takes a patch of 64
+// columns x W R rows of one ray (W waves): lane l of wave w holds column
+// u0 + l of the rows v0 + w R ... + R - 1, the plane before in registers;
+// u - 1 comes by a DPP lane shift, v - 1 from the row above (the last row of
+// the wave before, through LDS).  The patch's first column and row are the
+// upwind boundary (u = -1, v = -1: loaded at every plane, the sweep never
+// writes it) or, in the patches after the first, P columns and rows of the
+// neighbouring patch, computed again: step s leaves the first s of them
+// stale, so the columns and rows from P on are right after P planes, and
+// only those are stored.  No workgroup reads what another one of the launch
+// writes.
+// Three register sets hold the plane before, the current plane's kappa, S
+// and old intensities, and the next plane's, in flight meanwhile.
+// The four rays that go the same way along the planes read the same kappa
+// and S: their workgroups of one patch sit on one XCD, next to each other in
+// launch order, so that HBM is read once for the four; the patches of an XCD
+// are neighbours.
+// rt_node forms each value from the same operands as rt_sweep_plane_kernel:
+// the same bits.
+// Bound by VALU issue (84 instructions a node and 1.4 x the nodes, for the
+// repeated columns and rows) and, at the large sizes, HBM: a launch per plane
+// read the plane before again, kappa and S once per ray, and moved 41 bytes
+// a node and ray; this 26.  At 256^3 an iteration's sweeps take 3.0 ms of
+// 5.2, radiative step 23.4 -> 17.0 ms, cold solve of 211 x 150 x 187 14.2 ->
+// 8.2 ms.  (Tiles marched in wavefront order, which repeat nothing, read
+// kappa and S once per ray and start and end with an idle chip: 19.4 and
+// 10.6 ms.)
+template <int R> struct RtTilePlane {
+  double i[R], k[R], s[R];  // own rows; i: before the sweep, then after it
+  double ih, kh, sh;        // the row above them
+};
 
-__global__ __launch_bounds__(RT_MULTI_THREADS) void rt_sweep_multi_kernel(double *__restrict__ I,
-                                                             const double *__restrict__ kap_x,
-                                                             const double *__restrict__ S_x,
-                                                             const double *__restrict__ kap_y,
-                                                             const double *__restrict__ S_y,
-                                                             RtRays rays, int p0, int P,
-                                                             long ray_stride, unsigned *part) {
-  constexpr int W = RT_MULTI_COLS, X = RT_MULTI_COLS + RT_MULTI_PLANES, ROWS = RT_MULTI_ROWS;
-  constexpr int NT = RT_MULTI_THREADS, CPT = (X * ROWS + NT - 1) / NT;
-  __shared__ double Il[ROWS][X], Kl[ROWS][X], Sl[ROWS][X];
-  const RtRay &R = rays.r[blockIdx.y];
-  const int U0 = blockIdx.x * W;
-  // uniform over the workgroup
-  if (p0 >= R.nplanes || U0 >= R.nb || R.nc + 1 > ROWS || P < 1 || P > RT_MULTI_PLANES) return;
-  const double *__restrict__ kap = R.tr ? kap_y : kap_x;
-  const double *__restrict__ S = R.tr ? S_y : S_x;
-  double *Ir = I + ray_stride * R.id;
-  const int ext = W + P, ncell = ext * (R.nc + 1);
-  const int pend = min(p0 + P, R.nplanes);
-  // per cell: memory index at plane 0, role (0 none, 1 boundary, read every
-  // plane; 2 computed; 3 computed and owned, its value before the sweep read
-  // for the change; 4 the cone's far edge e = 0,
-  // read for the plane before p0 only: never valid after it, and its node
-  // may be written by another workgroup meanwhile), LDS position
-  int off[CPT], role[CPT], ce[CPT], cr[CPT];
-#pragma unroll
-  for (int q = 0; q < CPT; ++q) {
-    const int idx = threadIdx.x + q * NT;
-    const int e = idx % ext, r = idx / ext;
-    const int u = U0 - P + e, v = r - 1;
-    ce[q] = e;
-    cr[q] = r;
-    role[q] = 0;
-    off[q] = 0;
-    if (idx >= ncell || u < -1 || u >= R.nb) continue;
-    const int ib = R.sb > 0 ? u : R.nb - 1 - u;
-    const int ic = R.sc > 0 ? v : R.nc - 1 - v;
-    off[q] = R.start + ib * R.db + ic * R.dc;
-    if (u == -1 || v == -1) role[q] = 1;
-    else if (e == 0) role[q] = 4;
-    else role[q] = (u >= U0 && u < U0 + W) ? 3 : 2;
-  }
-  // the plane before p0
-#pragma unroll
-  for (int q = 0; q < CPT; ++q)
-    if (role[q]) {
-      const int c = off[q] + (p0 - 1) * R.da;
-      Il[cr[q]][ce[q]] = Ir[c];
-      Kl[cr[q]][ce[q]] = kap[c];
-      Sl[cr[q]][ce[q]] = S[c];
-    }
-  // kappa, S and the boundary (role 1) or before-sweep (role 3) intensity of
-  // a plane's cells; loads run two planes ahead of the computation
-  auto load = [&](int p, double *k, double *s, double *b) {
-#pragma unroll
-    for (int q = 0; q < CPT; ++q) {
-      k[q] = s[q] = b[q] = 0.0;
-      if (p < pend && role[q] && role[q] < 4) {
-        const int c = off[q] + p * R.da;
-        k[q] = kap[c];
-        s[q] = S[c];
-        if (role[q] == 1 || role[q] == 3) b[q] = Ir[c];
-      }
-    }
+template <int R, int W>
+__global__ __launch_bounds__(64 * W) void rt_sweep_tile_kernel(
+    double *__restrict__ I, const double *__restrict__ kap_x, const double *__restrict__ S_x,
+    const double *__restrict__ kap_y, const double *__restrict__ S_y, RtRays rays, RtPatches pt,
+    int p0, int P, long ray_stride, unsigned *part) {
+  constexpr int NR = W * R;
+  __shared__ double edge[2][W][64];
+  // blocks of one XCD (blockIdx % 8): consecutive patches, each for the
+  // pt.same rays of its group in turn
+  const int xcd = blockIdx.x % 8, idx = blockIdx.x / 8;
+  const int patch = xcd * pt.per_xcd + idx / pt.same;
+  int g = 0;
+  while (g < pt.groups && patch >= pt.start[g + 1]) ++g;
+  if (g == pt.groups) return;  // uniform over the workgroup, as are all below
+  const RtRay &Q = rays.r[g * pt.same + idx % pt.same];
+  const int na = rt_patches(Q.nb, 64, P);
+  const int a = (patch - pt.start[g]) % na, b = (patch - pt.start[g]) / na;
+  if (p0 >= Q.nplanes || b >= rt_patches(Q.nc, NR, P)) return;
+  const double *__restrict__ kap = Q.tr ? kap_y : kap_x;
+  const double *__restrict__ S = Q.tr ? S_y : S_x;
+  double *Ir = I + ray_stride * Q.id;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int pend = min(p0 + P, Q.nplanes);
+  const int u0 = rt_patch_first(a, 64, P), v0 = rt_patch_first(b, NR, P);
+  const int u_own = a ? u0 + P : 0, v_own = b ? v0 + P : 0;
+  // columns and rows past the ray's end load its last ones and store nothing
+  const int u = u0 + lane, uc = min(u, Q.nb - 1);
+  const bool own = u >= u_own && u < Q.nb, bound = u < 0;
+  // a node's address: a row's first node (ib = -1), uniform over the wave, and
+  // the lane's byte offset from it (0 .. 8 (nb + 1) db, below 4 GiB: the host
+  // checks that)
+  auto byte_of = [&](int ub) {
+    return (unsigned)((Q.sb > 0 ? ub + 1 : Q.nb - ub) * Q.db) * 8u;
   };
-  double kc[CPT], sc[CPT], bnd[CPT], k1[CPT], s1[CPT], b1[CPT];
-  load(p0, kc, sc, bnd);
-  load(p0 + 1, k1, s1, b1);
-  __syncthreads();
+  // old intensities are of use in owned nodes and on the boundary: in a patch
+  // without boundary rows the columns that are not owned load the nearest
+  // owned one, in one without boundary columns the rows likewise
+  const unsigned col = byte_of(uc);
+  const unsigned col_i = byte_of(min(max(u, a && b ? u_own : -1), Q.nb - 1));
+  auto row = [&](int v) {
+    v = max(min(v, Q.nc - 1), -1);
+    return Q.start - Q.db + (Q.sc > 0 ? v : Q.nc - 1 - v) * Q.dc;
+  };
+  const int vw = v0 + w * R;
+  int off[R], off_i[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    off[r] = row(vw + r);
+    off_i[r] = row(max(vw + r, a && b ? v_own : -1));
+  }
+  const int offh = row(vw - 1);
+  // element q of the lane: the address as a scalar base (pinned, or the
+  // compiler would fold the lane's part into it) plus 32 bits
+  auto at = [](const double *q, unsigned byte) {
+    unsigned long base = reinterpret_cast<unsigned long>(q);
+    asm("" : "+s"(base));
+    asm("" : "+v"(byte));
+    return reinterpret_cast<__attribute__((address_space(1))) double *>(base + byte);
+  };
+  auto load = [&](RtTilePlane<R> &x, int p, const int *oi, unsigned ci) {
+    const int d = p * Q.da;
+    x.kh = *at(kap + (offh + d), col);
+    x.sh = *at(S + (offh + d), col);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      x.k[r] = *at(kap + (off[r] + d), col);
+      x.s[r] = *at(S + (off[r] + d), col);
+      x.i[r] = *at(Ir + (oi[r] + d), ci);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // in flight before the plane is computed
+  };
+  auto exchange = [&](RtTilePlane<R> &x, int p) {
+    edge[p & 1][w][lane] = x.i[R - 1];
+    __syncthreads();
+    x.ih = edge[p & 1][w ? w - 1 : 0][lane];
+  };
+  RtTilePlane<R> x0, x1, x2;
+  load(x0, p0 - 1, off, col);
+  load(x1, p0, off_i, col_i);
+  exchange(x0, p0 - 1);
   unsigned best = 0u;
-  for (int p = p0; p < pend; ++p) {
-    double kn[CPT], sn[CPT], bn[CPT];
-    load(p + 2, kn, sn, bn);
-    double in[CPT];
+  auto step = [&](const RtTilePlane<R> &b4, RtTilePlane<R> &x, RtTilePlane<R> &nx, int p) {
+    load(nx, min(p + 1, pend - 1), off_i, col_i);
+    double I01 = b4.ih, K01 = b4.kh, S01 = b4.sh;
+    double I11 = lane_up(I01), K11 = lane_up(K01), S11 = lane_up(S01);
+    double now[R];
 #pragma unroll
-    for (int q = 0; q < CPT; ++q) {
-      in[q] = bnd[q];
-      if (role[q] == 2 || role[q] == 3) {
-        const int r = cr[q], e = ce[q];
-        in[q] = rt_node(R, Il[r][e], Il[r][e - 1], Il[r - 1][e], Il[r - 1][e - 1], Sl[r][e],
-                        Sl[r][e - 1], Sl[r - 1][e], Sl[r - 1][e - 1], Kl[r][e], Kl[r][e - 1],
-                        Kl[r - 1][e], Kl[r - 1][e - 1], kc[q], sc[q]);
-      }
+    for (int r = 0; r < R; ++r) {
+      const double I00 = b4.i[r], K00 = b4.k[r], S00 = b4.s[r];
+      const double I10 = lane_up(I00), K10 = lane_up(K00), S10 = lane_up(S00);
+      now[r] = rt_node(Q, I00, I10, I01, I11, S00, S10, S01, S11, K00, K10, K01, K11, x.k[r],
+                       x.s[r]);
+      I01 = I00; K01 = K00; S01 = S00;
+      I11 = I10; K11 = K10; S11 = S10;
     }
-    __syncthreads();
+    if (own) {
 #pragma unroll
-    for (int q = 0; q < CPT; ++q)
-      if (role[q] && role[q] < 4) {
-        Il[cr[q]][ce[q]] = in[q];
-        Kl[cr[q]][ce[q]] = kc[q];
-        Sl[cr[q]][ce[q]] = sc[q];
-        if (role[q] == 3) {
-          best = max(best, rt_change(in[q], bnd[q]));
-          Ir[off[q] + p * R.da] = in[q];
+      for (int r = 0; r < R; ++r)
+        if (vw + r >= v_own && vw + r < Q.nc) {
+          best = max(best, rt_change(now[r], x.i[r]));
+          *at(Ir + (off[r] + p * Q.da), col) = now[r];
         }
-      }
-#pragma unroll
-    for (int q = 0; q < CPT; ++q) {
-      kc[q] = k1[q];
-      sc[q] = s1[q];
-      bnd[q] = b1[q];
-      k1[q] = kn[q];
-      s1[q] = sn[q];
-      b1[q] = bn[q];
     }
-    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) x.i[r] = bound || vw + r < 0 ? x.i[r] : now[r];
+    exchange(x, p);
+  };
+  for (int p = p0;;) {
+    step(x0, x1, x2, p);
+    if (++p >= pend) break;
+    step(x1, x2, x0, p);
+    if (++p >= pend) break;
+    step(x2, x0, x1, p);
+    if (++p >= pend) break;
   }
   rt_block_max(best, part);
 }
 
-hipError_t launch_rt_sweep_multi(hipStream_t st, double *I, const double *kap, const double *S,
+constexpr int RT_TILE_R = 4;  // rows a wave holds (2: 18.3 ms for 17.0, 8: 22.8)
+
+hipError_t launch_rt_sweep_tiles(hipStream_t st, double *I, const double *kap, const double *S,
                                  const double *kap_y, const double *S_y, const RtRays &rays,
-                                 int nrays, int p0, int P, long ray_stride, int max_nb,
+                                 int nrays, int p0, int P, int rows, long ray_stride,
                                  unsigned *part) {
-  dim3 grid((max_nb + RT_MULTI_COLS - 1) / RT_MULTI_COLS, nrays);
-  hipLaunchKernelGGL(rt_sweep_multi_kernel, grid, dim3(RT_MULTI_THREADS), 0, st, I, kap, S, kap_y,
-                     S_y, rays, p0, P, ray_stride, part);
+  RtPatches pt;
+  pt.same = nrays % 4 == 0 ? 4 : 1;
+  pt.groups = nrays / pt.same;
+  pt.start[0] = 0;
+  for (int g = 0; g < pt.groups; ++g) {
+    int n = 0;
+    for (int m = 0; m < pt.same; ++m) {
+      const RtRay &Q = rays.r[g * pt.same + m];
+      if (p0 < Q.nplanes) n = max(n, rt_patches(Q.nb, 64, P) * rt_patches(Q.nc, rows, P));
+    }
+    pt.start[g + 1] = pt.start[g] + n;
+  }
+  if (!pt.start[pt.groups]) return hipSuccess;
+  pt.per_xcd = (pt.start[pt.groups] + 7) / 8;
+  const dim3 grid(8 * pt.per_xcd * pt.same);
+  if (rows == RT_ROWS_SMALL)
+    hipLaunchKernelGGL((rt_sweep_tile_kernel<RT_TILE_R, RT_ROWS_SMALL / RT_TILE_R>), grid,
+                       dim3(64 * RT_ROWS_SMALL / RT_TILE_R), 0, st, I, kap, S, kap_y, S_y, rays, pt, p0, P,
+                       ray_stride, part);
+  else
+    hipLaunchKernelGGL((rt_sweep_tile_kernel<RT_TILE_R, RT_ROWS / RT_TILE_R>), grid,
+                       dim3(64 * RT_ROWS / RT_TILE_R), 0, st, I, kap, S, kap_y, S_y, rays, pt, p0, P,
+                       ray_stride, part);
   return hipGetLastError();
 }
 

@@ -179,7 +179,7 @@ int check_rt(const misohip_grid *g, const misohip_rt_config *rt) {
   if (!g || !rt) return MISOHIP_E_ARG;
   if (rt->num_rays != 24 && rt->num_rays != 1) return MISOHIP_E_ARG;
   if (rt->max_iters < 1) return MISOHIP_E_ARG;
-  if (rt->sweep_planes < 0 || rt->sweep_planes > RT_MULTI_PLANES) return MISOHIP_E_ARG;
+  if (rt->sweep_planes < 0 || rt->sweep_planes > 16) return MISOHIP_E_ARG;
   const double n = (double)g->i_total * g->j_total * g->k_total;
   if (n >= 2147483647.0) return MISOHIP_E_RANGE;  // int indices within one ray
   if (!g->dx || !g->dy || !g->dz) return MISOHIP_E_ARG;
@@ -235,21 +235,41 @@ int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_c
     kap_y = ctx->rt_kap_y;
     src_y = ctx->rt_src_y;
   }
-  // Rays with a short c axis advance several planes per launch
-  // (rt_sweep_multi_kernel); the others go one plane per launch.
-  const int P = rt->sweep_planes;
-  RtRays mrays;
-  int nm = 0, m_planes = 0, m_nb = 0;
+  // Rays with two real transverse axes advance P planes per launch, patch by
+  // patch (rt_sweep_tile_kernel); the others one plane per launch.
+  const int P = std::min(rt->sweep_planes, RT_TILE_PLANES);
+  std::vector<RtRay> trays;
   std::vector<int> plane_rays;
   for (int n = 0; n < su.nrays; ++n) {
     const RtRay &R = su.rays.r[n];
-    if (P >= 2 && R.sb != 0 && R.sc != 0 && R.ua == R.da && R.nc + 1 <= RT_MULTI_ROWS) {
-      mrays.r[nm++] = R;
-      m_planes = std::max(m_planes, R.nplanes);
-      m_nb = std::max(m_nb, R.nb);
-    } else {
+    if (P >= 2 && R.sb != 0 && R.sc != 0 && R.ua == R.da && (R.nb + 2L) * R.db < 1L << 29)
+      trays.push_back(R);
+    else
       plane_rays.push_back(n);
-    }
+  }
+  // Rays that sweep the same planes next to each other (the 24 directions
+  // have every transverse sign: fours), and one chain of launches per
+  // sweep axis: the chains touch disjoint intensities and meet only in the
+  // change maximum (atomic), so they run side by side on three streams, one
+  // filling the CUs that the last workgroups of another's launch leave idle.
+  std::stable_sort(trays.begin(), trays.end(), [](const RtRay &x, const RtRay &y) {
+    const int ax = std::abs(x.da), ay = std::abs(y.da);
+    return x.tr != y.tr ? x.tr < y.tr : ax != ay ? ax < ay : x.da < y.da;
+  });
+  struct Chain {
+    RtRays rays;
+    int n = 0, planes = 0;
+    long blocks = 0;  // workgroups a launch in patches of RT_ROWS rows
+  };
+  std::vector<Chain> chains;
+  for (const RtRay &R : trays) {
+    if (chains.empty() || chains.back().rays.r[0].tr != R.tr ||
+        std::abs(chains.back().rays.r[0].da) != std::abs(R.da))
+      chains.emplace_back();
+    Chain &ch = chains.back();
+    ch.rays.r[ch.n++] = R;
+    ch.planes = std::max(ch.planes, R.nplanes);
+    ch.blocks += (long)rt_patches(R.nb, 64, P) * rt_patches(R.nc, RT_ROWS, P);
   }
   // Sweep phases: plane ranges over which the set of rays that still have
   // planes is constant; each phase launches only those rays, sized for
@@ -290,16 +310,14 @@ int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_c
   uf.It = It;
   uf.Jt = Jt;
   if (!ctx->rt_parts) MISOHIP_TRY(hipMalloc(&ctx->rt_parts, sizeof(unsigned) * 32 * RT_PARTS));
-  // The multi-plane rays and the plane rays touch disjoint intensities and
-  // meet only in the change maximum (atomic), so with both present the
-  // multi-plane sweeps run on a second stream beside the plane sweeps.
-  const bool split = nm > 0 && !phases.empty();
-  if (split && !ctx->rt_side) {
-    MISOHIP_TRY(hipStreamCreateWithFlags(&ctx->rt_side, hipStreamNonBlocking));
+  const int nside = std::min(2, std::max(0, (int)chains.size() - 1));
+  for (int i = 0; i < nside; ++i)
+    if (!ctx->rt_side[i]) {
+      MISOHIP_TRY(hipStreamCreateWithFlags(&ctx->rt_side[i], hipStreamNonBlocking));
+      MISOHIP_TRY(hipEventCreateWithFlags(&ctx->rt_join[i], hipEventDisableTiming));
+    }
+  if (nside > 0 && !ctx->rt_fork)
     MISOHIP_TRY(hipEventCreateWithFlags(&ctx->rt_fork, hipEventDisableTiming));
-    MISOHIP_TRY(hipEventCreateWithFlags(&ctx->rt_join, hipEventDisableTiming));
-  }
-  hipStream_t mst = split ? ctx->rt_side : ctx->stream;
   unsigned *parts = ctx->rt_parts;
   MISOHIP_TRY(launch_rt_parts_reduce(ctx->stream, parts, nullptr, true));
   int it = 0;
@@ -340,20 +358,30 @@ int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_c
                                        su.nrays));
           }
         }
-      if (split) {
-        MISOHIP_TRY(hipEventRecord(ctx->rt_fork, ctx->stream));
-        MISOHIP_TRY(hipStreamWaitEvent(ctx->rt_side, ctx->rt_fork, 0));
+      if (nside > 0) MISOHIP_TRY(hipEventRecord(ctx->rt_fork, ctx->stream));
+      for (int i = 0; i < nside; ++i)
+        MISOHIP_TRY(hipStreamWaitEvent(ctx->rt_side[i], ctx->rt_fork, 0));
+      int left = (int)chains.size();
+      for (int p0 = 0; left; p0 += P) {
+        left = 0;
+        for (size_t c = 0; c < chains.size(); ++c) {
+          const Chain &ch = chains[c];
+          if (p0 >= ch.planes) continue;
+          const int i = (int)c % (nside + 1);
+          MISOHIP_TRY(launch_rt_sweep_tiles(i ? ctx->rt_side[i - 1] : ctx->stream, I, kap, src,
+                                            kap_y, src_y, ch.rays, ch.n, p0, P,
+                                            ch.blocks < RT_FEW ? RT_ROWS_SMALL : RT_ROWS,
+                                            su.ray_stride, parts));
+          if (p0 + P < ch.planes) ++left;
+        }
       }
-      for (int p0 = 0; p0 < m_planes; p0 += P)
-        MISOHIP_TRY(launch_rt_sweep_multi(mst, I, kap, src, kap_y, src_y, mrays, nm, p0, P,
-                                          su.ray_stride, m_nb, parts));
       for (const Phase &ph : phases)
         for (int p = ph.p0; p < ph.p1; ++p)
           MISOHIP_TRY(launch_rt_sweep_plane(ctx->stream, I, kap, src, kap_y, src_y, ph.rays,
                                             ph.n, p, su.ray_stride, ph.max_nodes, parts));
-      if (split) {
-        MISOHIP_TRY(hipEventRecord(ctx->rt_join, ctx->rt_side));
-        MISOHIP_TRY(hipStreamWaitEvent(ctx->stream, ctx->rt_join, 0));
+      for (int i = 0; i < nside; ++i) {
+        MISOHIP_TRY(hipEventRecord(ctx->rt_join[i], ctx->rt_side[i]));
+        MISOHIP_TRY(hipStreamWaitEvent(ctx->stream, ctx->rt_join[i], 0));
       }
       MISOHIP_TRY(launch_rt_faces(ctx->stream, I, old, false, uf, su.ray_stride, su.nrays, parts));
       MISOHIP_TRY(launch_rt_parts_reduce(ctx->stream, parts, ctx->d_slot + 1, false));
