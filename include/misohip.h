@@ -339,9 +339,8 @@ int misohip_rt_quadrature(int num_rays, double *w, double *mu_x, double *mu_y, d
 /* RT::solve: iterate halo exchange, boundary, sweep until the float-
  * narrowed max change is below tolerance (rt_host.hpp:632-651).  Writes the
  * iteration count and the last max change; synchronises once per
- * iteration.  rint_old is the solver's scratch: the change is taken inside
- * the sweep, and rint_old keeps only each ray's upwind lattice faces as
- * they were at the start of the last iteration. */
+ * iteration.  rint_old is scratch that the present solver leaves alone: the
+ * change is taken where the intensities are written. */
 int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_config *rt,
                      const void *kappa, const void *S, void *rint, void *rint_old,
                      int *iters, double *max_diff);

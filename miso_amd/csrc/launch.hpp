@@ -65,12 +65,15 @@ struct RtRays {
   RtRay r[24];
 };
 
-// lattice (lo, n per axis), ray directions and layouts for rt_faces_kernel
-struct RtFaces {
-  int lo[3], n[3];
-  unsigned pos[3];  // bit r: ray r goes + along the axis
-  unsigned tr;      // bit r: ray r is kept y-fastest
-  int It, Jt;
+// the lattice's ends, the arrays' extents, ray directions and layouts and the
+// boundaries for rt_incoming_kernel
+struct RtIncoming {
+  int lo[3], hi[3], tot[3];
+  int periodic[3], kind[6];
+  double value[6];
+  unsigned pos[3];     // bit r: ray r goes + along the axis
+  unsigned moving[3];  // bit r: ray r has a component along it
+  unsigned tr;         // bit r: ray r is kept y-fastest
 };
 constexpr int RT_PARTS = 64;  // change-reduction slots, 32 words apart
 
@@ -81,15 +84,17 @@ hipError_t launch_rt_transpose_xy(hipStream_t, const double *, double *, int, in
 // The patched sweep: P <= RT_TILE_PLANES planes per launch (4, 6, 8 and 10
 // planes: 17.4, 17.0, 17.0, 17.3 ms for a radiative step of 256^3 and 9.2,
 // 8.6, 8.3, 8.5 ms for a cold solve of 211 x 150 x 187), in patches of 64 x
-// RT_ROWS nodes; of 64 x RT_ROWS_SMALL where a chain's launch would have
-// fewer than RT_FEW workgroups, so that a thin slab's x and y rays reach the
-// CUs that whole patches leave idle (slab solve of 384^2 x 27: 4.44 -> 3.83
-// ms; at 256^3, where the chip is full either way, the short patches'
-// repeated rows make 19.1 ms of 17.0).
+// RT_ROWS nodes (48 rows: 17.0 ms for 16.0 and 8.2 for 7.6; 36 of three a wave
+// 16.8 and 8.3); of 64 x RT_ROWS_SMALL where an axis' launch would have fewer
+// than RT_FEW workgroups, so that a thin slab's x and y rays, two patches
+// high, reach the CUs that whole patches leave idle (slab solve of 384^2 x
+// 27: 4.44 -> 3.56 ms; 16 rows, three patches high, 3.68; at 256^3, where the
+// chip is full either way, the short patches' repeated rows make 19.1 ms of
+// 17.0; a limit of 256 sends a 211 x 150 x 187 box there: 8.1 ms for 7.6).
 // The first patch of an axis starts on the upwind boundary and owns size - 1
 // nodes, the others start P nodes before the size - P they own.
 constexpr int RT_TILE_PLANES = 8;
-constexpr int RT_ROWS = 32, RT_ROWS_SMALL = 16, RT_FEW = 128;
+constexpr int RT_ROWS = 32, RT_ROWS_SMALL = 20, RT_FEW = 128;
 __host__ __device__ inline int rt_patches(int n, int size, int P) {
   return n < size ? 1 : 1 + (n - (size - 1) + size - P - 1) / (size - P);
 }
@@ -105,12 +110,8 @@ struct RtPatches {
 hipError_t launch_rt_sweep_tiles(hipStream_t, double *, const double *, const double *,
                                  const double *, const double *, const RtRays &, int, int, int,
                                  int, long, unsigned *);
-hipError_t launch_rt_halo(hipStream_t, double *, int, int, int, int, int, int, unsigned, unsigned,
-                          long, int);
-hipError_t launch_rt_face(hipStream_t, double *, const double *, int, int, int, int, int, int,
-                          int, int, int, double, unsigned, long, int);
-hipError_t launch_rt_faces(hipStream_t, const double *, double *, bool, const RtFaces &, long, int,
-                           unsigned *);
+hipError_t launch_rt_incoming(hipStream_t, double *, const double *, const double *,
+                              const RtIncoming &, long, int, unsigned *);
 hipError_t launch_rt_parts_reduce(hipStream_t, unsigned *, unsigned *, bool);
 hipError_t launch_rt_qrad(hipStream_t, const double *, const double *, const double *, double *,
                           const int[3], const int[3], int, int, long, int, unsigned,

@@ -51,8 +51,8 @@ __device__ __forceinline__ double rt_node(const RtRay &R, double I00, double I10
 // (rt_host.hpp:612-629); positive floats order like their bit patterns.
 // Every lattice node of a ray is either swept (exactly once per iteration,
 // so the sweep takes the change from the value it overwrites) or on one of
-// the ray's upwind faces (written only by the halo and face kernels; their
-// start values are saved first and compared after).  Workgroup maxima go
+// the ray's upwind faces (written once, by rt_incoming_kernel, which takes
+// the change as well).  Workgroup maxima go
 // by atomicMax into one of RT_PARTS slots, 32 words apart, then one small
 // kernel reduces them.
 __device__ __forceinline__ unsigned rt_change(double now, double before) {
@@ -253,7 +253,8 @@ __global__ __launch_bounds__(64 * W) void rt_sweep_tile_kernel(
   rt_block_max(best, part);
 }
 
-constexpr int RT_TILE_R = 4;  // rows a wave holds (2: 18.3 ms for 17.0, 8: 22.8)
+// rows a wave holds, in patches of RT_ROWS and of RT_ROWS_SMALL rows
+constexpr int RT_R = 4, RT_R_SMALL = 5;
 
 hipError_t launch_rt_sweep_tiles(hipStream_t st, double *I, const double *kap, const double *S,
                                  const double *kap_y, const double *S_y, const RtRays &rays,
@@ -275,88 +276,91 @@ hipError_t launch_rt_sweep_tiles(hipStream_t st, double *I, const double *kap, c
   pt.per_xcd = (pt.start[pt.groups] + 7) / 8;
   const dim3 grid(8 * pt.per_xcd * pt.same);
   if (rows == RT_ROWS_SMALL)
-    hipLaunchKernelGGL((rt_sweep_tile_kernel<RT_TILE_R, RT_ROWS_SMALL / RT_TILE_R>), grid,
-                       dim3(64 * RT_ROWS_SMALL / RT_TILE_R), 0, st, I, kap, S, kap_y, S_y, rays, pt, p0, P,
-                       ray_stride, part);
+    hipLaunchKernelGGL((rt_sweep_tile_kernel<RT_R_SMALL, RT_ROWS_SMALL / RT_R_SMALL>), grid,
+                       dim3(64 * RT_ROWS_SMALL / RT_R_SMALL), 0, st, I, kap, S, kap_y, S_y, rays,
+                       pt, p0, P, ray_stride, part);
   else
-    hipLaunchKernelGGL((rt_sweep_tile_kernel<RT_TILE_R, RT_ROWS / RT_TILE_R>), grid,
-                       dim3(64 * RT_ROWS / RT_TILE_R), 0, st, I, kap, S, kap_y, S_y, rays, pt, p0, P,
+    hipLaunchKernelGGL((rt_sweep_tile_kernel<RT_R, RT_ROWS / RT_R>), grid,
+                       dim3(64 * RT_ROWS / RT_R), 0, st, I, kap, S, kap_y, S_y, rays, pt, p0, P,
                        ray_stride, part);
   return hipGetLastError();
 }
 
-// periodic halo self-exchange along `axis` over the full transverse extent
-// (rt_host.hpp:236-452): + rays copy node b1 into b0, - rays b0 into b1.
-// rays outside ray_mask are left alone (the other layout's launch does them)
-__global__ __launch_bounds__(256) void rt_halo_kernel(double *__restrict__ I, int axis, int b0,
-                                                      int b1, int It, int Jt, int Kt,
-                                                      unsigned pos_mask, unsigned ray_mask,
-                                                      long ray_stride, int nrays) {
-  const int n1 = axis == 0 ? Jt : It, n2 = axis == 2 ? Jt : Kt;
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long)n1 * n2 * nrays) return;
-  const int u = (int)(t % n1);
-  const long r = t / n1;
-  const int v = (int)(r % n2), n = (int)(r / n2);
-  if (!((ray_mask >> n) & 1u)) return;
-  int i, j, k;
-  if (axis == 0) { j = u; k = v; i = 0; }
-  else if (axis == 1) { i = u; k = v; j = 0; }
-  else { i = u; j = v; k = 0; }
-  const bool pos = (pos_mask >> n) & 1u;
-  int s[3] = {i, j, k}, d[3] = {i, j, k};
-  s[axis] = pos ? b1 : b0;
-  d[axis] = pos ? b0 : b1;
-  double *Ir = I + ray_stride * n;
-  Ir[(d[2] * Jt + d[1]) * It + d[0]] = Ir[(s[2] * Jt + s[1]) * It + s[0]];
-}
-
-// incoming boundary on one physical face (rt_host.hpp:50-89): nodes of the
-// face layer over the lattice's transverse range, rays in `in_mask`.
-__global__ __launch_bounds__(256) void rt_face_kernel(double *__restrict__ I,
-                                                      const double *__restrict__ S, int axis,
-                                                      int layer, int lo0, int lo1, int n0, int n1,
-                                                      int It, int Jt, int kind, double value,
-                                                      unsigned in_mask, long ray_stride,
-                                                      int nrays) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long)n0 * n1 * nrays) return;
-  const int u = lo0 + (int)(t % n0);
-  const long r = t / n0;
-  const int v = lo1 + (int)(r % n1), n = (int)(r / n1);
-  if (!((in_mask >> n) & 1u)) return;
-  int i, j, k;
-  if (axis == 0) { i = layer; j = u; k = v; }
-  else if (axis == 1) { j = layer; i = u; k = v; }
-  else { k = layer; i = u; j = v; }
-  const int c = (k * Jt + j) * It + i;
-  I[ray_stride * n + c] = kind == 1 ? S[c] : (kind == 2 ? 0.0 : value);
-}
-
-// The upwind faces of every ray over the lattice (axes with more than one
-// node; blockIdx.y = ray * 3 + axis): the layer x_a = lo_a (ray going +) or
-// lo_a + n_a - 1, all lattice nodes of the other two axes.  save: old = I
-// there; otherwise the change of I against old, into the parts.
-__global__ __launch_bounds__(256) void rt_faces_kernel(const double *__restrict__ I,
-                                                       double *__restrict__ old, int save,
-                                                       RtFaces f, long ray_stride,
-                                                       unsigned *part) {
+// The rays' upwind boundary nodes before a sweep (blockIdx.y = ray * 3 +
+// axis): what the periodic halo self-exchange along z, y and x
+// (rt_host.hpp:236-452: + rays copy node b1 into b0, - rays b0 into b1, over
+// the full transverse extent), then the incoming boundaries of the physical
+// faces in axis order (rt_host.hpp:50-101: the lattice's transverse range)
+// leave there, in one pass: a node on several faces takes the value of the
+// last physical one, or else the start value with every periodic coordinate
+// moved to the far end.  That source lies on no face that this pass writes
+// (where it would, so does the node itself, and takes the face's value), so
+// the order of the threads does not matter.  Each node belongs to its lowest
+// axis.  The change of the lattice nodes goes into the parts.
+// Bound by the strided faces (x of an x-fastest ray, y of a y-fastest one: a
+// cache line per node), which this pass reads and writes once.  As launches
+// of their own, saving the faces, the exchange, the boundaries and the
+// comparison read them four times: 155 us an iteration at 384^2 x 28, this
+// pass 41 (radiative step of 256^3 17.0 -> 16.5 ms, cold solve of 211 x 150 x
+// 187 8.2 -> 7.7 ms).
+__global__ __launch_bounds__(256) void rt_incoming_kernel(double *__restrict__ I,
+                                                          const double *__restrict__ S_x,
+                                                          const double *__restrict__ S_y,
+                                                          RtIncoming f, long ray_stride,
+                                                          unsigned *part) {
   const int n = blockIdx.y / 3, a = blockIdx.y % 3;
-  if (f.n[a] <= 1) return;  // uniform over the block
-  const int t0 = a == 0 ? 1 : 0, t1 = a == 2 ? 1 : 2;
+  if (f.hi[a] <= f.lo[a]) return;  // uniform over the block
+  const bool tr = (f.tr >> n) & 1u;
+  // the face's nodes, the faster axis of the ray's layout first
+  const int t0 = a == 0 ? 1 : a == 1 ? 0 : tr ? 1 : 0, t1 = 3 - a - t0;
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   unsigned best = 0u;
-  if (t < f.n[t0] * f.n[t1]) {
-    int x[3];
-    x[a] = f.lo[a] + (((f.pos[a] >> n) & 1u) ? 0 : f.n[a] - 1);
-    x[t0] = f.lo[t0] + t % f.n[t0];
-    x[t1] = f.lo[t1] + t / f.n[t0];
-    const long c = ray_stride * n + (((f.tr >> n) & 1u) ? ((long)x[2] * f.It + x[0]) * f.Jt + x[1]
-                                                         : ((long)x[2] * f.Jt + x[1]) * f.It + x[0]);
-    if (save) old[c] = I[c];
-    else best = rt_change(I[c], old[c]);
+  if (t < f.tot[t0] * f.tot[t1]) {
+    int x[3], up[3];
+    bool on[3], in = true;
+    x[t0] = t % f.tot[t0];
+    x[t1] = t / f.tot[t0];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      up[d] = ((f.pos[d] >> n) & 1u) ? f.lo[d] : f.hi[d];
+      if (d == a) x[d] = up[d];
+      on[d] = f.hi[d] > f.lo[d] && x[d] == up[d];
+      in = in && x[d] >= f.lo[d] && x[d] <= f.hi[d];
+    }
+    if (!(a > 0 && on[0]) && !(a > 1 && on[1])) {
+      auto at = [&](const int *q) {
+        return tr ? ((long)q[2] * f.tot[0] + q[0]) * f.tot[1] + q[1]
+                  : ((long)q[2] * f.tot[1] + q[1]) * f.tot[0] + q[0];
+      };
+      const long c = at(x);
+      int kind = 0;
+      double value = 0.0;
+      int src[3];
+      bool moved = false;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        src[d] = x[d];
+        if (!on[d]) continue;
+        const int side = up[d] == f.lo[d] ? 0 : 1;
+        if (f.periodic[d]) {
+          src[d] = side ? f.lo[d] : f.hi[d];
+          moved = true;
+        } else if (in && f.kind[2 * d + side] && ((f.moving[d] >> n) & 1u)) {
+          kind = f.kind[2 * d + side];
+          value = f.value[2 * d + side];
+        }
+      }
+      if (kind || moved) {
+        double *In = I + ray_stride * n;
+        const double before = In[c];
+        const double now = kind == 1 ? (tr ? S_y : S_x)[c] : kind == 2 ? 0.0
+                         : kind ? value : In[at(src)];
+        In[c] = now;
+        if (in) best = rt_change(now, before);
+      }
+    }
   }
-  if (!save) rt_block_max(best, part);
+  rt_block_max(best, part);
 }
 
 // slot = max of the parts; the parts are cleared for the next iteration
@@ -454,35 +458,13 @@ hipError_t launch_rt_transpose_xy(hipStream_t st, const double *src, double *dst
   return hipGetLastError();
 }
 
-hipError_t launch_rt_halo(hipStream_t st, double *I, int axis, int b0, int b1, int It, int Jt,
-                          int Kt, unsigned pos_mask, unsigned ray_mask, long ray_stride,
-                          int nrays) {
-  const int n1 = axis == 0 ? Jt : It, n2 = axis == 2 ? Jt : Kt;
-  const long n = (long)n1 * n2 * nrays;
-  hipLaunchKernelGGL(rt_halo_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, I, axis,
-                     b0, b1, It, Jt, Kt, pos_mask, ray_mask, ray_stride, nrays);
-  return hipGetLastError();
-}
-
-hipError_t launch_rt_face(hipStream_t st, double *I, const double *S, int axis, int layer,
-                          int lo0, int lo1, int n0, int n1, int It, int Jt, int kind, double value,
-                          unsigned in_mask, long ray_stride, int nrays) {
-  const long n = (long)n0 * n1 * nrays;
-  hipLaunchKernelGGL(rt_face_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, I, S,
-                     axis, layer, lo0, lo1, n0, n1, It, Jt, kind, value, in_mask, ray_stride,
-                     nrays);
-  return hipGetLastError();
-}
-
-hipError_t launch_rt_faces(hipStream_t st, const double *I, double *old, bool save,
-                          const RtFaces &f, long ray_stride, int nrays, unsigned *part) {
+hipError_t launch_rt_incoming(hipStream_t st, double *I, const double *S, const double *S_y,
+                              const RtIncoming &f, long ray_stride, int nrays, unsigned *part) {
   int m = 1;
-  for (int a = 0; a < 3; ++a) {
-    const int t0 = a == 0 ? 1 : 0, t1 = a == 2 ? 1 : 2;
-    m = max(m, f.n[t0] * f.n[t1]);
-  }
-  hipLaunchKernelGGL(rt_faces_kernel, dim3((m + 255) / 256, 3 * nrays), dim3(256), 0, st, I, old,
-                     save ? 1 : 0, f, ray_stride, part);
+  for (int a = 0; a < 3; ++a)
+    if (f.hi[a] > f.lo[a]) m = max(m, f.tot[(a + 1) % 3] * f.tot[(a + 2) % 3]);
+  hipLaunchKernelGGL(rt_incoming_kernel, dim3((m + 255) / 256, 3 * nrays), dim3(256), 0, st, I, S,
+                     S_y, f, ray_stride, part);
   return hipGetLastError();
 }
 

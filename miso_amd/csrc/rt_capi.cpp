@@ -3,18 +3,16 @@
 // Host side of RT::solve (miso/include/miso/rt_host.hpp:632-651): per-ray
 // sweep constants are computed here with the reference's expressions
 // (rt_host.hpp:461-508, float-narrowed max/min included), then every
-// iteration is: save the rays' upwind faces into rint_old, periodic halo
-// (z, y, x), incoming boundary on physical faces, the sweeps (which take
-// the change of every node they write), the change on the upwind faces,
-// and the max change read back to decide convergence.  That is the
-// reference's max over the lattice of |rint - rint_old| with rint_old a
-// full copy (rt_host.hpp:612-651), without the copy.
+// iteration is: the rays' upwind boundaries (periodic halo z, y, x and the
+// incoming boundaries of the physical faces), the sweeps, each taking the
+// change of every node it writes, and the max change read back to decide
+// convergence.  That is the reference's max over the lattice of
+// |rint - rint_old| with rint_old a full copy (rt_host.hpp:612-651), without
+// the copy.
 //
 // Rays whose dominant axis is x run in the y-fastest frame (node (i, j, k)
 // at (k * i_total + i) * j_total + j): their constants are those of the
-// x-fastest frame with the strides of x and y swapped, and each halo, face
-// and reduction launch comes in two, one per frame, with x and y swapped in
-// the second.
+// x-fastest frame with the strides of x and y swapped.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -167,14 +165,6 @@ int setup(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_config *rt, 
   return MISOHIP_OK;
 }
 
-// (lo, cnt, It, Jt, axis) of the y-fastest frame: x and y swapped
-inline void swap_xy(const int in[3], int out[3]) {
-  out[0] = in[1];
-  out[1] = in[0];
-  out[2] = in[2];
-}
-inline int frame_axis(int a, bool y) { return y && a < 2 ? 1 - a : a; }
-
 int check_rt(const misohip_grid *g, const misohip_rt_config *rt) {
   if (!g || !rt) return MISOHIP_E_ARG;
   if (rt->num_rays != 24 && rt->num_rays != 1) return MISOHIP_E_ARG;
@@ -204,19 +194,9 @@ int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_c
   RtSetup su;
   if (int rc = setup(ctx, g, rt, su)) return rc;
   double *I = static_cast<double *>(rint);
-  double *old = static_cast<double *>(rint_old);
   const double *kap = static_cast<const double *>(kappa);
   const double *src = static_cast<const double *>(S);
   const int It = g->i_total, Jt = g->j_total, Kt = g->k_total;
-  int lo[3], cnt[3], lo_y[3], cnt_y[3];
-  for (int a = 0; a < 3; ++a) {
-    lo[a] = su.b0[a];
-    cnt[a] = su.b1[a] - su.b0[a] + 1;
-  }
-  swap_xy(lo, lo_y);
-  swap_xy(cnt, cnt_y);
-  const unsigned all = su.nrays >= 32 ? ~0u : ((1u << su.nrays) - 1u);
-  const unsigned x_mask = all & ~su.tr_mask;
   const double *kap_y = nullptr, *src_y = nullptr;
   if (su.tr_mask) {
     const size_t cells = (size_t)su.ray_stride;
@@ -258,18 +238,34 @@ int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_c
   });
   struct Chain {
     RtRays rays;
-    int n = 0, planes = 0;
-    long blocks = 0;  // workgroups a launch in patches of RT_ROWS rows
+    int n = 0, planes = 0, rows = RT_ROWS_SMALL;
+    long blocks = 0;  // workgroups of a launch in patches of RT_ROWS rows
   };
-  std::vector<Chain> chains;
+  std::vector<Chain> axes;
   for (const RtRay &R : trays) {
-    if (chains.empty() || chains.back().rays.r[0].tr != R.tr ||
-        std::abs(chains.back().rays.r[0].da) != std::abs(R.da))
-      chains.emplace_back();
-    Chain &ch = chains.back();
+    if (axes.empty() || axes.back().rays.r[0].tr != R.tr ||
+        std::abs(axes.back().rays.r[0].da) != std::abs(R.da))
+      axes.emplace_back();
+    Chain &ch = axes.back();
     ch.rays.r[ch.n++] = R;
     ch.planes = std::max(ch.planes, R.nplanes);
     ch.blocks += (long)rt_patches(R.nb, 64, P) * rt_patches(R.nc, RT_ROWS, P);
+  }
+  // chains of few workgroups take shorter patches and share their launches
+  std::vector<Chain> chains;
+  int few = -1;
+  for (Chain &ch : axes) {
+    if (ch.blocks >= RT_FEW) {
+      ch.rows = RT_ROWS;
+    } else if (few < 0) {
+      few = (int)chains.size();
+    } else {
+      Chain &to = chains[few];
+      for (int r = 0; r < ch.n; ++r) to.rays.r[to.n++] = ch.rays.r[r];
+      to.planes = std::max(to.planes, ch.planes);
+      continue;
+    }
+    chains.push_back(ch);
   }
   // Sweep phases: plane ranges over which the set of rays that still have
   // planes is constant; each phase launches only those rays, sized for
@@ -300,15 +296,24 @@ int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_c
       p0 = e;
     }
   }
-  RtFaces uf;  // the rays' upwind faces
+  RtIncoming in;  // the rays' upwind boundaries
+  in.tot[0] = It;
+  in.tot[1] = Jt;
+  in.tot[2] = Kt;
   for (int a = 0; a < 3; ++a) {
-    uf.lo[a] = lo[a];
-    uf.n[a] = cnt[a];
-    uf.pos[a] = su.pos_mask[a];
+    in.lo[a] = su.b0[a];
+    in.hi[a] = su.b1[a];
+    in.periodic[a] = rt->periodic[a] ? 1 : 0;
+    in.pos[a] = su.pos_mask[a];
+    in.moving[a] = 0u;
+    for (int n = 0; n < su.nrays; ++n)
+      if (su.mu[a][n] != 0.0) in.moving[a] |= 1u << n;
+    for (int side = 0; side < 2; ++side) {
+      in.kind[2 * a + side] = rt->face_kind[2 * a + side];
+      in.value[2 * a + side] = rt->face_value[2 * a + side];
+    }
   }
-  uf.tr = su.tr_mask;
-  uf.It = It;
-  uf.Jt = Jt;
+  in.tr = su.tr_mask;
   if (!ctx->rt_parts) MISOHIP_TRY(hipMalloc(&ctx->rt_parts, sizeof(unsigned) * 32 * RT_PARTS));
   const int nside = std::min(2, std::max(0, (int)chains.size() - 1));
   for (int i = 0; i < nside; ++i)
@@ -325,39 +330,8 @@ int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_c
   for (it = 0; it < rt->max_iters; ++it) {
     {
       Timed t_(ctx, MISOHIP_KIND_RT);
-      MISOHIP_TRY(launch_rt_faces(ctx->stream, I, old, true, uf, su.ray_stride, su.nrays, parts));
-      for (int a = 2; a >= 0; --a)
-        if (rt->periodic[a] && su.size[a] > 1) {
-          if (x_mask)
-            MISOHIP_TRY(launch_rt_halo(ctx->stream, I, a, su.b0[a], su.b1[a], It, Jt, Kt,
-                                       su.pos_mask[a], x_mask, su.ray_stride, su.nrays));
-          if (su.tr_mask)
-            MISOHIP_TRY(launch_rt_halo(ctx->stream, I, frame_axis(a, true), su.b0[a], su.b1[a],
-                                       Jt, It, Kt, su.pos_mask[a], su.tr_mask, su.ray_stride,
-                                       su.nrays));
-        }
-      for (int a = 0; a < 3; ++a)
-        for (int side = 0; side < 2; ++side) {
-          const int kind = rt->face_kind[2 * a + side];
-          if (rt->periodic[a] || su.size[a] <= 1 || kind == 0) continue;
-          unsigned in_mask = 0u;
-          for (int n = 0; n < su.nrays; ++n) {
-            const double mu = su.mu[a][n];
-            if (side == 0 ? mu > 0.0 : mu < 0.0) in_mask |= 1u << n;
-          }
-          for (int y = 0; y < 2; ++y) {
-            const unsigned m = in_mask & (y ? su.tr_mask : x_mask);
-            if (!m) continue;
-            const int fa = frame_axis(a, y);
-            const int t0 = fa == 0 ? 1 : 0, t1 = fa == 2 ? 1 : 2;
-            const int *fl = y ? lo_y : lo, *fc = y ? cnt_y : cnt;
-            MISOHIP_TRY(launch_rt_face(ctx->stream, I, y ? src_y : src, fa,
-                                       side == 0 ? su.b0[a] : su.b1[a], fl[t0], fl[t1], fc[t0],
-                                       fc[t1], y ? Jt : It, y ? It : Jt, kind,
-                                       rt->face_value[2 * a + side], m, su.ray_stride,
-                                       su.nrays));
-          }
-        }
+      MISOHIP_TRY(launch_rt_incoming(ctx->stream, I, src, src_y, in, su.ray_stride, su.nrays,
+                                     parts));
       if (nside > 0) MISOHIP_TRY(hipEventRecord(ctx->rt_fork, ctx->stream));
       for (int i = 0; i < nside; ++i)
         MISOHIP_TRY(hipStreamWaitEvent(ctx->rt_side[i], ctx->rt_fork, 0));
@@ -369,8 +343,7 @@ int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_c
           if (p0 >= ch.planes) continue;
           const int i = (int)c % (nside + 1);
           MISOHIP_TRY(launch_rt_sweep_tiles(i ? ctx->rt_side[i - 1] : ctx->stream, I, kap, src,
-                                            kap_y, src_y, ch.rays, ch.n, p0, P,
-                                            ch.blocks < RT_FEW ? RT_ROWS_SMALL : RT_ROWS,
+                                            kap_y, src_y, ch.rays, ch.n, p0, P, ch.rows,
                                             su.ray_stride, parts));
           if (p0 + P < ch.planes) ++left;
         }
@@ -383,7 +356,6 @@ int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_c
         MISOHIP_TRY(hipEventRecord(ctx->rt_join[i], ctx->rt_side[i]));
         MISOHIP_TRY(hipStreamWaitEvent(ctx->stream, ctx->rt_join[i], 0));
       }
-      MISOHIP_TRY(launch_rt_faces(ctx->stream, I, old, false, uf, su.ray_stride, su.nrays, parts));
       MISOHIP_TRY(launch_rt_parts_reduce(ctx->stream, parts, ctx->d_slot + 1, false));
     }
     MISOHIP_TRY(hipMemcpyAsync(ctx->h_slot + 1, ctx->d_slot + 1, sizeof(unsigned),
