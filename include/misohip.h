@@ -352,6 +352,13 @@ int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_c
 int misohip_rt_ray_layout(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_config *rt,
                           unsigned *yfast_mask);
 
+/* out = rint with every ray's field x-fastest (the fields of yfast_mask
+ * transposed, the others copied), on the given stream of the current device
+ * (NULL = the null stream); out may not be rint.  MISOHIP_E_ARG above 32 rays
+ * or 65535 z cells. */
+int misohip_rt_xfast(const misohip_grid *g, int num_rays, unsigned yfast_mask, const void *rint,
+                     void *out, void *stream);
+
 /* Q_rad = 4 pi kappa (J - S), J = sum_r w_r I_r, on the RT lattice (no
  * counterpart in the reference, which has no MHD coupling). */
 int misohip_rt_qrad(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_config *rt,

@@ -110,6 +110,7 @@ struct RtPatches {
 hipError_t launch_rt_sweep_tiles(hipStream_t, double *, const double *, const double *,
                                  const double *, const double *, const RtRays &, int, int, int,
                                  int, long, unsigned *);
+hipError_t launch_rt_xfast(hipStream_t, const double *, double *, int, int, int, int, unsigned);
 hipError_t launch_rt_incoming(hipStream_t, double *, const double *, const double *,
                               const RtIncoming &, long, int, unsigned *);
 hipError_t launch_rt_parts_reduce(hipStream_t, unsigned *, unsigned *, bool);

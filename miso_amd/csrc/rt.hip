@@ -450,6 +450,42 @@ __global__ __launch_bounds__(256) void rt_transpose_xy_kernel(const double *__re
   }
 }
 
+// Every ray's field x-fastest (blockIdx.z = ray): 32 x 32 tiles of a plane,
+// through LDS where the ray is kept y-fastest.  Bound by HBM (each value read
+// and written once); a clone followed by a transpose of each y-fastest ray
+// wrote those rays twice.
+__global__ __launch_bounds__(256) void rt_xfast_kernel(const double *__restrict__ I,
+                                                       double *__restrict__ out, int It, int Jt,
+                                                       int tiles_i, unsigned tr, long ray_stride) {
+  __shared__ double tile[32][33];
+  const int ti = blockIdx.x % tiles_i, tj = blockIdx.x / tiles_i, l = threadIdx.x & 31;
+  const long plane = ray_stride * blockIdx.z + (long)It * Jt * blockIdx.y;
+  const bool y = (tr >> blockIdx.z) & 1u;  // uniform over the block
+  if (y) {
+    for (int r = threadIdx.x >> 5; r < 32; r += 8) {
+      const int j = tj * 32 + l, i = ti * 32 + r;
+      if (i < It && j < Jt) tile[r][l] = I[plane + (long)i * Jt + j];
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    const int r = (threadIdx.x >> 5) + 8 * m, i = ti * 32 + l, j = tj * 32 + r;
+    if (i < It && j < Jt) {
+      const long c = plane + (long)j * It + i;
+      out[c] = y ? tile[l][r] : I[c];
+    }
+  }
+}
+
+hipError_t launch_rt_xfast(hipStream_t st, const double *I, double *out, int It, int Jt, int Kt,
+                           int nrays, unsigned tr) {
+  const int ti = (It + 31) / 32, tj = (Jt + 31) / 32;
+  hipLaunchKernelGGL(rt_xfast_kernel, dim3(ti * tj, Kt, nrays), dim3(256), 0, st, I, out, It, Jt,
+                     ti, tr, (long)It * Jt * Kt);
+  return hipGetLastError();
+}
+
 hipError_t launch_rt_transpose_xy(hipStream_t st, const double *src, double *dst, int It, int Jt,
                                   int Kt) {
   const int ti = (It + 31) / 32, tj = (Jt + 31) / 32;

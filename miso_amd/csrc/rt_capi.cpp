@@ -406,6 +406,17 @@ int misohip_rt_ray_layout(misohip_ctx *ctx, const misohip_grid *g, const misohip
   return MISOHIP_OK;
 }
 
+int misohip_rt_xfast(const misohip_grid *g, int num_rays, unsigned yfast_mask, const void *rint,
+                     void *out, void *stream) {
+  if (!g || !rint || !out || rint == out || num_rays < 1 || num_rays > 32) return MISOHIP_E_ARG;
+  if (g->i_total < 1 || g->j_total < 1 || g->k_total < 1 || g->k_total > 65535)
+    return MISOHIP_E_ARG;
+  MISOHIP_TRY(launch_rt_xfast(static_cast<hipStream_t>(stream), static_cast<const double *>(rint),
+                              static_cast<double *>(out), g->i_total, g->j_total, g->k_total,
+                              num_rays, yfast_mask));
+  return MISOHIP_OK;
+}
+
 int misohip_rt_source(misohip_ctx *ctx, const misohip_grid *g, const misohip_fields *qq,
                       double gm, double kappa0, double s_rad, void *kappa, void *S) {
   if (!ctx || !g || !qq || !kappa || !S || !qq->q[0] || !qq->q[7]) return MISOHIP_E_ARG;

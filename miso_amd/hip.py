@@ -119,6 +119,7 @@ SIGNATURES = {
     "misohip_rt_qrad": [C.c_void_p, _P(MisohipGrid), _P(MisohipRtConfig), C.c_void_p, C.c_void_p,
                         C.c_void_p, C.c_void_p],
     "misohip_rt_ray_layout": [C.c_void_p, _P(MisohipGrid), _P(MisohipRtConfig), _P(C.c_uint)],
+    "misohip_rt_xfast": [_P(MisohipGrid), C.c_int, C.c_uint, C.c_void_p, C.c_void_p, C.c_void_p],
     "misohip_rt_source": [C.c_void_p, _P(MisohipGrid), _P(MisohipFields), C.c_double, C.c_double,
                           C.c_double,
                           C.c_void_p, C.c_void_p],

@@ -66,11 +66,12 @@ class RT:
         mask = self.yfast_mask
         if not mask:
             return self.rint
-        out = self.rint.clone()
-        kt, jt, it = self.rint.shape[1:]
-        for n in range(self.num_rays):
-            if (mask >> n) & 1:
-                out[n] = self.rint[n].reshape(kt, it, jt).permute(0, 2, 1)
+        import torch
+        out = torch.empty_like(self.rint)
+        with torch.cuda.device(out.device):
+            hip.call("misohip_rt_xfast", C.byref(self.grid.c_struct()), self.num_rays, mask,
+                     C.c_void_p(self.rint.data_ptr()), C.c_void_p(out.data_ptr()),
+                     C.c_void_p(torch.cuda.current_stream(out.device).cuda_stream))
         return out
 
     def solve(self, ctx, **kw):
