@@ -1,26 +1,29 @@
 // Per-column MLP surrogate of the radiative heating: BF16 operands on the
-// CDNA4 matrix cores (v_mfma_f32_32x32x16_bf16), FP32 accumulation, FP32
+// CDNA4 matrix cores (v_mfma_f32_16x16x32_bf16), FP32 accumulation, FP32
 // master weights.  No counterpart in the reference (it has no MHD-RT
 // coupling at all).
 //
-// Network: x (3*nz features of one column) -> 256 -> 256 -> 256 -> nz,
-// SiLU on the hidden layers.  Weights are stored [out][in] (row-major), so
-// a forward layer is C = X * W^T and the weight gradient is dW = dY^T * X.
+// Network: x (3*nz or 4*nz features of one column) -> hidden -> ... -> nz,
+// SiLU on the hidden layers; every width a multiple of 32.
 //
-// GEMM tile: 128 x 128 outputs per 256-thread block, each wave a 64 x 64
-// quadrant (2 x 2 MFMA 32x32 tiles), K staged through LDS 32 at a time.
-// MFMA 32x32x16 lane layout: lane l holds A[l%32][8*(l/32) .. +7],
-// B[8*(l/32) .. +7][l%32], and accumulator v holds
-// D[8*(v/4) + 4*(l/32) + v%4][l%32].
+// MFMA 16x16x32 lane layout: lane l holds A[l%16][8*(l/16) .. +7],
+// B[8*(l/16) .. +7][l%16], and accumulator v holds D[4*(l/16) + v][l%16].
+// Every operand that a kernel takes from global memory is kept in blocks of
+// 16 rows x 32 k (1 KiB), the lane's 8 values next to each other ("packed"),
+// so that a wave loads a fragment as 1 KiB of consecutive bytes.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include "launch.hpp"
+#include <type_traits>
+
+#include "mlp.hpp"
 
 namespace misohip {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+// the caller's fp32 arrays: four floats at any multiple of four bytes
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 __device__ __forceinline__ uint16_t f2bf(float f) {  // round to nearest even
   uint32_t u = __float_as_uint(f);
@@ -28,187 +31,380 @@ __device__ __forceinline__ uint16_t f2bf(float f) {  // round to nearest even
   u += 0x7fffu + ((u >> 16) & 1u);
   return (uint16_t)(u >> 16);
 }
-__device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
+__device__ __forceinline__ uint2 f2bf4(f32x4 x) {
+  return make_uint2((uint32_t)f2bf(x[0]) | (uint32_t)f2bf(x[1]) << 16,
+                    (uint32_t)f2bf(x[2]) | (uint32_t)f2bf(x[3]) << 16);
+}
+__device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
 
-constexpr int BM = 128, BN = 128, BK = 32, LDK = BK + 8;  // LDS row pitch in bf16
+// The network from its input columns to its output (TRAIN: and back from the
+// gradient of the mean squared error to every layer's pre-activation gradient;
+// Y, where given, receives the output) in one launch: a workgroup
+// takes NS = 16 NT columns through all layers.  A layer is D = W a: the
+// weights are the A operand, from their packed copies (L2 holds all of them),
+// the activations the B operand, rows of one column in one of two buffers in
+// LDS (WIDE: in the workgroup's part of g0, g1, where two of them do not fit);
+// lanes are columns in D, so that a lane holds four consecutive outputs of
+// one column.  X passes through LDS in chunks of xw features (all but the last
+// a multiple of 32 PD: the k-steps in flight keep their places).
+//   A wave takes cnt <= RT row tiles of 16 outputs at a time and keeps PD
+// k-steps of their weights in flight; the first PD of the next layer are
+// loaded before the barrier that ends a layer.
+//   TRAIN keeps what the weight gradients read, packed with the columns as k:
+// X and the activations (aT), the pre-activation gradients (dT); and the
+// hidden layers' pre-activations in FP32, which the lane that wrote them
+// reads again.
+// Bound by the weights' way from L2 into the CU (64 bytes a clock): 1.24 MB
+// forward and 0.46 back for 1536-256-256-256-384.
+// NT = 1 (16 waves) spreads a batch of 1024 over 64 CUs; NT = 4 (four waves,
+// two workgroups a CU) reads the weights a quarter as often, for large
+// batches of inference.
+// At that size and a batch of 1024 a training step's chain takes 37 us, where
+// a launch per layer, product and elementwise step (128 x 128 tiles: 16
+// workgroups) took 232; 147456 columns of inference, their Q_rad field
+// included, 721 us for 957.  Every sum is taken in the order of k, 32 at a
+// time, as those took it: the same bits.
+template <int NT, int WAVES, int RT, int PD, bool TRAIN, bool WIDE>
+__global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 4) void mlp_chain_kernel(
+    const MlpLayer *__restrict__ L, int nl, const uint16_t *__restrict__ X, int M,
+    float *__restrict__ Y, MlpLoss ls, MlpField fo, uint16_t *g0, uint16_t *g1, int bw, int xoff,
+    int xw) {
+  constexpr int NS = 16 * NT, NTHR = 64 * WAVES;
+  static_assert(NT == 1 || !TRAIN, "the packed columns of a training tile are 16");
+  extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, kq = lane >> 4;
+  const int s0 = blockIdx.x * NS;
+  const int pitch = bw + 8, xpitch = xw + 8;  // odd multiples of 16 bytes: no bank conflicts
+  // the input layer writes the first buffer (X may be staged in the second)
+  uint16_t *nxt = WIDE ? g0 + (long)s0 * pitch : lds;
+  uint16_t *cur = WIDE ? g1 + (long)s0 * pitch : lds + NS * pitch;
+  uint16_t *xbuf = lds + xoff;
+  const int n_in = L[0].in;
 
-// C[m][n] = sum_k A(m,k) B(k,n) over the block's K range.
-//   TA = false: A stored [M][lda] (A(m,k) at m*lda+k);  true: [K][lda] (k*lda+m)
-//   TB = true : B stored [N][ldb] (B(k,n) at n*ldb+k);  false: [K][ldb] (k*ldb+n)
-// K must be a multiple of 32 within each split; M, N arbitrary.
-// EPI 0: raw fp32 to C (+ split offset);  1: pre = acc + bias -> C, and
-// bf16(silu(pre)) -> H;  2: acc + bias -> C (output layer);  3: as 1
-// without C (inference: the pre-activations are kept only for training).
-template <bool TA, bool TB, int EPI>
-__global__ __launch_bounds__(256) void gemm_bf16_kernel(const uint16_t *__restrict__ A,
-                                                        const uint16_t *__restrict__ B,
-                                                        float *__restrict__ C,
-                                                        uint16_t *__restrict__ H,
-                                                        const float *__restrict__ bias, int M,
-                                                        int N, int K, int lda, int ldb, int ldc,
-                                                        int k_per_split) {
-  __shared__ uint16_t As[BM * LDK];
-  __shared__ uint16_t Bs[BN * LDK];
-  const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
-  const int kb = blockIdx.z * k_per_split;
-  const int ke = min(K, kb + k_per_split);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-  f32x16 acc[2][2];
+  bf16x8 a[PD][RT];
+  f32x4 acc[RT][NT];
+  auto frag = [&](const uint16_t *wp, int KT, int tile, int kt) {
+    return *reinterpret_cast<const bf16x8 *>(wp + ((long)tile * KT + kt) * 512 + lane * 8);
+  };
+  // row tiles per wave in a pass over a layer of OT row tiles, evened out
+  auto tiles_of = [&](int OT) {
+    const int np = (OT + WAVES * RT - 1) / (WAVES * RT);
+    return (OT + np * WAVES - 1) / (np * WAVES);
+  };
+  // first k-steps of the weights (tiles past the last one load the last)
+  auto preload = [&](const uint16_t *wp, int KT, int OT, int base, int cnt) {
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+    for (int p = 0; p < PD; ++p)
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+      for (int r = 0; r < RT; ++r)
+        if (r < cnt)
+          a[p][r] = frag(wp, KT, min(base + wave * cnt + r, OT - 1), min(p, KT - 1));
+  };
+  // 8 consecutive columns of feature f per lane, in blocks of 16 f x 32 columns
+  auto pack = [&](const uint16_t *src, int sp, int nf, uint16_t *dst, int f0) {
+    for (int t = tid; t < 2 * nf; t += NTHR) {
+      const int f = t & 15, o = (t >> 4) & 1, ft = t >> 5;
+      uint32_t v[4];
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.f;
-
-  for (int k0 = kb; k0 < ke; k0 += BK) {
-    // ---- stage A tile (BM x BK) as As[m][k]
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      const int c = tid + 256 * r;
-      if (!TA) {
-        const int row = c >> 2, kc = (c & 3) * 8;
-        uint4 v = make_uint4(0, 0, 0, 0);
-        if (m0 + row < M) v = *reinterpret_cast<const uint4 *>(A + (long)(m0 + row) * lda + k0 + kc);
-        *reinterpret_cast<uint4 *>(&As[row * LDK + kc]) = v;
-      } else {
-        const int kr = c >> 4, mc = (c & 15) * 8;
-        uint16_t e[8];
-        if (m0 + mc + 7 < M) {
-          uint4 v = *reinterpret_cast<const uint4 *>(A + (long)(k0 + kr) * lda + m0 + mc);
-          const uint16_t *p = reinterpret_cast<const uint16_t *>(&v);
-#pragma unroll
-          for (int q = 0; q < 8; ++q) e[q] = p[q];
-        } else {
-#pragma unroll
-          for (int q = 0; q < 8; ++q)
-            e[q] = (m0 + mc + q < M) ? A[(long)(k0 + kr) * lda + m0 + mc + q] : (uint16_t)0;
-        }
-#pragma unroll
-        for (int q = 0; q < 8; ++q) As[(mc + q) * LDK + kr] = e[q];
+      for (int e = 0; e < 4; ++e) {
+        const uint16_t *q = src + (8 * o + 2 * e) * sp + ft * 16 + f;
+        v[e] = (uint32_t)q[0] | (uint32_t)q[sp] << 16;
       }
+      const long blk = (long)(f0 / 16 + ft) * (M >> 5) + (s0 >> 5);
+      *reinterpret_cast<uint4 *>(dst + blk * 512 + (f + 16 * (o + ((s0 >> 3) & 2))) * 8) =
+          make_uint4(v[0], v[1], v[2], v[3]);
     }
-    // ---- stage B tile (BK x BN) as Bs[n][k]
+  };
+  // features [f0, f0 + cw) of the workgroup's columns into xbuf
+  auto stage = [&](int f0) {
+    const int cw = min(xw, n_in - f0), per = cw >> 3, n = NS * per;
+    __syncthreads();
+    for (int t = tid; t < n; t += 4 * NTHR) {
+      uint4 v[4];
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      const int c = tid + 256 * r;
-      if (TB) {
-        const int col = c >> 2, kc = (c & 3) * 8;
-        uint4 v = make_uint4(0, 0, 0, 0);
-        if (n0 + col < N) v = *reinterpret_cast<const uint4 *>(B + (long)(n0 + col) * ldb + k0 + kc);
-        *reinterpret_cast<uint4 *>(&Bs[col * LDK + kc]) = v;
-      } else {
-        const int kr = c >> 4, nc = (c & 15) * 8;
-        uint16_t e[8];
-        if (n0 + nc + 7 < N) {
-          uint4 v = *reinterpret_cast<const uint4 *>(B + (long)(k0 + kr) * ldb + n0 + nc);
-          const uint16_t *p = reinterpret_cast<const uint16_t *>(&v);
+      for (int e = 0; e < 4; ++e) {
+        const int q = t + e * NTHR, r = q / per, c = q - r * per;
+        v[e] = make_uint4(0, 0, 0, 0);
+        if (q < n && s0 + r < M)
+          v[e] = *reinterpret_cast<const uint4 *>(X + (long)(s0 + r) * n_in + f0 + 8 * c);
+      }
 #pragma unroll
-          for (int q = 0; q < 8; ++q) e[q] = p[q];
-        } else {
-#pragma unroll
-          for (int q = 0; q < 8; ++q)
-            e[q] = (n0 + nc + q < N) ? B[(long)(k0 + kr) * ldb + n0 + nc + q] : (uint16_t)0;
-        }
-#pragma unroll
-        for (int q = 0; q < 8; ++q) Bs[(nc + q) * LDK + kr] = e[q];
+      for (int e = 0; e < 4; ++e) {
+        const int q = t + e * NTHR, r = q / per, c = q - r * per;
+        if (q < n) *reinterpret_cast<uint4 *>(xbuf + r * xpitch + 8 * c) = v[e];
       }
     }
     __syncthreads();
+    return cw;
+  };
+  // acc = W b over all k for `cnt` row tiles; input: b is X, chunk by chunk
+  auto gemm = [&](auto cnt_, const uint16_t *wp, int KT, int OT, int base, const uint16_t *b,
+                  bool input, bool keep) {
+    constexpr int cnt = decltype(cnt_)::value;
+    int tile[cnt];
 #pragma unroll
-    for (int ks = 0; ks < BK; ks += 16) {
-      const int kk = ks + 8 * (lane >> 5);
-      bf16x8 af[2], bfv[2];
+    for (int r = 0; r < cnt; ++r) tile[r] = min(base + wave * cnt + r, OT - 1);
 #pragma unroll
-      for (int a = 0; a < 2; ++a)
-        af[a] = *reinterpret_cast<const bf16x8 *>(&As[(wm + 32 * a + (lane & 31)) * LDK + kk]);
+    for (int r = 0; r < cnt; ++r)
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
-        bfv[b] = *reinterpret_cast<const bf16x8 *>(&Bs[(wn + 32 * b + (lane & 31)) * LDK + kk]);
+      for (int n = 0; n < NT; ++n) acc[r][n] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    const uint16_t *row = input ? xbuf + col * xpitch + kq * 8 : b + col * pitch + kq * 8;
+    const int rp = input ? 16 * xpitch : 16 * pitch, chunk = input ? xw >> 5 : KT;
+    for (int k0 = 0; k0 < KT; k0 += chunk) {
+      if (input) {
+        const int cw = stage(k0 * 32);
+        if (TRAIN && keep) pack(xbuf, xpitch, cw, L[0].aT, k0 * 32);
+      }
+      const int ke = min(chunk, KT - k0);
+      for (int k = 0; k < ke; k += PD) {
 #pragma unroll
-      for (int a = 0; a < 2; ++a)
+        for (int p = 0; p < PD; ++p) {
+          if (k + p >= ke) break;
+          bf16x8 bv[NT];
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
-          acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[a], bfv[b], acc[a][b], 0, 0, 0);
-    }
-    __syncthreads();
-  }
-
-  // ---- epilogue
-  float *Cs = C + (EPI == 0 ? (long)blockIdx.z * M * ldc : 0);
+          for (int n = 0; n < NT; ++n)
+            bv[n] = *reinterpret_cast<const bf16x8 *>(row + n * rp + (k + p) * 32);
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+          for (int r = 0; r < cnt; ++r) {
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int m = m0 + wm + 32 * a + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-        const int n = n0 + wn + 32 * b + (lane & 31);
-        if (m >= M || n >= N) continue;
-        float x = acc[a][b][v];
-        if (EPI >= 1) x += bias[n];
-        if (EPI != 3) Cs[(long)m * ldc + n] = x;
-        if (EPI == 1 || EPI == 3) {
-          const float s = x / (1.f + expf(-x));
-          H[(long)m * ldc + n] = f2bf(s);
+            for (int n = 0; n < NT; ++n) acc[r][n] = mfma(a[p][r], bv[n], acc[r][n]);
+            a[p][r] = frag(wp, KT, tile[r], min(k0 + k + p + PD, KT - 1));
+          }
         }
       }
-}
+    }
+  };
+  auto product = [&](int cnt, const uint16_t *wp, int KT, int OT, int base, const uint16_t *b,
+                     bool input, bool keep) {
+    if constexpr (RT == 1) {
+      gemm(std::integral_constant<int, 1>{}, wp, KT, OT, base, b, input, keep);
+    } else {
+      static_assert(RT == 4, "");
+      if (cnt == 4) gemm(std::integral_constant<int, 4>{}, wp, KT, OT, base, b, input, keep);
+      else if (cnt == 3) gemm(std::integral_constant<int, 3>{}, wp, KT, OT, base, b, input, keep);
+      else if (cnt == 2) gemm(std::integral_constant<int, 2>{}, wp, KT, OT, base, b, input, keep);
+      else gemm(std::integral_constant<int, 1>{}, wp, KT, OT, base, b, input, keep);
+    }
+  };
 
-// sum of split-K partials (fixed order, deterministic)
-__global__ void splitk_reduce_kernel(const float *__restrict__ part, float *__restrict__ out,
-                                     long n, int splits) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  float s = 0.f;
-  for (int z = 0; z < splits; ++z) s += part[(long)z * n + t];
-  out[t] = s;
-}
-
-// dpre = dact * silu'(pre); dact is fp32 (loss grad) or accumulated; out bf16 + fp32
-__global__ void silu_backward_kernel(const float *__restrict__ dact, const float *__restrict__ pre,
-                                     uint16_t *__restrict__ dpre_bf, long n) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const float x = pre[t];
-  const float sg = 1.f / (1.f + expf(-x));
-  dpre_bf[t] = f2bf(dact[t] * sg * (1.f + x * (1.f - sg)));
-}
-
-// column sums db[n] = sum_m d[m][n]: 64 columns per block along the lanes,
-// 16 row groups (rows g, g+16, ...) summed in a fixed order (deterministic)
-__global__ __launch_bounds__(1024) void colsum_bf16_kernel(const uint16_t *__restrict__ d,
-                                                           float *__restrict__ db, int M, int N) {
-  __shared__ float part[16][64];
-  const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
-  const int n = blockIdx.x * 64 + lane;
-  float s = 0.f;
-  if (n < N)
-    for (int m = g; m < M; m += 16) s += bf2f(d[(long)m * N + n]);
-  part[g][lane] = s;
-  __syncthreads();
-  if (g == 0 && n < N) {
-    float t = part[0][lane];
+  // ---- forward
+  preload(L[0].wp, n_in / 32, L[0].out / 16, 0, tiles_of(L[0].out / 16));
+  for (int l = 0; l < nl; ++l) {
+    const bool last = l == nl - 1;
+    const int KT = L[l].in / 32, OT = L[l].out / 16, cnt = tiles_of(OT);
+    const uint16_t *wp = L[l].wp;
+    for (int base = 0; base < OT; base += WAVES * cnt) {
+      if (base) preload(wp, KT, OT, base, cnt);
+      product(cnt, wp, KT, OT, base, cur, l == 0, base == 0);
 #pragma unroll
-    for (int r = 1; r < 16; ++r) t += part[r][lane];
-    db[n] = t;
+      for (int r = 0; r < RT; ++r) {
+        const int tile = base + wave * cnt + r;
+        if (r >= cnt || tile >= OT) break;
+        const int o = tile * 16 + 4 * kq;
+        const f32x4 bias = *reinterpret_cast<const f32x4 *>(L[l].b + o);
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+          const int sl = 16 * n + col, s = s0 + sl;
+          f32x4 x = acc[r][n] + bias;
+          if (!last) {
+            if (TRAIN)
+              *reinterpret_cast<f32x4 *>(L[l].pre + ((long)blockIdx.x * OT + tile) * 256 +
+                                         lane * 4) = x;
+            f32x4 h;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) h[v] = x[v] / (1.f + expf(-x[v]));
+            *reinterpret_cast<uint2 *>(nxt + sl * pitch + o) = f2bf4(h);
+          } else if (TRAIN) {
+            const f32x4 t = *reinterpret_cast<const f32x4u *>(ls.T + (long)s * L[l].out + o);
+            f32x4 g;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+              const float d = x[v] - t[v];
+              g[v] = 2.f * d * ls.scale;
+            }
+            *reinterpret_cast<uint2 *>(nxt + sl * pitch + o) = f2bf4(g);
+            if (Y) *reinterpret_cast<f32x4u *>(Y + (long)s * L[l].out + o) = x;
+          } else if (s < M) {
+            *reinterpret_cast<f32x4u *>(Y + (long)s * L[l].out + o) = x;
+            if (fo.qrad) {
+              const Shape &sh = fo.sh;
+              const int ni = sh.It - 2 * sh.mi, cs = fo.col0 + s;
+              const int j = cs / ni, i = cs - j * ni;
+              const int c0 = sh.idx(sh.mi + i, sh.mj + j, sh.mk + o), st = sh.It * sh.Jt;
+              if (fo.flag && fo.flag[cs]) {  // fallback column: last plain-RT value
+#pragma unroll
+                for (int v = 0; v < 4; ++v) fo.qrad[c0 + v * st] = fo.q_rt[c0 + v * st];
+              } else {
+                const f32x4 mu = *reinterpret_cast<const f32x4 *>(fo.mu + o);
+                const f32x4 sd = *reinterpret_cast<const f32x4 *>(fo.sd + o);
+                double q[4];
+#pragma unroll
+                for (int v = 0; v < 4; ++v) q[v] = (double)(x[v] * sd[v] + mu[v]);
+                if (fo.corr) {
+#pragma unroll
+                  for (int v = 0; v < 4; ++v) q[v] += fo.corr[c0 + v * st];
+                }
+#pragma unroll
+                for (int v = 0; v < 4; ++v) fo.qrad[c0 + v * st] = q[v];
+              }
+            }
+          }
+        }
+      }
+    }
+    if (!last)
+      preload(L[l + 1].wp, L[l + 1].in / 32, L[l + 1].out / 16, 0, tiles_of(L[l + 1].out / 16));
+    else if (TRAIN && l > 0)
+      preload(L[l].wtp, L[l].out / 32, L[l].in / 16, 0, tiles_of(L[l].in / 16));
+    if (!last || TRAIN) {
+      __syncthreads();
+      if (TRAIN) pack(nxt, pitch, L[l].out, last ? L[l].dT : L[l + 1].aT, 0);
+      uint16_t *t = cur;
+      cur = nxt;
+      nxt = t;
+    }
+  }
+  if constexpr (TRAIN) {
+    // ---- back: the gradient of layer l's input, times silu' of layer l - 1
+    for (int l = nl - 1; l > 0; --l) {
+      const int KT = L[l].out / 32, OT = L[l].in / 16, cnt = tiles_of(OT);
+      const uint16_t *wp = L[l].wtp;
+      for (int base = 0; base < OT; base += WAVES * cnt) {
+        if (base) preload(wp, KT, OT, base, cnt);
+        product(cnt, wp, KT, OT, base, cur, false, false);
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+          const int tile = base + wave * cnt + r;
+          if (r >= cnt || tile >= OT) break;
+          const f32x4 x = *reinterpret_cast<const f32x4 *>(
+              L[l - 1].pre + ((long)blockIdx.x * OT + tile) * 256 + lane * 4);
+          f32x4 g;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const float sg = 1.f / (1.f + expf(-x[v]));
+            g[v] = acc[r][0][v] * sg * (1.f + x[v] * (1.f - sg));
+          }
+          *reinterpret_cast<uint2 *>(nxt + col * pitch + tile * 16 + 4 * kq) = f2bf4(g);
+        }
+      }
+      if (l > 1)
+        preload(L[l - 1].wtp, L[l - 1].out / 32, L[l - 1].in / 16, 0, tiles_of(L[l - 1].in / 16));
+      __syncthreads();
+      pack(nxt, pitch, L[l].in, L[l - 1].dT, 0);
+      uint16_t *t = cur;
+      cur = nxt;
+      nxt = t;
+    }
   }
 }
 
-// MSE loss on a batch: dY = 2 (Y - T) / (M N) (bf16), per-block partial losses
-__global__ void mse_kernel(const float *__restrict__ Y, const float *__restrict__ T,
-                           uint16_t *__restrict__ dY, float *__restrict__ part, long n,
-                           float scale) {
+// Weight and bias gradients of every layer in one launch: gW = dpre^T a, the
+// batch as k, a wave per 32 x 32 tile with eight k-steps of its operands in
+// flight; then a wave per 32 biases.  `per` k-steps go into a sum of their own
+// (a sixteenth of the batch where that divides), so that no chain of
+// additions grows with the batch, and these sums are added in order; a bias
+// is 16 sums, of every 16th column each, added in order.
+// Bound by the operands' way from L2 (64 bytes a clock and CU): 80 MB at a
+// batch of 1024 and 1536-256-256-256-384: 10.5 us, where a launch per layer
+// that transposed through LDS, its partial sums in memory and column sums by
+// four workgroups took 134.
+__global__ __launch_bounds__(64) void mlp_wgrad_kernel(const MlpLayer *__restrict__ L, int nl,
+                                                       int SB, int per, int tiles) {
+  const int lane = threadIdx.x, row = lane & 15, kq = lane >> 4;
+  int blk = blockIdx.x, l = 0;
+  if (blk >= tiles) {  // lane: bias o, octets of columns of one parity
+    blk -= tiles;
+    while (blk >= L[l].out / 32) blk -= L[l++].out / 32;
+    const int o = lane & 31, par = lane >> 5;
+    const uint16_t *d = L[l].dT + ((long)(2 * blk + (o >> 4)) * SB * 64 + (o & 15)) * 8;
+    float s[8] = {};
+#pragma unroll 8
+    for (int q = par; q < 4 * SB; q += 2) {
+      const uint4 v = *reinterpret_cast<const uint4 *>(d + ((long)(q >> 2) * 64 + 16 * (q & 3)) * 8);
+      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        s[e] += __uint_as_float(e & 1 ? w[e >> 1] & 0xffff0000u : w[e >> 1] << 16);
+    }
+    float t = s[0];
+#pragma unroll
+    for (int e = 1; e < 8; ++e) t += s[e];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) t += __shfl(s[e], lane | 32, 64);
+    if (par == 0) L[l].gb[32 * blk + o] = t;
+    return;
+  }
+  while (l + 1 < nl && blk >= L[l + 1].tile0) ++l;
+  const int I = L[l].in, nti = I / 32;
+  const int t = blk - L[l].tile0, to = t / nti, ti = t - to * nti;
+  const uint16_t *pa[2], *pb[2];
+#pragma unroll
+  for (int x = 0; x < 2; ++x) {
+    pa[x] = L[l].dT + (long)(to * 2 + x) * SB * 512 + lane * 8;
+    pb[x] = L[l].aT + (long)(ti * 2 + x) * SB * 512 + lane * 8;
+  }
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4 acc[2][2], sum[2][2];
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y) acc[x][y] = sum[x][y] = zero;
+  constexpr int PD = 8;
+  bf16x8 a[PD][2], b[PD][2];
+  auto load = [&](int p, int s) {
+    s = min(s, SB - 1);
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      a[p][x] = *reinterpret_cast<const bf16x8 *>(pa[x] + (long)s * 512);
+      b[p][x] = *reinterpret_cast<const bf16x8 *>(pb[x] + (long)s * 512);
+    }
+  };
+#pragma unroll
+  for (int p = 0; p < PD; ++p) load(p, p);
+  int c = 0;
+  for (int s = 0; s < SB; s += PD)
+#pragma unroll
+    for (int p = 0; p < PD; ++p) {
+      if (s + p >= SB) break;
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) acc[x][y] = mfma(a[p][x], b[p][y], acc[x][y]);
+      load(p, s + p + PD);
+      if (++c == per && per < SB) {
+        c = 0;
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+          for (int y = 0; y < 2; ++y) {
+            sum[x][y] += acc[x][y];
+            acc[x][y] = zero;
+          }
+      }
+    }
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y) {
+      const f32x4 g = per < SB ? sum[x][y] : acc[x][y];
+      float *gw = L[l].gw + (long)(to * 32 + x * 16 + 4 * kq) * I + ti * 32 + y * 16 + row;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) gw[(long)v * I] = g[v];
+    }
+}
+
+// sums of squares of the misses, 256 consecutive values of the batch each
+__global__ __launch_bounds__(256) void mlp_loss_kernel(const float *__restrict__ Y,
+                                                       const float *__restrict__ T,
+                                                       float *__restrict__ part, long n) {
   __shared__ float red[256];
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  float e = 0.f;
-  if (t < n) {
-    const float d = Y[t] - T[t];
-    dY[t] = f2bf(2.f * d * scale);
-    e = d * d;
-  }
-  red[threadIdx.x] = e;
+  const long t = (long)blockIdx.x * 256 + threadIdx.x;
+  const float d = t < n ? Y[t] - T[t] : 0.f;
+  red[threadIdx.x] = d * d;
   __syncthreads();
   for (int s = 128; s > 0; s >>= 1) {
     if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
@@ -217,27 +413,69 @@ __global__ void mse_kernel(const float *__restrict__ Y, const float *__restrict_
   if (threadIdx.x == 0) part[blockIdx.x] = red[0];
 }
 
-// Adam on fp32 master weights, then the bf16 copy used by the GEMMs
-__global__ void adam_kernel(float *__restrict__ w, uint16_t *__restrict__ wb,
-                            const float *__restrict__ g, float *__restrict__ m1,
-                            float *__restrict__ m2, long n, float lr, float b1, float b2,
-                            float eps, float c1, float c2, float wd) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const float gr = g[t] + wd * w[t];
-  const float a = b1 * m1[t] + (1.f - b1) * gr;
-  const float b = b2 * m2[t] + (1.f - b2) * gr * gr;
-  m1[t] = a;
-  m2[t] = b;
-  const float upd = (a / c1) / (sqrtf(b / c2) + eps);
-  const float nw = w[t] - lr * upd;
-  w[t] = nw;
-  if (wb) wb[t] = f2bf(nw);
+__device__ __forceinline__ float adam_step(float &w, float g, float &m1, float &m2,
+                                           const MlpAdam &p, float wd) {
+  const float gr = g + wd * w;
+  const float a = p.b1 * m1 + (1.f - p.b1) * gr;
+  const float b = p.b2 * m2 + (1.f - p.b2) * gr * gr;
+  m1 = a;
+  m2 = b;
+  const float upd = (a / p.c1) / (sqrtf(b / p.c2) + p.eps);
+  w = w - p.lr * upd;
+  return w;
 }
 
-__global__ void to_bf16_kernel(const float *__restrict__ x, uint16_t *__restrict__ y, long n) {
-  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) y[t] = f2bf(x[t]);
+// Adam on the fp32 master weights and biases of the layers from l0 on, a
+// workgroup per 32 x 32 tile, and the two packed bf16 copies of the tile: wp
+// (rows = outputs, k = inputs) for the forward product, wtp (rows = inputs, k
+// = outputs) for the way back.  UPDATE false: the copies alone.
+// Bound by HBM or the last-level cache, 32 bytes a weight: 6.2 us for 622592
+// weights (28 as eight launches).
+template <bool UPDATE>
+__global__ __launch_bounds__(256) void mlp_adam_kernel(const MlpLayer *__restrict__ L, int nl,
+                                                       int l0, MlpAdam p) {
+  __shared__ __attribute__((aligned(16))) uint16_t tile[32][40];
+  const int blk = blockIdx.x + L[l0].tile0;
+  int l = l0;
+  while (l + 1 < nl && blk >= L[l + 1].tile0) ++l;
+  const int I = L[l].in, O = L[l].out, nti = I / 32;
+  const int t = blk - L[l].tile0, to = t / nti, ti = t - to * nti;
+  const int tid = threadIdx.x, r = tid >> 3, c = 4 * (tid & 7);
+  const long at = (long)(to * 32 + r) * I + ti * 32 + c;
+  f32x4 w = *reinterpret_cast<const f32x4 *>(L[l].w + at);
+  if (UPDATE) {
+    const f32x4 g = *reinterpret_cast<const f32x4 *>(L[l].gw + at);
+    f32x4 m1 = *reinterpret_cast<const f32x4 *>(L[l].mw + at);
+    f32x4 m2 = *reinterpret_cast<const f32x4 *>(L[l].vw + at);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      float x = w[v], y = m1[v], z = m2[v];
+      adam_step(x, g[v], y, z, p, p.wd);
+      w[v] = x; m1[v] = y; m2[v] = z;
+    }
+    *reinterpret_cast<f32x4 *>(L[l].w + at) = w;
+    *reinterpret_cast<f32x4 *>(L[l].mw + at) = m1;
+    *reinterpret_cast<f32x4 *>(L[l].vw + at) = m2;
+    if (ti == 0 && tid < 32) {
+      const int o = to * 32 + tid;
+      adam_step(L[l].b[o], L[l].gb[o], L[l].mb[o], L[l].vb[o], p, 0.f);
+    }
+  }
+  *reinterpret_cast<uint2 *>(&tile[r][c]) = f2bf4(w);
+  __syncthreads();
+  const int lane = tid & 63, row = lane & 15, k = 8 * (lane >> 4), h = (tid >> 6) & 1;
+  if (tid < 128) {
+    *reinterpret_cast<uint4 *>(L[l].wp + ((long)(to * 2 + h) * nti + ti) * 512 + lane * 8) =
+        *reinterpret_cast<const uint4 *>(&tile[16 * h + row][k]);
+  } else {
+    uint32_t v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      v[e] = (uint32_t)tile[k + 2 * e][16 * h + row] |
+             (uint32_t)tile[k + 2 * e + 1][16 * h + row] << 16;
+    *reinterpret_cast<uint4 *>(L[l].wtp + ((long)(ti * 2 + h) * (O / 32) + to) * 512 + lane * 8) =
+        make_uint4(v[0], v[1], v[2], v[3]);
+  }
 }
 
 // Column features of the radiative box: for column (i, j) and cell kz of the
@@ -299,42 +537,6 @@ __global__ __launch_bounds__(256) void column_features_kernel(
   }
 }
 
-// Q_rad field from the network output: qrad = y * sd_q[kz] + mu_q[kz]
-// (+ corr, the column correction the last plain solve left).  Tiled like
-// the features: Y rows (heights of a column) are read along the heights,
-// the field is written along x.
-__global__ __launch_bounds__(256) void column_output_kernel(
-    const float *__restrict__ Y, Shape sh, const float *__restrict__ mu,
-    const float *__restrict__ sd, const int *__restrict__ flag, const double *__restrict__ q_rt,
-    const double *__restrict__ corr, double *__restrict__ qrad) {
-  __shared__ float tile[FT_Z][FT_X + 1];
-  const int ni = sh.It - 2 * sh.mi, nz = sh.Kt - 2 * sh.mk;
-  const int i0 = blockIdx.x * FT_X, j = blockIdx.y, kz0 = blockIdx.z * FT_Z;
-  {
-    const int zl = threadIdx.x & (FT_Z - 1), pr = threadIdx.x / FT_Z;
-    const int kz = kz0 + zl;
-    for (int il = pr; il < FT_X; il += 256 / FT_Z)
-      if (i0 + il < ni && kz < nz) tile[zl][il] = Y[((long)j * ni + i0 + il) * nz + kz];
-  }
-  __syncthreads();
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int i = i0 + lane;
-  if (i >= ni) return;
-  const long col = (long)j * ni + i;
-  const bool fallback = flag && flag[col];
-  for (int r = wv; r < FT_Z; r += 4) {
-    const int kz = kz0 + r;
-    if (kz >= nz) break;
-    const int c = sh.idx(sh.mi + i, sh.mj + j, sh.mk + kz);
-    if (fallback) {
-      qrad[c] = q_rt[c];  // fallback column: last plain-RT value
-      continue;
-    }
-    const double net = (double)(tile[r][lane] * sd[kz] + mu[kz]);
-    qrad[c] = corr ? net + corr[c] : net;
-  }
-}
-
 // residual indicator per column: relative L2 of (mlp - rt) over the column
 // above `tol` -> flag = 1; corr (optional) receives rt - mlp on every cell
 __global__ void column_residual_kernel(const float *__restrict__ Y, Shape sh,
@@ -358,73 +560,93 @@ __global__ void column_residual_kernel(const float *__restrict__ Y, Shape sh,
 }
 
 // ------------------------------------------------------------- launchers
-template <bool TA, bool TB, int EPI>
-static hipError_t gemm_t(hipStream_t st, const uint16_t *A, const uint16_t *B, float *C,
-                         uint16_t *H, const float *bias, int M, int N, int K, int lda, int ldb,
-                         int ldc, int splits) {
-  const int kps = ((K / splits + BK - 1) / BK) * BK;
-  const int nz = (K + kps - 1) / kps;
-  dim3 grid((M + BM - 1) / BM, (N + BN - 1) / BN, nz);
-  hipLaunchKernelGGL((gemm_bf16_kernel<TA, TB, EPI>), grid, dim3(256), 0, st, A, B, C, H, bias, M,
-                     N, K, lda, ldb, ldc, kps);
-  return hipGetLastError();
+namespace {
+
+// columns from which inference takes 64 to a workgroup: fewer leave CUs idle
+constexpr int MLP_TALL = 8192;
+constexpr int LDS_BYTES = 160 * 1024;
+// features of X that a 16-column workgroup stages at a time
+int x_width(int n_in) { return n_in < 2048 ? n_in : 2048; }
+// LDS of a workgroup of ns columns: two activation buffers of width bw (none
+// where they live in global memory) and, beside them, xw features of X
+size_t chain_lds(int ns, int bw, int xw) {
+  return sizeof(uint16_t) * ns * ((bw ? 2 * (bw + 8) : 0) + (xw ? xw + 8 : 0));
 }
 
-hipError_t launch_gemm_bf16(hipStream_t st, int ta, int tb, int epi, const uint16_t *A,
-                            const uint16_t *B, float *C, uint16_t *H, const float *bias, int M,
-                            int N, int K, int lda, int ldb, int ldc, int splits) {
-  if (K % BK) return hipErrorInvalidValue;
-  if (splits < 1) splits = 1;
-  if (epi != 0 && splits != 1) return hipErrorInvalidValue;
-  if (!ta && tb) {
-    if (epi == 0) return gemm_t<false, true, 0>(st, A, B, C, H, bias, M, N, K, lda, ldb, ldc, splits);
-    if (epi == 1) return gemm_t<false, true, 1>(st, A, B, C, H, bias, M, N, K, lda, ldb, ldc, 1);
-    if (epi == 3) return gemm_t<false, true, 3>(st, A, B, C, H, bias, M, N, K, lda, ldb, ldc, 1);
-    return gemm_t<false, true, 2>(st, A, B, C, H, bias, M, N, K, lda, ldb, ldc, 1);
+template <int NT, int WAVES, int RT, int PD, bool TRAIN, bool WIDE>
+hipError_t chain(hipStream_t st, const MlpLayer *L, int nl, const uint16_t *X, int M, float *Y,
+                 const MlpLoss &ls, const MlpField &fo, uint16_t *g0, uint16_t *g1, int bw,
+                 int xoff, int xw, size_t bytes) {
+  auto k = mlp_chain_kernel<NT, WAVES, RT, PD, TRAIN, WIDE>;
+  if (bytes > 65536) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e != hipSuccess) return e;
   }
-  if (!ta && !tb) return gemm_t<false, false, 0>(st, A, B, C, H, bias, M, N, K, lda, ldb, ldc, splits);
-  if (ta && !tb) return gemm_t<true, false, 0>(st, A, B, C, H, bias, M, N, K, lda, ldb, ldc, splits);
-  return gemm_t<true, true, 0>(st, A, B, C, H, bias, M, N, K, lda, ldb, ldc, splits);
-}
-
-hipError_t launch_splitk_reduce(hipStream_t st, const float *part, float *out, long n,
-                                int splits) {
-  hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
-                     part, out, n, splits);
+  hipLaunchKernelGGL(k, dim3((M + 16 * NT - 1) / (16 * NT)), dim3(64 * WAVES), bytes, st, L, nl,
+                     X, M, Y, ls, fo, g0, g1, bw, xoff, xw);
   return hipGetLastError();
 }
 
-hipError_t launch_silu_backward(hipStream_t st, const float *dact, const float *pre,
-                                uint16_t *dpre, long n) {
-  hipLaunchKernelGGL(silu_backward_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
-                     dact, pre, dpre, n);
+}  // namespace
+
+bool mlp_is_wide(int n_in, int maxw) {
+  return chain_lds(16, maxw, x_width(n_in)) + 1024 > (size_t)LDS_BYTES;
+}
+
+hipError_t launch_mlp_forward(hipStream_t st, const MlpLayer *L, int nl, int n_in, int n_hidden,
+                              bool wide, int maxw, const uint16_t *X, int M, float *Y,
+                              const MlpField &fo, uint16_t *g0, uint16_t *g1) {
+  const MlpLoss none{};
+  // X passes through the second buffer (the input layer writes the first),
+  // in chunks of whole rounds of the two k-steps in flight
+  const int xt = (n_hidden + 63) / 64 * 64;
+  const size_t tall = sizeof(uint16_t) * 64 * (n_hidden + 8 + xt + 8);
+  if (M >= MLP_TALL && tall <= (size_t)LDS_BYTES)
+    return chain<4, 4, 4, 2, false, false>(st, L, nl, X, M, Y, none, fo, g0, g1, n_hidden,
+                                           64 * (n_hidden + 8), xt, tall);
+  const int xw = x_width(n_in);
+  if (wide)
+    return chain<1, 16, 1, 8, false, true>(st, L, nl, X, M, Y, none, fo, g0, g1, maxw, 0, xw,
+                                           chain_lds(16, 0, xw));
+  return chain<1, 16, 1, 8, false, false>(st, L, nl, X, M, Y, none, fo, g0, g1, maxw,
+                                          32 * (maxw + 8), xw, chain_lds(16, maxw, xw));
+}
+
+hipError_t launch_mlp_grad(hipStream_t st, const MlpLayer *L, int nl, int n_in, bool wide,
+                           int maxw, int tiles, int bias_tiles, const uint16_t *X, int M,
+                           const MlpLoss &ls, float *Y, uint16_t *g0, uint16_t *g1) {
+  const MlpField none{};
+  const int xw = x_width(n_in);
+  hipError_t e =
+      wide ? chain<1, 16, 1, 8, true, true>(st, L, nl, X, M, Y, ls, none, g0, g1, maxw, 0, xw,
+                                            chain_lds(16, 0, xw))
+           : chain<1, 16, 1, 8, true, false>(st, L, nl, X, M, Y, ls, none, g0, g1, maxw,
+                                             32 * (maxw + 8), xw, chain_lds(16, maxw, xw));
+  if (e != hipSuccess) return e;
+  int splits = 16;  // equal sums of whole k-steps
+  while (M % (32 * splits)) --splits;
+  hipLaunchKernelGGL(mlp_wgrad_kernel, dim3(tiles + bias_tiles), dim3(64), 0, st, L, nl, M / 32,
+                     M / 32 / splits, tiles);
   return hipGetLastError();
 }
 
-hipError_t launch_colsum_bf16(hipStream_t st, const uint16_t *d, float *db, int M, int N) {
-  hipLaunchKernelGGL(colsum_bf16_kernel, dim3((N + 63) / 64), dim3(1024), 0, st, d, db, M, N);
+hipError_t launch_mlp_loss(hipStream_t st, const float *Y, const float *T, float *part, long n,
+                           int *parts) {
+  *parts = (int)((n + 255) / 256);
+  hipLaunchKernelGGL(mlp_loss_kernel, dim3(*parts), dim3(256), 0, st, Y, T, part, n);
   return hipGetLastError();
 }
 
-hipError_t launch_mse(hipStream_t st, const float *Y, const float *T, uint16_t *dY, float *part,
-                      long n, float scale, int *nblocks) {
-  const int nb = (int)((n + 255) / 256);
-  *nblocks = nb;
-  hipLaunchKernelGGL(mse_kernel, dim3(nb), dim3(256), 0, st, Y, T, dY, part, n, scale);
+hipError_t launch_mlp_adam(hipStream_t st, const MlpLayer *L, int nl, int tiles,
+                           const MlpAdam &p) {
+  hipLaunchKernelGGL((mlp_adam_kernel<true>), dim3(tiles), dim3(256), 0, st, L, nl, 0, p);
   return hipGetLastError();
 }
 
-hipError_t launch_adam(hipStream_t st, float *w, uint16_t *wb, const float *g, float *m1,
-                       float *m2, long n, float lr, float b1, float b2, float eps, float c1,
-                       float c2, float wd) {
-  hipLaunchKernelGGL(adam_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, w, wb, g,
-                     m1, m2, n, lr, b1, b2, eps, c1, c2, wd);
-  return hipGetLastError();
-}
-
-hipError_t launch_to_bf16(hipStream_t st, const float *x, uint16_t *y, long n) {
-  hipLaunchKernelGGL(to_bf16_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, x, y,
-                     n);
+hipError_t launch_mlp_pack(hipStream_t st, const MlpLayer *L, int nl, int layer, int tiles) {
+  hipLaunchKernelGGL((mlp_adam_kernel<false>), dim3(tiles), dim3(256), 0, st, L, nl, layer,
+                     MlpAdam{});
   return hipGetLastError();
 }
 
@@ -436,16 +658,6 @@ hipError_t launch_column_features(hipStream_t st, const Fld<const double> &q, co
   dim3 grid((ni + FT_X - 1) / FT_X, nj, (nz + FT_Z - 1) / FT_Z);
   hipLaunchKernelGGL(column_features_kernel, grid, dim3(256), 0, st, q, sh, gm, mu, sd, X, Xf,
                      nfeat, h);
-  return hipGetLastError();
-}
-
-hipError_t launch_column_output(hipStream_t st, const float *Y, const Shape &sh, const float *mu,
-                                const float *sd, const int *flag, const double *q_rt,
-                                const double *corr, double *qrad) {
-  const int ni = sh.It - 2 * sh.mi, nj = sh.Jt - 2 * sh.mj, nz = sh.Kt - 2 * sh.mk;
-  dim3 grid((ni + FT_X - 1) / FT_X, nj, (nz + FT_Z - 1) / FT_Z);
-  hipLaunchKernelGGL(column_output_kernel, grid, dim3(256), 0, st, Y, sh, mu, sd, flag, q_rt, corr,
-                     qrad);
   return hipGetLastError();
 }
 

@@ -1,50 +1,27 @@
 // C ABI of the per-column MLP surrogate (include/misohip.h, misohip_mlp_*).
-// The library owns the network state; every GEMM is the bf16 MFMA kernel of
-// mlp.hip, every elementwise step a kernel of the same file.
+// The library owns the network state; the network, its gradients and its
+// update are kernels of mlp.hip.
 #include <cmath>
 #include <cstring>
 #include <new>
 #include <vector>
 
 #include "ctx_internal.hpp"
-#include "launch.hpp"
+#include "mlp.hpp"
 
 using namespace misohip;
-
-namespace misohip {
-hipError_t launch_gemm_bf16(hipStream_t, int, int, int, const uint16_t *, const uint16_t *,
-                            float *, uint16_t *, const float *, int, int, int, int, int, int, int);
-hipError_t launch_splitk_reduce(hipStream_t, const float *, float *, long, int);
-hipError_t launch_silu_backward(hipStream_t, const float *, const float *, uint16_t *, long);
-hipError_t launch_colsum_bf16(hipStream_t, const uint16_t *, float *, int, int);
-hipError_t launch_mse(hipStream_t, const float *, const float *, uint16_t *, float *, long, float,
-                      int *);
-hipError_t launch_adam(hipStream_t, float *, uint16_t *, const float *, float *, float *, long,
-                       float, float, float, float, float, float, float);
-hipError_t launch_to_bf16(hipStream_t, const float *, uint16_t *, long);
-hipError_t launch_column_features(hipStream_t, const Fld<const double> &, const Shape &, double,
-                                  const float *, const float *, uint16_t *, float *, int, int);
-hipError_t launch_column_output(hipStream_t, const float *, const Shape &, const float *,
-                                const float *, const int *, const double *, const double *,
-                                double *);
-hipError_t launch_column_residual(hipStream_t, const float *, const Shape &, const float *,
-                                  const float *, const double *, int *, float, double *);
-}  // namespace misohip
 
 struct misohip_mlp {
   int n_in, n_hidden, n_out, n_layers;  // n_layers = hidden layers + output layer
   int max_batch;
-  int splits;
+  int maxw;    // the widest activation
+  bool wide;   // activations in g0, g1 instead of LDS
+  int tiles, bias_tiles;
   long t;  // Adam step
-  std::vector<int> in, out;
-  std::vector<float *> w, b, gw, gb, mw, vw, mb, vb;
-  std::vector<uint16_t *> wb;
-  std::vector<float *> pre;      // [max_batch][out_l] fp32
-  std::vector<uint16_t *> act;   // [max_batch][out_l] bf16 (hidden layers)
-  float *dact = nullptr;         // [max_batch][max width] fp32
-  uint16_t *dpre = nullptr;      // [max_batch][max width] bf16
-  uint16_t *dpre2 = nullptr;
-  float *part = nullptr;         // split-K partials
+  std::vector<MlpLayer> layer;
+  MlpLayer *d_layer = nullptr;   // the same, on the device
+  uint16_t *g0 = nullptr, *g1 = nullptr;
+  float *y = nullptr;            // the network's output where the loss is asked for
   float *loss_part = nullptr;
   float *h_loss = nullptr;       // pinned
   float *mu_in = nullptr, *sd_in = nullptr, *mu_out = nullptr, *sd_out = nullptr;
@@ -63,49 +40,10 @@ template <typename T> hipError_t alloc(misohip_mlp *m, T **p, size_t n) {
   return e;
 }
 
-// keep_pre: store the hidden layers' pre-activations (the backward pass
-// reads them; inference does not need them)
 int forward(misohip_ctx *ctx, misohip_mlp *m, const uint16_t *X, int batch, float *Y,
-            bool keep_pre = true) {
-  const uint16_t *inp = X;
-  for (int l = 0; l < m->n_layers; ++l) {
-    const bool last = l == m->n_layers - 1;
-    float *C = last && Y ? Y : m->pre[l];
-    MISOHIP_TRY(launch_gemm_bf16(ctx->stream, 0, 1, last ? 2 : keep_pre ? 1 : 3, inp, m->wb[l], C,
-                                 last ? nullptr : m->act[l], m->b[l], batch, m->out[l], m->in[l],
-                                 m->in[l], m->in[l], m->out[l], 1));
-    inp = m->act[l];
-  }
-  return MISOHIP_OK;
-}
-
-// gradients of all weights from dpre of the output layer (bf16, in m->dpre)
-int backward(misohip_ctx *ctx, misohip_mlp *m, const uint16_t *X, int batch) {
-  uint16_t *dcur = m->dpre, *dnext = m->dpre2;
-  for (int l = m->n_layers - 1; l >= 0; --l) {
-    const uint16_t *inp = l == 0 ? X : m->act[l - 1];
-    const int O = m->out[l], I = m->in[l];
-    // gW = dpre^T * inp  ([O][I], reduction over the batch, split over K)
-    // split the batch reduction into equal multiples of 32 (or not at all)
-    int splits = m->splits;
-    while (splits > 1 && (batch % splits || (batch / splits) % 32)) --splits;
-    if (splits > 1) {
-      MISOHIP_TRY(launch_gemm_bf16(ctx->stream, 1, 0, 0, dcur, inp, m->part, nullptr, nullptr, O,
-                                   I, batch, O, I, I, splits));
-      MISOHIP_TRY(launch_splitk_reduce(ctx->stream, m->part, m->gw[l], (long)O * I, splits));
-    } else {
-      MISOHIP_TRY(launch_gemm_bf16(ctx->stream, 1, 0, 0, dcur, inp, m->gw[l], nullptr, nullptr, O,
-                                   I, batch, O, I, I, 1));
-    }
-    MISOHIP_TRY(launch_colsum_bf16(ctx->stream, dcur, m->gb[l], batch, O));
-    if (l > 0) {
-      // dact = dpre * W  ([batch][I]); dpre_prev = dact * silu'(pre_prev)
-      MISOHIP_TRY(launch_gemm_bf16(ctx->stream, 0, 0, 0, dcur, m->wb[l], m->dact, nullptr,
-                                   nullptr, batch, I, O, O, I, I, 1));
-      MISOHIP_TRY(launch_silu_backward(ctx->stream, m->dact, m->pre[l - 1], dnext, (long)batch * I));
-      std::swap(dcur, dnext);
-    }
-  }
+            const MlpField &field) {
+  MISOHIP_TRY(launch_mlp_forward(ctx->stream, m->d_layer, m->n_layers, m->n_in, m->n_hidden,
+                                 m->wide, m->maxw, X, batch, Y, field, m->g0, m->g1));
   return MISOHIP_OK;
 }
 
@@ -141,48 +79,49 @@ int misohip_mlp_create(misohip_ctx *ctx, int n_in, int n_hidden, int n_hidden_la
   m->n_out = n_out;
   m->n_layers = n_hidden_layers + 1;
   m->max_batch = max_batch;
-  m->splits = 16;
   m->t = 0;
-  int maxw = n_hidden > n_out ? n_hidden : n_out;
-  if (n_in > maxw) maxw = n_in;
+  m->maxw = n_hidden > n_out ? n_hidden : n_out;
+  m->wide = mlp_is_wide(n_in, m->maxw);
+  m->tiles = m->bias_tiles = 0;
   hipError_t e = hipSuccess;
   for (int l = 0; l < m->n_layers && e == hipSuccess; ++l) {
+    const bool last = l == m->n_layers - 1;
     const int I = l == 0 ? n_in : n_hidden;
-    const int O = l == m->n_layers - 1 ? n_out : n_hidden;
-    m->in.push_back(I);
-    m->out.push_back(O);
-    float *p[8] = {};
-    uint16_t *pb = nullptr;
+    const int O = last ? n_out : n_hidden;
     const size_t nw = (size_t)O * I;
-    e = alloc(m, &p[0], nw);
-    if (e == hipSuccess) e = alloc(m, &p[1], O);
-    if (e == hipSuccess) e = alloc(m, &p[2], nw);
-    if (e == hipSuccess) e = alloc(m, &p[3], O);
-    if (e == hipSuccess) e = alloc(m, &p[4], nw);
-    if (e == hipSuccess) e = alloc(m, &p[5], nw);
-    if (e == hipSuccess) e = alloc(m, &p[6], O);
-    if (e == hipSuccess) e = alloc(m, &p[7], O);
-    if (e == hipSuccess) e = alloc(m, &pb, nw);
-    m->w.push_back(p[0]); m->b.push_back(p[1]); m->gw.push_back(p[2]); m->gb.push_back(p[3]);
-    m->mw.push_back(p[4]); m->vw.push_back(p[5]); m->mb.push_back(p[6]); m->vb.push_back(p[7]);
-    m->wb.push_back(pb);
-    float *pre = nullptr;
-    uint16_t *act = nullptr;
-    if (e == hipSuccess) e = alloc(m, &pre, (size_t)max_batch * O);
-    if (e == hipSuccess && l < m->n_layers - 1) e = alloc(m, &act, (size_t)max_batch * O);
-    m->pre.push_back(pre);
-    m->act.push_back(act);
+    MlpLayer y{};
+    y.in = I;
+    y.out = O;
+    y.tile0 = m->tiles;
+    m->tiles += (O / 32) * (I / 32);
+    m->bias_tiles += O / 32;
+    for (float **p : {&y.w, &y.gw, &y.mw, &y.vw})
+      if (e == hipSuccess) e = alloc(m, p, nw);
+    for (float **p : {&y.b, &y.gb, &y.mb, &y.vb})
+      if (e == hipSuccess) e = alloc(m, p, O);
+    for (uint16_t **p : {&y.wp, &y.wtp})
+      if (e == hipSuccess) e = alloc(m, p, nw);
+    if (e == hipSuccess && !last) e = alloc(m, &y.pre, (size_t)max_batch * O);
+    if (e == hipSuccess) e = alloc(m, &y.aT, (size_t)max_batch * I);
+    if (e == hipSuccess) e = alloc(m, &y.dT, (size_t)max_batch * O);
+    m->layer.push_back(y);
   }
-  if (e == hipSuccess) e = alloc(m, &m->dact, (size_t)max_batch * maxw);
-  if (e == hipSuccess) e = alloc(m, &m->dpre, (size_t)max_batch * maxw);
-  if (e == hipSuccess) e = alloc(m, &m->dpre2, (size_t)max_batch * maxw);
-  if (e == hipSuccess) e = alloc(m, &m->part, (size_t)m->splits * maxw * maxw);
+  if (e == hipSuccess) e = alloc(m, &m->d_layer, m->layer.size());
+  if (e == hipSuccess)
+    e = hipMemcpy(m->d_layer, m->layer.data(), sizeof(MlpLayer) * m->layer.size(),
+                  hipMemcpyHostToDevice);
+  if (m->wide) {
+    if (e == hipSuccess) e = alloc(m, &m->g0, (size_t)max_batch * (m->maxw + 8));
+    if (e == hipSuccess) e = alloc(m, &m->g1, (size_t)max_batch * (m->maxw + 8));
+  }
   if (e == hipSuccess) e = alloc(m, &m->loss_part, (size_t)max_batch * n_out / 256 + 1);
+  if (e == hipSuccess) e = alloc(m, &m->y, (size_t)max_batch * n_out);
   if (e == hipSuccess) e = alloc(m, &m->mu_in, n_in);
   if (e == hipSuccess) e = alloc(m, &m->sd_in, n_in);
   if (e == hipSuccess) e = alloc(m, &m->mu_out, n_out);
   if (e == hipSuccess) e = alloc(m, &m->sd_out, n_out);
-  if (e == hipSuccess) e = hipHostMalloc(&m->h_loss, sizeof(float) * ((size_t)max_batch * n_out / 256 + 1), hipHostMallocDefault);
+  if (e == hipSuccess)
+    e = hipHostMalloc(&m->h_loss, sizeof(float) * ((size_t)max_batch * n_out / 256 + 1), hipHostMallocDefault);
   if (e != hipSuccess) {
     for (void *q : m->allocs) (void)hipFree(q);
     delete m;
@@ -205,14 +144,15 @@ int misohip_mlp_set_layer(misohip_ctx *ctx, misohip_mlp *m, int layer, const flo
                           const float *b_host) {
   if (!ctx || !m || layer < 0 || layer >= m->n_layers || !w_host || !b_host) return MISOHIP_E_ARG;
   MISOHIP_TRY(hipSetDevice(ctx->device));
-  const size_t nw = (size_t)m->out[layer] * m->in[layer];
-  MISOHIP_TRY(hipMemcpy(m->w[layer], w_host, sizeof(float) * nw, hipMemcpyHostToDevice));
-  MISOHIP_TRY(hipMemcpy(m->b[layer], b_host, sizeof(float) * m->out[layer], hipMemcpyHostToDevice));
-  MISOHIP_TRY(launch_to_bf16(ctx->stream, m->w[layer], m->wb[layer], (long)nw));
-  MISOHIP_TRY(hipMemsetAsync(m->mw[layer], 0, sizeof(float) * nw, ctx->stream));
-  MISOHIP_TRY(hipMemsetAsync(m->vw[layer], 0, sizeof(float) * nw, ctx->stream));
-  MISOHIP_TRY(hipMemsetAsync(m->mb[layer], 0, sizeof(float) * m->out[layer], ctx->stream));
-  MISOHIP_TRY(hipMemsetAsync(m->vb[layer], 0, sizeof(float) * m->out[layer], ctx->stream));
+  const MlpLayer &y = m->layer[layer];
+  const size_t nw = (size_t)y.out * y.in;
+  MISOHIP_TRY(hipMemcpy(y.w, w_host, sizeof(float) * nw, hipMemcpyHostToDevice));
+  MISOHIP_TRY(hipMemcpy(y.b, b_host, sizeof(float) * y.out, hipMemcpyHostToDevice));
+  MISOHIP_TRY(launch_mlp_pack(ctx->stream, m->d_layer, m->n_layers, layer, (int)(nw / 1024)));
+  MISOHIP_TRY(hipMemsetAsync(y.mw, 0, sizeof(float) * nw, ctx->stream));
+  MISOHIP_TRY(hipMemsetAsync(y.vw, 0, sizeof(float) * nw, ctx->stream));
+  MISOHIP_TRY(hipMemsetAsync(y.mb, 0, sizeof(float) * y.out, ctx->stream));
+  MISOHIP_TRY(hipMemsetAsync(y.vb, 0, sizeof(float) * y.out, ctx->stream));
   MISOHIP_TRY(hipStreamSynchronize(ctx->stream));
   m->t = 0;
   return MISOHIP_OK;
@@ -224,10 +164,10 @@ int misohip_mlp_get_layer(misohip_ctx *ctx, misohip_mlp *m, int layer, int which
     return MISOHIP_E_ARG;
   MISOHIP_TRY(hipSetDevice(ctx->device));
   MISOHIP_TRY(hipStreamSynchronize(ctx->stream));
-  const size_t nw = (size_t)m->out[layer] * m->in[layer];
-  const float *src = which == 0 ? m->w[layer] : which == 1 ? m->b[layer]
-                   : which == 2 ? m->gw[layer] : m->gb[layer];
-  const size_t n = (which == 0 || which == 2) ? nw : (size_t)m->out[layer];
+  const MlpLayer &y = m->layer[layer];
+  const size_t nw = (size_t)y.out * y.in;
+  const float *src = which == 0 ? y.w : which == 1 ? y.b : which == 2 ? y.gw : y.gb;
+  const size_t n = (which == 0 || which == 2) ? nw : (size_t)y.out;
   MISOHIP_TRY(hipMemcpy(host, src, sizeof(float) * n, hipMemcpyDeviceToHost));
   return MISOHIP_OK;
 }
@@ -248,7 +188,7 @@ int misohip_mlp_forward(misohip_ctx *ctx, misohip_mlp *m, const void *X, int bat
   if (int rc = check_batch(m, batch)) return rc;
   MISOHIP_TRY(hipSetDevice(ctx->device));
   Timed t_(ctx, MISOHIP_KIND_MLP);
-  return forward(ctx, m, static_cast<const uint16_t *>(X), batch, Y);
+  return forward(ctx, m, static_cast<const uint16_t *>(X), batch, Y, MlpField{});
 }
 
 // loss and gradients (MSE on the batch); *loss receives the mean squared error
@@ -260,18 +200,18 @@ int misohip_mlp_grad(misohip_ctx *ctx, misohip_mlp *m, const void *X, const floa
   MISOHIP_TRY(hipSetDevice(ctx->device));
   {
     Timed t_(ctx, MISOHIP_KIND_MLP);
-    const uint16_t *Xb = static_cast<const uint16_t *>(X);
-    if (int rc = forward(ctx, m, Xb, batch, nullptr)) return rc;
     const long n = (long)batch * m->n_out;
+    MlpLoss ls;
+    ls.T = T;
+    ls.scale = 1.f / (float)n;
+    MISOHIP_TRY(launch_mlp_grad(ctx->stream, m->d_layer, m->n_layers, m->n_in, m->wide, m->maxw,
+                                m->tiles, m->bias_tiles, static_cast<const uint16_t *>(X), batch,
+                                ls, loss ? m->y : nullptr, m->g0, m->g1));
     int nb = 0;
-    MISOHIP_TRY(launch_mse(ctx->stream, m->pre[m->n_layers - 1], T, m->dpre, m->loss_part, n,
-                           1.f / (float)n, &nb));
-    if (int rc = backward(ctx, m, Xb, batch)) return rc;
+    if (loss) MISOHIP_TRY(launch_mlp_loss(ctx->stream, m->y, T, m->loss_part, n, &nb));
     if (loss) {
       MISOHIP_TRY(hipMemcpyAsync(m->h_loss, m->loss_part, sizeof(float) * nb,
                                  hipMemcpyDeviceToHost, ctx->stream));
-    }
-    if (loss) {
       MISOHIP_TRY(hipStreamSynchronize(ctx->stream));
       double s = 0.0;
       for (int i = 0; i < nb; ++i) s += m->h_loss[i];
@@ -289,13 +229,8 @@ int misohip_mlp_adam(misohip_ctx *ctx, misohip_mlp *m, float lr, float beta1, fl
   Timed t_(ctx, MISOHIP_KIND_MLP);
   m->t += 1;
   const float c1 = 1.f - std::pow(beta1, (float)m->t), c2 = 1.f - std::pow(beta2, (float)m->t);
-  for (int l = 0; l < m->n_layers; ++l) {
-    const long nw = (long)m->out[l] * m->in[l];
-    MISOHIP_TRY(launch_adam(ctx->stream, m->w[l], m->wb[l], m->gw[l], m->mw[l], m->vw[l], nw, lr,
-                            beta1, beta2, eps, c1, c2, weight_decay));
-    MISOHIP_TRY(launch_adam(ctx->stream, m->b[l], nullptr, m->gb[l], m->mb[l], m->vb[l],
-                            m->out[l], lr, beta1, beta2, eps, c1, c2, 0.f));
-  }
+  const MlpAdam p = {lr, beta1, beta2, eps, c1, c2, weight_decay};
+  MISOHIP_TRY(launch_mlp_adam(ctx->stream, m->d_layer, m->n_layers, m->tiles, p));
   return MISOHIP_OK;
 }
 
@@ -327,15 +262,23 @@ int misohip_mlp_qrad(misohip_ctx *ctx, misohip_mlp *m, const misohip_grid *g, co
   if (flags && !q_rt) return MISOHIP_E_ARG;
   MISOHIP_TRY(hipSetDevice(ctx->device));
   Timed t_(ctx, MISOHIP_KIND_MLP);
-  for (int c0 = 0; c0 < ncol; c0 += m->max_batch) {
-    const int nb = ncol - c0 < m->max_batch ? ncol - c0 : m->max_batch;
+  MlpField f;
+  f.mu = m->mu_out;
+  f.sd = m->sd_out;
+  f.flag = flags;
+  f.q_rt = static_cast<const double *>(q_rt);
+  f.corr = static_cast<const double *>(corr);
+  f.qrad = static_cast<double *>(qrad);
+  f.sh = shape_of(g);
+  // activations in LDS: any number of columns; else as many as g0, g1 hold
+  const int step = m->wide ? m->max_batch : ncol;
+  for (int c0 = 0; c0 < ncol; c0 += step) {
+    const int nb = ncol - c0 < step ? ncol - c0 : step;
+    f.col0 = c0;
     if (int rc = forward(ctx, m, static_cast<const uint16_t *>(X) + (long)c0 * m->n_in, nb,
-                         Y + (long)c0 * m->n_out, false))
+                         Y + (long)c0 * m->n_out, f))
       return rc;
   }
-  MISOHIP_TRY(launch_column_output(ctx->stream, Y, shape_of(g), m->mu_out, m->sd_out, flags,
-                                   static_cast<const double *>(q_rt),
-                                   static_cast<const double *>(corr), static_cast<double *>(qrad)));
   return MISOHIP_OK;
 }
 
