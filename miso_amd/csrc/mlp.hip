@@ -14,6 +14,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "mlp.hpp"
@@ -39,6 +40,9 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// features of X that a workgroup of 64 columns takes at a time
+constexpr int MLP_X_TALL = 128;
+
 // The network from its input columns to its output (TRAIN: and back from the
 // gradient of the mean squared error to every layer's pre-activation gradient;
 // Y, where given, receives the output) in one launch: a workgroup
@@ -58,20 +62,24 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
 // reads again.
 // Bound by the weights' way from L2 into the CU (64 bytes a clock): 1.24 MB
 // forward and 0.46 back for 1536-256-256-256-384.
-// NT = 1 (16 waves) spreads a batch of 1024 over 64 CUs; NT = 4 (four waves,
+// NT = 1 (16 waves) spreads a batch of 1024 over 64 CUs; NT = 4 (eight waves,
 // two workgroups a CU) reads the weights a quarter as often, for large
-// batches of inference.
+// batches of inference (NT = 2: 736 us for 635 at 147456 columns; four waves
+// of twice the row tiles 680; three row tiles a wave spill: 994; features of
+// X by 256, one workgroup a CU: 850).
 // At that size and a batch of 1024 a training step's chain takes 37 us, where
 // a launch per layer, product and elementwise step (128 x 128 tiles: 16
 // workgroups) took 232; 147456 columns of inference, their Q_rad field
-// included, 721 us for 957.  Every sum is taken in the order of k, 32 at a
-// time, as those took it: the same bits.
+// included, 635 us for 957 (without
+// its 1.1 GB of Y, corrections and Q_rad it would take 363).  Every sum is
+// taken in the order of k, 32 at a time, as those took it: the same bits.
 template <int NT, int WAVES, int RT, int PD, bool TRAIN, bool WIDE>
-__global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 4) void mlp_chain_kernel(
+__global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
     const MlpLayer *__restrict__ L, int nl, const uint16_t *__restrict__ X, int M,
     float *__restrict__ Y, MlpLoss ls, MlpField fo, uint16_t *g0, uint16_t *g1, int bw, int xoff,
     int xw) {
   constexpr int NS = 16 * NT, NTHR = 64 * WAVES;
+  static_assert(RT <= 3, "product()");
   static_assert(NT == 1 || !TRAIN, "the packed columns of a training tile are 16");
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -141,6 +149,26 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 4) void mlp_chain_kern
     __syncthreads();
     return cw;
   };
+  // NT > 1: the thread's part of XW features of the workgroup's columns, in
+  // flight while the chunk before is multiplied
+  constexpr int XW = MLP_X_TALL, XE = NT > 1 ? NS * XW / 8 / NTHR : 1;
+  uint4 xr[XE];
+  auto fetch = [&](int f0) {
+#pragma unroll
+    for (int e = 0; e < XE; ++e) {
+      const int q = tid + e * NTHR, r = q / (XW / 8), f = f0 + 8 * (q % (XW / 8));
+      xr[e] = make_uint4(0, 0, 0, 0);
+      if (s0 + r < M && f < n_in)
+        xr[e] = *reinterpret_cast<const uint4 *>(X + (long)(s0 + r) * n_in + f);
+    }
+  };
+  auto put = [&](uint16_t *xb) {
+#pragma unroll
+    for (int e = 0; e < XE; ++e) {
+      const int q = tid + e * NTHR;
+      *reinterpret_cast<uint4 *>(xb + q / (XW / 8) * xpitch + 8 * (q % (XW / 8))) = xr[e];
+    }
+  };
   // acc = W b over all k for `cnt` row tiles; input: b is X, chunk by chunk
   auto gemm = [&](auto cnt_, const uint16_t *wp, int KT, int OT, int base, const uint16_t *b,
                   bool input, bool keep) {
@@ -152,14 +180,8 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 4) void mlp_chain_kern
     for (int r = 0; r < cnt; ++r)
 #pragma unroll
       for (int n = 0; n < NT; ++n) acc[r][n] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    const uint16_t *row = input ? xbuf + col * xpitch + kq * 8 : b + col * pitch + kq * 8;
-    const int rp = input ? 16 * xpitch : 16 * pitch, chunk = input ? xw >> 5 : KT;
-    for (int k0 = 0; k0 < KT; k0 += chunk) {
-      if (input) {
-        const int cw = stage(k0 * 32);
-        if (TRAIN && keep) pack(xbuf, xpitch, cw, L[0].aT, k0 * 32);
-      }
-      const int ke = min(chunk, KT - k0);
+    // k-steps k0 .. k0 + ke - 1, their B operand from `row` on
+    auto steps = [&](const uint16_t *row, int rp, int k0, int ke) {
       for (int k = 0; k < ke; k += PD) {
 #pragma unroll
         for (int p = 0; p < PD; ++p) {
@@ -176,18 +198,82 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 4) void mlp_chain_kern
           }
         }
       }
+    };
+    if (!input) {
+      steps(b + col * pitch + kq * 8, 16 * pitch, 0, KT);
+    } else if constexpr (NT > 1) {
+      fetch(0);
+      if (base) __syncthreads();
+      put(xbuf);
+      for (int k0 = 0, h = 0; k0 < KT; k0 += XW / 32, h ^= 1) {
+        __syncthreads();
+        if (k0 + XW / 32 < KT) fetch(k0 * 32 + XW);
+        steps(xbuf + (h * NS + col) * xpitch + kq * 8, 16 * xpitch, k0, min(XW / 32, KT - k0));
+        if (k0 + XW / 32 < KT) put(xbuf + (h ^ 1) * NS * xpitch);
+      }
+    } else {
+      for (int k0 = 0; k0 < KT; k0 += xw >> 5) {
+        const int cw = stage(k0 * 32);
+        if (TRAIN && keep) pack(xbuf, xpitch, cw, L[0].aT, k0 * 32);
+        steps(xbuf + col * xpitch + kq * 8, 16 * xpitch, k0, cw >> 5);
+      }
     }
   };
   auto product = [&](int cnt, const uint16_t *wp, int KT, int OT, int base, const uint16_t *b,
                      bool input, bool keep) {
-    if constexpr (RT == 1) {
+    if (RT > 2 && cnt == 3)
+      gemm(std::integral_constant<int, (RT > 2 ? 3 : 1)>{}, wp, KT, OT, base, b, input, keep);
+    else if (RT > 1 && cnt == 2)
+      gemm(std::integral_constant<int, (RT > 1 ? 2 : 1)>{}, wp, KT, OT, base, b, input, keep);
+    else
       gemm(std::integral_constant<int, 1>{}, wp, KT, OT, base, b, input, keep);
-    } else {
-      static_assert(RT == 4, "");
-      if (cnt == 4) gemm(std::integral_constant<int, 4>{}, wp, KT, OT, base, b, input, keep);
-      else if (cnt == 3) gemm(std::integral_constant<int, 3>{}, wp, KT, OT, base, b, input, keep);
-      else if (cnt == 2) gemm(std::integral_constant<int, 2>{}, wp, KT, OT, base, b, input, keep);
-      else gemm(std::integral_constant<int, 1>{}, wp, KT, OT, base, b, input, keep);
+  };
+
+  // the output of row tile r, from output o on: Y, and the Q_rad field, 32
+  // columns at a time; loads go before the stores, which the compiler takes
+  // for possible aliases
+  auto store_output = [&](int r, int o, f32x4 bias) {
+    constexpr int H = NT < 2 ? NT : 2;
+    const int no = L[nl - 1].out, st = fo.sh.It * fo.sh.Jt;
+    f32x4 mu, sd;
+    if (fo.qrad) {
+      mu = *reinterpret_cast<const f32x4 *>(fo.mu + o);
+      sd = *reinterpret_cast<const f32x4 *>(fo.sd + o);
+    }
+#pragma unroll
+    for (int n0 = 0; n0 < NT; n0 += H) {
+      double other[H][4];
+      int c0[H], fall[H];
+      if (fo.qrad) {
+#pragma unroll
+        for (int n = 0; n < H; ++n) {
+          const int cs = fo.col0 + min(s0 + 16 * (n0 + n) + col, M - 1);
+          const int ni = fo.sh.It - 2 * fo.sh.mi, j = cs / ni, i = cs - j * ni;
+          c0[n] = fo.sh.idx(fo.sh.mi + i, fo.sh.mj + j, fo.sh.mk + o);
+          fall[n] = fo.flag ? fo.flag[cs] : 0;
+        }
+#pragma unroll
+        for (int n = 0; n < H; ++n) {
+          const double *q = fall[n] ? fo.q_rt : fo.corr;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) other[n][v] = q ? q[c0[n] + v * st] : 0.0;
+        }
+      }
+#pragma unroll
+      for (int n = 0; n < H; ++n) {
+        const int s = s0 + 16 * (n0 + n) + col;
+        if (s >= M) continue;
+        const f32x4 x = acc[r][n0 + n] + bias;
+        *reinterpret_cast<f32x4u *>(Y + (long)s * no + o) = x;
+        if (fo.qrad) {
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const double net = (double)(x[v] * sd[v] + mu[v]);
+            fo.qrad[c0[n] + v * st] =
+                fall[n] ? other[n][v] : fo.corr ? net + other[n][v] : net;
+          }
+        }
+      }
     }
   };
 
@@ -210,6 +296,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 4) void mlp_chain_kern
         for (int n = 0; n < NT; ++n) {
           const int sl = 16 * n + col, s = s0 + sl;
           f32x4 x = acc[r][n] + bias;
+          if (!TRAIN && last) break;
           if (!last) {
             if (TRAIN)
               *reinterpret_cast<f32x4 *>(L[l].pre + ((long)blockIdx.x * OT + tile) * 256 +
@@ -228,32 +315,9 @@ __global__ __launch_bounds__(64 * WAVES, WAVES == 4 ? 2 : 4) void mlp_chain_kern
             }
             *reinterpret_cast<uint2 *>(nxt + sl * pitch + o) = f2bf4(g);
             if (Y) *reinterpret_cast<f32x4u *>(Y + (long)s * L[l].out + o) = x;
-          } else if (s < M) {
-            *reinterpret_cast<f32x4u *>(Y + (long)s * L[l].out + o) = x;
-            if (fo.qrad) {
-              const Shape &sh = fo.sh;
-              const int ni = sh.It - 2 * sh.mi, cs = fo.col0 + s;
-              const int j = cs / ni, i = cs - j * ni;
-              const int c0 = sh.idx(sh.mi + i, sh.mj + j, sh.mk + o), st = sh.It * sh.Jt;
-              if (fo.flag && fo.flag[cs]) {  // fallback column: last plain-RT value
-#pragma unroll
-                for (int v = 0; v < 4; ++v) fo.qrad[c0 + v * st] = fo.q_rt[c0 + v * st];
-              } else {
-                const f32x4 mu = *reinterpret_cast<const f32x4 *>(fo.mu + o);
-                const f32x4 sd = *reinterpret_cast<const f32x4 *>(fo.sd + o);
-                double q[4];
-#pragma unroll
-                for (int v = 0; v < 4; ++v) q[v] = (double)(x[v] * sd[v] + mu[v]);
-                if (fo.corr) {
-#pragma unroll
-                  for (int v = 0; v < 4; ++v) q[v] += fo.corr[c0 + v * st];
-                }
-#pragma unroll
-                for (int v = 0; v < 4; ++v) fo.qrad[c0 + v * st] = q[v];
-              }
-            }
           }
         }
+        if (!TRAIN && last) store_output(r, o, bias);
       }
     }
     if (!last)
@@ -480,60 +544,93 @@ __global__ __launch_bounds__(256) void mlp_adam_kernel(const MlpLayer *__restric
 
 // Column features of the radiative box: for column (i, j) and cell kz of the
 // interior, x[col][f*nz + kz] = (feat_f - mu[f*nz+kz]) / sd[f*nz+kz] with
-// feat = (ln ro, ln T, |B|^2), T = (gm-1) ei.  Columns run i fastest.
-// Column features, tiled through LDS: a block reads 64 consecutive x cells
-// (one y row) x 32 heights with lanes along x (coalesced field reads),
-// then writes each column's 32 consecutive heights (coalesced row writes of
-// X).  nfeat == 4 adds the horizontal Laplacian of ln T at stride h (x and y
-// periodic: neighbours wrap inside the interior).
-constexpr int FT_X = 64, FT_Z = 32;
+// feat = (ln ro, ln T, |B|^2), T = (gm-1) ei, and with nfeat == 4 the
+// horizontal Laplacian of ln T at stride FT_H (x and y periodic: neighbours
+// wrap inside the interior).  Columns run i fastest.
+// A block reads 64 consecutive x cells (one y row) x 32 heights with lanes
+// along x, and ln T of the FT_H cells beside them, so that the x neighbours'
+// logarithms are taken once, from LDS; then it writes each column's 32
+// heights, four per lane.  Each XCD takes a contiguous range of blocks, x
+// fastest, then y: the rows FT_H above and below are in its L2 (2.6 GB read
+// at 384^3, of 2.3 without any row twice).
+// Bound by HBM: 3.1 GB at 4.2 TB/s, 722 us at 384^3; with every neighbour's
+// logarithm taken anew and the rows spread over the XCDs 943.
+constexpr int FT_X = 64, FT_Z = 32, FT_H = 4;
+typedef uint16_t u16x4u __attribute__((ext_vector_type(4), aligned(2)));
 
 __global__ __launch_bounds__(256) void column_features_kernel(
     Fld<const double> q, Shape sh, double gm, const float *__restrict__ mu,
     const float *__restrict__ sd, uint16_t *__restrict__ X, float *__restrict__ Xf, int nfeat,
-    int h) {
-  __shared__ float tile[4][FT_Z][FT_X + 1];
+    int nbx, int nb) {
+  __shared__ float tile[3][FT_Z][FT_X + 1];         // ln ro, |B|^2, Laplacian
+  __shared__ float lnt[FT_Z][FT_X + 2 * FT_H + 1];  // ln T from x = i0 - FT_H on
   const int ni = sh.It - 2 * sh.mi, nj = sh.Jt - 2 * sh.mj, nz = sh.Kt - 2 * sh.mk;
-  const int i0 = blockIdx.x * FT_X, j = blockIdx.y, kz0 = blockIdx.z * FT_Z;
+  const int V = xcd_virtual_block(blockIdx.x, nb), rest = V / nbx;
+  const int i0 = (V - rest * nbx) * FT_X, j = rest % nj, kz0 = rest / nj * FT_Z;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int i = i0 + lane;
-  for (int r = wv; r < FT_Z; r += 4) {
-    const int kz = kz0 + r;
-    if (i >= ni || kz >= nz) continue;
-    const int k = sh.mk + kz;
-    const int c = sh.idx(sh.mi + i, sh.mj + j, k);
-    // the features end in FP32 (then BF16): logarithms in FP32 of the FP64
-    // arguments, sums in FP64
-    const double ro = q.q[0][c], ei = q.q[7][c];
+  // the features end in FP32 (then BF16): logarithms in FP32 of the FP64
+  // arguments, sums in FP64
+  auto ln_t = [&](int c) { return logf((float)((gm - 1.0) * q.q[7][c])); };
+  if (nfeat == 4) {
+    static_assert(FT_Z * 2 * FT_H == 256, "a thread per cell beside the tile");
+    const int r = threadIdx.x / (2 * FT_H), h = threadIdx.x % (2 * FT_H);
+    const int p = h < FT_H ? h - FT_H : FT_X + h - FT_H;  // from i0
+    const int i = ((i0 + p) % ni + ni) % ni;
+    if (kz0 + r < nz) lnt[r][p + FT_H] = ln_t(sh.idx(sh.mi + i, sh.mj + j, sh.mk + kz0 + r));
+  }
+  const int i = (i0 + lane) % ni;  // lanes past the row's end: neighbours of its last cells
+  const int up = ((j + FT_H) % nj - j) * sh.It, dn = ((j - FT_H % nj + nj) % nj - j) * sh.It;
+  float y[FT_Z / 4][2];
+#pragma unroll
+  for (int m = 0; m < FT_Z / 4; ++m) {
+    const int r = wv + 4 * m;
+    if (kz0 + r >= nz) break;
+    const int c = sh.idx(sh.mi + i, sh.mj + j, sh.mk + kz0 + r);
     const double bx = q.q[4][c], by = q.q[5][c], bz = q.q[6][c];
-    const double lnT = (double)logf((float)((gm - 1.0) * ei));
-    tile[0][r][lane] = logf((float)ro);
-    tile[1][r][lane] = (float)lnT;
-    tile[2][r][lane] = (float)(bx * bx + by * by + bz * bz);
+    tile[0][r][lane] = logf((float)q.q[0][c]);
+    lnt[r][lane + FT_H] = ln_t(c);
+    tile[1][r][lane] = (float)(bx * bx + by * by + bz * bz);
     if (nfeat == 4) {
-      const int ip = (i + h) % ni, im = (i - h % ni + ni) % ni;
-      const int jp = (j + h) % nj, jm = (j - h % nj + nj) % nj;
-      const double s =
-          (double)logf((float)((gm - 1.0) * q.q[7][sh.idx(sh.mi + ip, sh.mj + j, k)])) +
-          (double)logf((float)((gm - 1.0) * q.q[7][sh.idx(sh.mi + im, sh.mj + j, k)])) +
-          (double)logf((float)((gm - 1.0) * q.q[7][sh.idx(sh.mi + i, sh.mj + jp, k)])) +
-          (double)logf((float)((gm - 1.0) * q.q[7][sh.idx(sh.mi + i, sh.mj + jm, k)]));
-      tile[3][r][lane] = (float)(s - 4.0 * lnT);
+      y[m][0] = ln_t(c + up);
+      y[m][1] = ln_t(c + dn);
     }
   }
   __syncthreads();
-  // write: 32 lanes along the heights of one (column, feature) pair
-  const int zl = threadIdx.x & (FT_Z - 1), pr = threadIdx.x / FT_Z;  // 8 pairs per pass
-  const int kz = kz0 + zl;
-  if (kz >= nz) return;
-  for (int p = pr; p < nfeat * FT_X; p += 256 / FT_Z) {
-    const int f = p / FT_X, il = p % FT_X;
-    if (i0 + il >= ni) continue;
-    const long col = (long)j * ni + i0 + il;
-    const int fi = f * nz + kz;
-    const float x = (tile[f][zl][il] - mu[fi]) / sd[fi];
-    X[col * nfeat * nz + fi] = f2bf(x);
-    if (Xf) Xf[col * nfeat * nz + fi] = x;
+  if (nfeat == 4) {
+#pragma unroll
+    for (int m = 0; m < FT_Z / 4; ++m) {
+      const int r = wv + 4 * m;
+      if (kz0 + r >= nz) break;
+      const double s = (double)lnt[r][lane + 2 * FT_H] + (double)lnt[r][lane] + (double)y[m][0] +
+                       (double)y[m][1];
+      tile[2][r][lane] = (float)(s - 4.0 * (double)lnt[r][lane + FT_H]);
+    }
+    __syncthreads();
+  }
+  // write: 8 lanes along the heights of one (column, feature) pair
+  const int zl = 4 * (threadIdx.x & 7), kz = kz0 + zl;
+  if (kz >= nz) return;  // nz is a multiple of 8
+  for (int f = 0; f < nfeat; ++f) {
+    float m4[4], s4[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      m4[v] = mu[f * nz + kz + v];
+      s4[v] = sd[f * nz + kz + v];
+    }
+#pragma unroll
+    for (int il = threadIdx.x >> 3; il < FT_X; il += 32) {
+      if (i0 + il >= ni) break;
+      f32x4 x;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float t = f == 1 ? lnt[zl + v][il + FT_H] : tile[f ? f - 1 : 0][zl + v][il];
+        x[v] = (t - m4[v]) / s4[v];
+      }
+      const long at = ((long)j * ni + i0 + il) * nfeat * nz + f * nz + kz;
+      const u16x4u h = {f2bf(x[0]), f2bf(x[1]), f2bf(x[2]), f2bf(x[3])};
+      *reinterpret_cast<u16x4u *>(X + at) = h;
+      if (Xf) *reinterpret_cast<f32x4u *>(Xf + at) = x;
+    }
   }
 }
 
@@ -598,13 +695,14 @@ hipError_t launch_mlp_forward(hipStream_t st, const MlpLayer *L, int nl, int n_i
                               bool wide, int maxw, const uint16_t *X, int M, float *Y,
                               const MlpField &fo, uint16_t *g0, uint16_t *g1) {
   const MlpLoss none{};
-  // X passes through the second buffer (the input layer writes the first),
-  // in chunks of whole rounds of the two k-steps in flight
-  const int xt = (n_hidden + 63) / 64 * 64;
-  const size_t tall = sizeof(uint16_t) * 64 * (n_hidden + 8 + xt + 8);
+  // X passes through the place of the second buffer, two chunks of it (the
+  // input layer writes the first buffer)
+  constexpr int NT = 4, NS = 16 * NT;
+  const size_t tall = sizeof(uint16_t) * NS *
+                      (n_hidden + 8 + std::max(n_hidden + 8, 2 * (MLP_X_TALL + 8)));
   if (M >= MLP_TALL && tall <= (size_t)LDS_BYTES)
-    return chain<4, 4, 4, 2, false, false>(st, L, nl, X, M, Y, none, fo, g0, g1, n_hidden,
-                                           64 * (n_hidden + 8), xt, tall);
+    return chain<NT, 8, 2, 2, false, false>(st, L, nl, X, M, Y, none, fo, g0, g1, n_hidden,
+                                            NS * (n_hidden + 8), MLP_X_TALL, tall);
   const int xw = x_width(n_in);
   if (wide)
     return chain<1, 16, 1, 8, false, true>(st, L, nl, X, M, Y, none, fo, g0, g1, maxw, 0, xw,
@@ -652,12 +750,14 @@ hipError_t launch_mlp_pack(hipStream_t st, const MlpLayer *L, int nl, int layer,
 
 hipError_t launch_column_features(hipStream_t st, const Fld<const double> &q, const Shape &sh,
                                   double gm, const float *mu, const float *sd, uint16_t *X,
-                                  float *Xf, int nfeat, int h) {
+                                  float *Xf, int nfeat) {
   const int ni = sh.It - 2 * sh.mi, nj = sh.Jt - 2 * sh.mj, nz = sh.Kt - 2 * sh.mk;
-  if (nfeat < 3 || nfeat > 4) return hipErrorInvalidValue;
-  dim3 grid((ni + FT_X - 1) / FT_X, nj, (nz + FT_Z - 1) / FT_Z);
-  hipLaunchKernelGGL(column_features_kernel, grid, dim3(256), 0, st, q, sh, gm, mu, sd, X, Xf,
-                     nfeat, h);
+  if (nfeat < 3 || nfeat > 4 || nz % 4) return hipErrorInvalidValue;
+  const int nbx = (ni + FT_X - 1) / FT_X;
+  const long nb = (long)nbx * nj * ((nz + FT_Z - 1) / FT_Z);
+  if (nb > 2147483647L) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(column_features_kernel, dim3((unsigned)nb), dim3(256), 0, st, q, sh, gm, mu,
+                     sd, X, Xf, nfeat, nbx, (int)nb);
   return hipGetLastError();
 }
 

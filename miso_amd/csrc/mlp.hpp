@@ -53,7 +53,7 @@ hipError_t launch_mlp_adam(hipStream_t, const MlpLayer *, int nl, int tiles, con
 // the packed copies of one layer's weights
 hipError_t launch_mlp_pack(hipStream_t, const MlpLayer *, int nl, int layer, int tiles);
 hipError_t launch_column_features(hipStream_t, const Fld<const double> &, const Shape &, double,
-                                  const float *, const float *, uint16_t *, float *, int, int);
+                                  const float *, const float *, uint16_t *, float *, int);
 hipError_t launch_column_residual(hipStream_t, const float *, const Shape &, const float *,
                                   const float *, const double *, int *, float, double *);
 

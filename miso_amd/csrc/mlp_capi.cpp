@@ -246,7 +246,7 @@ int misohip_mlp_features(misohip_ctx *ctx, misohip_mlp *m, const misohip_grid *g
   for (int f = 0; f < 9; ++f) q.q[f] = static_cast<const double *>(qq->q[f]);
   Timed t_(ctx, MISOHIP_KIND_MLP);
   MISOHIP_TRY(launch_column_features(ctx->stream, q, shape_of(g), gm, m->mu_in, m->sd_in,
-                                     static_cast<uint16_t *>(X), Xf, nfeat, 4));
+                                     static_cast<uint16_t *>(X), Xf, nfeat));
   return MISOHIP_OK;
 }
 
