@@ -477,7 +477,7 @@ __device__ __forceinline__ void av_walk_block(const Fld<const R> &qq, const Fld<
   }
   if (CFLF) {
     best = wave_umin(best);
-    if ((threadIdx.x & 63) == 0) atomicMin(cf->slot, best);
+    if ((threadIdx.x & 63) == 0) slot_min(cf->slot, best);
   }
 }
 
@@ -839,6 +839,19 @@ __global__ __launch_bounds__(256) __attribute__((
   }
 }
 
+// Blocks that run at a time, and the rows a chunk costs more than it covers
+// (split_rounds): the y and z walks hold one FP64 wave per SIMD (256 registers
+// and a few more) or three FP32 ones; the x-y walk holds more, but is bound by
+// VALU issue, so that what counts is how evenly its blocks fall on the CUs.
+// Walks halved until the launch had 2^18 threads, as before, at 64^3 and 205 x
+// 131 x 93 in FP64: x-y 61 -> 49 and 229 -> 198 us, z with its CFL 27 -> 21
+// and 163 -> 122 (512 blocks: 24 and 132), y of 256^2 16 -> 8; FP32 of 181 x
+// 97 x 260: z 102 -> 92 (512 blocks: 102).
+template <typename R> constexpr int WALK_SLOTS = sizeof(R) == 8 ? 256 : 768;
+constexpr double WALK_START = 4.0;
+constexpr int XY_SLOTS = 256;
+constexpr double XY_START = 5.0;
+
 template <typename R, int DIR>
 static hipError_t launch_av_t(hipStream_t st, const Fld<const R> &q, const Fld<R> &r, R *cc_store,
                               const R *cc_in, const R *dd, const Shape &sh, const AvScalars &sc) {
@@ -868,7 +881,8 @@ static hipError_t launch_walk_t(hipStream_t st, const Fld<const R> &q, const Fld
   const int nbx = ((sh.It - 2 * sh.mi + 63) / 64 + wx - 1) / wx;
   const int nbo = (n_oth + 4 / wx - 1) / (4 / wx);
   int chunk, nchunks;  // even walk lengths
-  walk_split(n_dir, 256L * nbx * nbo, sc.chunk, chunk, nchunks);
+  split_rounds(n_dir, (long)nbx * nbo, sc.chunk, WALK_SLOTS<R>, WALK_START, 2.0, chunk,
+               nchunks);
   if (sc.nparts && (sc.part0 < 0 || sc.nparts < 0 || sc.part0 + sc.nparts > nchunks))
     return hipErrorInvalidValue;
   const long nbl = (long)(sc.nparts ? sc.nparts : nchunks) * nbx * nbo;
@@ -932,7 +946,8 @@ static hipError_t launch_walk_cfl_t(hipStream_t st, const Fld<const R> &q, const
   const int nbx = ((sh.It - 2 * sh.mi + 63) / 64 + wx - 1) / wx;
   const int nbo = (n_oth + 4 / wx - 1) / (4 / wx);
   int chunk, nchunks;  // even walk lengths
-  walk_split(n_dir, 256L * nbx * nbo, sc.chunk, chunk, nchunks);
+  split_rounds(n_dir, (long)nbx * nbo, sc.chunk, WALK_SLOTS<R>, WALK_START, 2.0, chunk,
+               nchunks);
   if (sc.nparts && (sc.part0 < 0 || sc.nparts < 0 || sc.part0 + sc.nparts > nchunks))
     return hipErrorInvalidValue;
   const long nbl = (long)(sc.nparts ? sc.nparts : nchunks) * nbx * nbo;
@@ -964,7 +979,8 @@ hipError_t launch_av_sweep_xy(hipStream_t st, const Fld<const R> &q, const Fld<R
   if (!sh.is || !sh.js || !sh.ks || nj < 2 || sh.mj < 2) return hipErrorInvalidValue;
   const int nseg = (sh.It - 2 * sh.mi + 59) / 60;
   int chunk, nchunks;  // even walk lengths
-  walk_split(nj, 64L * nseg * (sh.Kt - 2 * sh.mk + 2), sc.chunk, chunk, nchunks);
+  split_rounds(nj, (nseg * (sh.Kt - 2L * sh.mk + 2) + 3) / 4, sc.chunk, XY_SLOTS, XY_START, 4.0, chunk,
+               nchunks);
   const int npl = sh.Kt - 2 * sh.mk + 2;  // interior planes and the two z ring planes
   if (sc.nparts && (sc.nparts < 0 || sc.nparts > npl || sc.part0 < sh.mk - 1 ||
                     sc.part0 > sh.Kt - sh.mk))
@@ -1061,14 +1077,18 @@ hipError_t launch_batch_av(hipStream_t st, int dir, int mode, const BatchInst<R>
   return hipErrorInvalidValue;
 }
 
+template <typename R>
 void av_walk_split(const Shape &sh, int dir, int chunk_req, int *chunk, int *nchunks) {
   const int n_dir = dir == 1 ? sh.Jt - 2 * sh.mj : sh.Kt - 2 * sh.mk;
   const int n_oth = dir == 1 ? sh.Kt - 2 * sh.mk : sh.Jt - 2 * sh.mj;
   const int wx = walk_waves_x(n_oth);
   const int nbx = ((sh.It - 2 * sh.mi + 63) / 64 + wx - 1) / wx;
   const int nbo = (n_oth + 4 / wx - 1) / (4 / wx);
-  walk_split(n_dir, 256L * nbx * nbo, chunk_req, *chunk, *nchunks);
+  split_rounds(n_dir, (long)nbx * nbo, chunk_req, WALK_SLOTS<R>, WALK_START, 2.0, *chunk,
+               *nchunks);
 }
+template void av_walk_split<double>(const Shape &, int, int, int *, int *);
+template void av_walk_split<float>(const Shape &, int, int, int *, int *);
 
 template hipError_t launch_batch_av<double>(hipStream_t, int, int, const BatchInst<double> *,
                                             const BatchDyn<double> *, const int *, int, int, int,

@@ -228,7 +228,7 @@ int tail_overlap_t(misohip_ctx *ctx, const misohip_grid *g, const misohip_params
   MISOHIP_TRY(hipStreamIsCapturing(ctx->stream, &cs));
   if (cs != hipStreamCaptureStatusNone) return TAIL_NOT_TAKEN;
   int zch, znch;
-  av_walk_split(sh, 2, ctx->tile.sweep_chunk, &zch, &znch);
+  av_walk_split<R>(sh, 2, ctx->tile.sweep_chunk, &zch, &znch);
   const bool pz = wrap & 4;
   TailPlan P;
   if ((!pz && b.periodic[2] != 2) || !tail_plan(sh.Kt, sh.mk, zch, znch, pz, &P))

@@ -9,6 +9,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <cmath>
+
 namespace misohip {
 
 template <typename R> struct Const {
@@ -149,22 +151,49 @@ __device__ __forceinline__ int wrap_coord(int x, int total, int m, bool on) {
   return x < m ? x + n : (x >= total - m ? x - n : x);
 }
 
-// Blocks of the z-march kernel: (nbx, nby) columns of 64 x 4 cells, each cut
-// into nzc chunks of kz planes; x fastest, then y, then the chunk, so that
-// with xcd_virtual_block every XCD walks compact x-y regions of one slab.
-// The requested chunk is halved (not below 4 planes) while there would be
-// fewer blocks than the 256 CUs (a small grid in long chunks would leave
-// most of the chip idle); every chunk loads its own first planes, so the
-// results do not depend on the split.
+// Chunks of a march or walk over n cells, none longer than `most`, in a
+// launch of per_chunk blocks each: of all counts the one with the least
+// rounds x length, where `slots` blocks run at a time and each costs `start`
+// cells more than it covers (its first window is loaded, and its first slopes
+// formed, anew).  The last round of a launch is then nearly full, and a small
+// grid is spread over the chip as far as the repeated cells allow.  Past
+// `even` rounds the blocks no longer end together: half a round is lost at the
+// end, and nothing is gained by more chunks (the FP32 z walk of 512^3, 2.7
+// rounds of 256 planes: 3.1 ms; 4 of 171: 3.3).  Every chunk starts from the
+// fields, so the results do not depend on the split.
+inline void split_rounds(int n, long per_chunk, int most, long slots, double start, double even,
+                         int &chunk, int &nchunks) {
+  const int least = most < 1 ? 1 : most;
+  double best = 0.0, rounds = 0.0;
+  nchunks = 0;
+  for (int m = (n + least - 1) / least; m <= n && rounds <= even; ++m) {
+    const int c = (n + m - 1) / m;
+    if ((n + c - 1) / c != m) continue;  // the same length as fewer chunks'
+    const double full = (double)per_chunk * m / slots;
+    const double cost = (full <= even ? std::ceil(full) : full + 0.5) * (c + start);
+    if (nchunks && cost > 0.98 * best) continue;
+    best = cost;
+    rounds = full;
+    chunk = c;
+    nchunks = m;
+  }
+}
+
+// Blocks of the z-march kernel: (nbx, nby) columns of 64 x TY cells, each cut
+// into nzc chunks of at most kz_ planes; x fastest, then y, then the chunk, so
+// that with xcd_virtual_block every XCD walks compact x-y regions of one slab.
+// A CU holds one block of the 8- and 12-row columns (LDS), two of the 4-row
+// ones.  Chunks halved until there were 256 blocks left a nearly empty last
+// round: FP64 stages of 300 x 222 x 150 920 -> 648 us, of 205 x 131 x 93 232 ->
+// 211, of 64^3 (now down to two planes) 31 -> 22, FP32 of 181 x 97 x 260 250 ->
+// 194; 512^3, four full rounds of 256 planes, is split as before.
+constexpr double MARCH_START = 2.5;
 struct March {
   int nbx, nby, nzc, kz, nb;
-  __host__ bool init(int nbx_, int nby_, int nk, int kz_) {
+  __host__ bool init(int nbx_, int nby_, int nk, int kz_, int slots) {
     if (kz_ < 1 || nk < 1) return false;
     nbx = nbx_; nby = nby_;
-    while (kz_ > 4 && (long)nbx * nby * ((nk + kz_ - 1) / kz_) < 256)
-      kz_ = (kz_ + 1) / 2 < 4 ? 4 : (kz_ + 1) / 2;
-    nzc = (nk + kz_ - 1) / kz_;
-    kz = (nk + nzc - 1) / nzc;  // the chunks as even as the count allows
+    split_rounds(nk, (long)nbx * nby, kz_, slots, MARCH_START, 4.0, kz, nzc);
     const long n = (long)nbx * nby * nzc;
     if (n > 2147483647L || n <= 0) return false;
     nb = (int)n;
@@ -228,6 +257,14 @@ __device__ __forceinline__ float cfl_candidate_v(R ro, R vx, R vy, R vz, R bx, R
   const R ca = dsqrt((+bx * bx + by * by + bz * bz) / ro * Const<R>::pii4);
   const R total_vel = cs + vv + ca;
   return static_cast<float>(cfl * hmin / total_vel);
+}
+
+// slot = min(slot, v).  The load lets most of a launch's waves do without the
+// atomic (a value read too early is only larger): all of them on one word
+// take about 10 ns each in turn (y walk of 1131 x 757 in FP32 59 -> 39 us; where
+// the slots are many, a batch's, the load is what costs: 180 -> 229).
+__device__ __forceinline__ void slot_min(unsigned *slot, unsigned v) {
+  if (v < __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(slot, v);
 }
 
 // minimum over the 64 lanes of a wave (all lanes must be active)

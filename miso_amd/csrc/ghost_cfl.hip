@@ -141,7 +141,7 @@ __global__ __launch_bounds__(256) void cfl_kernel(Fld<const R> q, const R *__res
   if (threadIdx.x == 0) {
     unsigned b = red[0];
     for (int w = 1; w < (int)(blockDim.x >> 6); ++w) b = min(b, red[w]);
-    atomicMin(slot, b);
+    slot_min(slot, b);
   }
 }
 

@@ -142,11 +142,10 @@ hipError_t launch_stream(hipStream_t, const void *, void *, size_t, int, double 
 // waves then take four rows of that axis).
 __host__ __device__ inline int walk_waves_x(int n_other) { return n_other < 4 ? 4 : 1; }
 
-// Chunks of a walk over n_dir cells: the requested length (at least 4),
-// halved while the launch would have fewer than 2^18 threads (a small grid
-// walked in long chunks leaves the chip idle), then evened out.  Every
-// chunk recomputes its first slopes and flux from the fields, so the
-// results do not depend on the split.
+// Chunks of a walk over n_dir cells in a batch: the requested length (at
+// least 4), halved while the launch would have fewer than 2^18 threads, then
+// evened out.  Every chunk recomputes its first slopes and flux from the
+// fields, so the results do not depend on the split.
 inline void walk_split(int n_dir, long threads_per_chunk, int chunk_req, int &chunk,
                        int &nchunks) {
   int c = chunk_req < 4 ? 4 : chunk_req;
@@ -247,6 +246,7 @@ template <typename R>
 hipError_t launch_av_sweep_xy(hipStream_t, const Fld<const R> &, const Fld<R> &, R *, const R *,
                               const R *, const Shape &, const BcDev &, const AvScalars &);
 // the chunks a y (dir 1) or z (dir 2) walk of this shape is cut into
+template <typename R>
 void av_walk_split(const Shape &sh, int dir, int chunk_req, int *chunk, int *nchunks);
 template <typename R>
 hipError_t launch_char_vel(hipStream_t, const Fld<const R> &, R *, int, const AvScalars &);

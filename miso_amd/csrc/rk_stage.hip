@@ -889,7 +889,7 @@ static hipError_t launch_rk_t(hipStream_t st, const Fld<const R> &o, const Fld<c
     const int ty = sc.variant == 4 ? 4 : (sc.variant == 6 && sizeof(R) == 4) ? 12 : 8;
     March mc;
     if (sh.mi < 2 || sh.mj < 2 || sh.mk < 2 ||
-        !mc.init((ni + 63) / 64, (nj + ty - 1) / ty, nk, sc.zchunk))
+        !mc.init((ni + 63) / 64, (nj + ty - 1) / ty, nk, sc.zchunk, ty == 4 ? 512 : 256))
       return hipErrorInvalidValue;
     bool same = true;
     for (int m = 0; m < 9; ++m) same = same && o.q[m] == a.q[m];
