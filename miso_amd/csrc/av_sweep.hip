@@ -315,7 +315,7 @@ __device__ __forceinline__ void av_cell_update(const AvCons<R> &a, const R fdw[9
 }
 
 // CFLF: also reduce the CFL candidates of the stored results into cf.slot
-// (one atomicMin per wave), the next step's dt.
+// (at most one atomicMin per block), the next step's dt.
 template <typename R, int DIR, bool DEGEN = false, bool CFLF = false>
 __device__ __forceinline__ void av_walk_block(const Fld<const R> &qq, const Fld<R> &rslt,
                                               const R *__restrict__ cc,
@@ -438,9 +438,10 @@ __device__ __forceinline__ void av_walk_block(const Fld<const R> &qq, const Fld<
       d0[f] = d1;
     }
     const R dd = dd_arr[__builtin_amdgcn_readfirstlane(m_dir + p0 + t)];
-    if (CFLF) {
+    if (CFLF || (DIR == 1 && DEGEN)) {
       R st[9];
       av_cell_update<R, DEGEN>(a0, fdw, fup, dd, dt, rslt, c, cc_0, ep, fh, dz0, st);
+      if constexpr (CFLF) {
       if (cf->heat_q) {  // the heating kernel's expression on the stored values
         const double e = double(st[7]) + cf->heat_dt * cf->heat_q[c] / double(st[0]);
         st[7] = R(e);
@@ -451,6 +452,8 @@ __device__ __forceinline__ void av_walk_block(const Fld<const R> &qq, const Fld<
       const float cand = cfl_candidate_v(st[0], st[1], st[2], st[3], st[4], st[5], st[6], st[7],
                                          R(cf->gm), R(cf->cfl), hmin);
       best = min(best, __float_as_uint(cand));
+      }
+      if (DIR == 1 && DEGEN && sc.img.on) ghost_images(rslt, sh, sc.img, i, pd, st);
     } else {
       av_cell_update<R, DEGEN>(a0, fdw, fup, dd, dt, rslt, c, cc_0, ep, fh, dz0);
     }
@@ -476,8 +479,11 @@ __device__ __forceinline__ void av_walk_block(const Fld<const R> &qq, const Fld<
   if (t < len) step(nb0, cb0, t);
   }
   if (CFLF) {
+    __shared__ unsigned red[4];
     best = wave_umin(best);
-    if ((threadIdx.x & 63) == 0) slot_min(cf->slot, best);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = best;
+    __syncthreads();
+    if (threadIdx.x == 0) slot_min(cf->slot, min(min(red[0], red[1]), min(red[2], red[3])));
   }
 }
 
@@ -549,7 +555,11 @@ __device__ __forceinline__ void av_xshfl_block(const Fld<const R> &qq, const Fld
     fup[f] = flux_core(a.v[f], vp, d, dn, cup, fh);
     fdw[f] = lane_up(fup[f]);
   }
-  if (out_lane) av_cell_update(a, fdw, fup, dxi[i], dt, rslt, c);
+  if (out_lane) {
+    R st[9];
+    av_cell_update(a, fdw, fup, dxi[i], dt, rslt, c, R(0), R(0), R(0), R(0), st);
+    if (sc.img.on) ghost_images(rslt, sh, sc.img, i, j, st);
+  }
 }
 
 template <typename R>
@@ -558,6 +568,7 @@ __global__ __launch_bounds__(256) void av_xshfl_kernel(Fld<const R> qq, Fld<R> r
                                                       const R *__restrict__ dxi, Shape sh,
                                                       int j_lo, int k_lo, int j_n, int k_n,
                                                       int nseg, int nb, AvScalars sc) {
+  if (sc.clear && blockIdx.x == 0 && threadIdx.x == 0) *sc.clear = CFL_NONE;
   av_xshfl_block<R>(qq, rslt, cc_store, dxi, sh, j_lo, k_lo, j_n, k_n, nseg, sc, R(sc.dt),
                     xcd_virtual_block(blockIdx.x, nb));
 }
@@ -715,6 +726,7 @@ __global__ __launch_bounds__(256) __attribute__((
                                                         const R *__restrict__ dyi, Shape sh,
                                                         BcDev bc, int chunk, int nchunks,
                                                         int nseg, int nwaves, AvScalars sc) {
+  if (sc.clear && blockIdx.x == 0 && threadIdx.x == 0) *sc.clear = CFL_NONE;
   const int w = xcd_virtual_block(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6);
   if (w >= nwaves) return;  // whole wave; the kernel has no block barrier
   const int seg = w % nseg, rr = w / nseg, ch = rr % nchunks;
@@ -1020,6 +1032,7 @@ __global__ __launch_bounds__(256) void batch_av_kernel(const BatchInst<R> *__res
                                                        const int *__restrict__ start, int n,
                                                        int total, int in_set, int out_set,
                                                        AvScalars sc) {
+  sc.img.on = 0;  // a batch fills the ghost cells of all runs in one launch
   const int V = xcd_virtual_block(blockIdx.x, total);
   const int m = batch_find(start, n, V);
   const int b = V - start[m];

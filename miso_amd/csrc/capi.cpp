@@ -123,7 +123,7 @@ BcDev make_bc(const misohip_bc *bc) {
 template <typename R>
 int rk_stage_t(misohip_ctx *ctx, const misohip_grid *g, const misohip_params *p,
                const misohip_fields *o, const misohip_fields *a, const misohip_fields *r,
-               R dt_s, R ch2, R damp, int wrap = 0) {
+               R dt_s, R ch2, R damp, int wrap = 0, const GhostImg &img = {}) {
   // a user source first writes src.vx, src.vy, src.vz, src.ei of this
   // stage's argm (the reference evaluates the functor on argm inside the
   // stage, mhd_integrator_host.hpp:134,151,168,241)
@@ -139,6 +139,7 @@ int rk_stage_t(misohip_ctx *ctx, const misohip_grid *g, const misohip_params *p,
   sc.variant = ctx->tile.rk_variant;
   sc.zchunk = ctx->tile.rk_zchunk;
   sc.wrap = wrap;
+  sc.img = img;
   MISOHIP_TRY(launch_rk_stage<R>(ctx->stream, cfld<R>(o), cfld<R>(a), fld<R>(r),
                                  static_cast<const R *>(g->dxi), static_cast<const R *>(g->dyi),
                                  static_cast<const R *>(g->dzi), make_shape(g), sc));
@@ -155,11 +156,14 @@ template <typename R> AvScalars av_scalars(const misohip_params *p, R dt, int ch
 
 template <typename R>
 int av_sweep_t(misohip_ctx *ctx, const misohip_grid *g, const misohip_params *p, int dir, R dt,
-               const misohip_fields *q, const misohip_fields *r, void *cc, int wrap = 0) {
+               const misohip_fields *q, const misohip_fields *r, void *cc, int wrap = 0,
+               const GhostImg &img = {}, unsigned *clear = nullptr) {
   const R *dd = static_cast<const R *>(dir == 0 ? g->dxi : dir == 1 ? g->dyi : g->dzi);
   Timed t_(ctx, MISOHIP_KIND_AV_X + dir);
   AvScalars sc = av_scalars<R>(p, dt, ctx->tile.sweep_chunk);
   sc.wrap = wrap;
+  sc.img = img;
+  sc.clear = clear;
   MISOHIP_TRY(launch_av_sweep<R>(ctx->stream, dir, cfld<R>(q), fld<R>(r), static_cast<R *>(cc),
                                  static_cast<const R *>(cc), dd, make_shape(g), sc));
   return MISOHIP_OK;
@@ -322,6 +326,9 @@ int update_t(misohip_ctx *ctx, const misohip_grid *g, const misohip_params *p,
   if (fuse_xy && ctx->tile.rk_variant >= 4 && ctx->tile.rk_variant <= 6)
     for (int a = 0; a < 3; ++a)
       if (bc->periodic[a] == 1) wrap |= 1 << a;
+  // In an x-y run with periodic and mirrored axes every pass stores the ghost
+  // cells with their sources instead, and no fill runs.
+  const GhostImg img = ctx->bc_fn ? GhostImg{} : ghost_img(sh, b);
   // stage 1 reads qq as both orgn and argm; later stages ping-pong between
   // the two workspace field sets.
   const misohip_fields *argm = qq;
@@ -330,9 +337,9 @@ int update_t(misohip_ctx *ctx, const misohip_grid *g, const misohip_params *p,
     const misohip_fields *out = s == 3 ? &w->rslt : bufs[s & 1];
     if (s == 3 && argm == &w->rslt) out = &w->argm;
     const R damp = (R)std::exp(-dts[s] / tau);
-    int rc = rk_stage_t<R>(ctx, g, p, qq, argm, out, dts[s], ch2, damp, wrap);
+    int rc = rk_stage_t<R>(ctx, g, p, qq, argm, out, dts[s], ch2, damp, wrap, img);
     if (rc) return rc;
-    rc = ghost_t<R>(ctx, out, sh, b, 7 & ~wrap);
+    rc = ghost_t<R>(ctx, out, sh, b, img.on ? 0 : 7 & ~wrap);
     if (rc) return rc;
     argm = out;
   }
@@ -365,6 +372,7 @@ int update_t(misohip_ctx *ctx, const misohip_grid *g, const misohip_params *p,
       Timed t_(ctx, MISOHIP_KIND_AV_X);
       AvScalars sc = av_scalars<R>(p, dt, ctx->tile.av_xy_chunk);
       sc.wrap = wrap;
+      sc.clear = fuse_cfl ? ctx->d_slot : nullptr;
       sc.xy_waves = ctx->tile.av_fuse_xy == 2 || ctx->tile.av_fuse_xy == 4 ? 2 : 3;
       MISOHIP_TRY(launch_av_sweep_xy<R>(ctx->stream, cfld<R>(cur), fld<R>(dst),
                                         static_cast<R *>(w->cc), static_cast<const R *>(g->dxi),
@@ -381,22 +389,24 @@ int update_t(misohip_ctx *ctx, const misohip_grid *g, const misohip_params *p,
       cf.slot = ctx->d_slot;
       cf.heat_q = heat_q;
       cf.heat_dt = (double)dt;
-      MISOHIP_TRY(launch_cfl_init(ctx->stream, ctx->d_slot));
       AvScalars sc = av_scalars<R>(p, dt, ctx->tile.sweep_chunk);
       sc.wrap = fuse_xy ? wrap : 0;
+      sc.img = img;
       MISOHIP_TRY(launch_av_last_sweep_cfl<R>(
           ctx->stream, cfld<R>(cur), fld<R>(dst), static_cast<const R *>(w->cc),
           static_cast<const R *>(g->dyi), static_cast<const R *>(g->dzi), sh, sc, cf));
       rc = MISOHIP_OK;
     } else if (dir == 1 && fuse_z) {
       Timed t_(ctx, MISOHIP_KIND_AV_Y);
+      AvScalars sc = av_scalars<R>(p, dt, ctx->tile.sweep_chunk);
+      sc.img = img;
       MISOHIP_TRY(launch_av_sweep_y_degen_z<R>(
           ctx->stream, cfld<R>(cur), fld<R>(dst), static_cast<const R *>(w->cc),
-          static_cast<const R *>(g->dyi), static_cast<const R *>(g->dzi), sh,
-          av_scalars<R>(p, dt, ctx->tile.sweep_chunk)));
+          static_cast<const R *>(g->dyi), static_cast<const R *>(g->dzi), sh, sc));
       rc = MISOHIP_OK;
     } else {
-      rc = av_sweep_t<R>(ctx, g, p, dir, dt, cur, dst, w->cc, fuse_xy ? wrap : 0);
+      rc = av_sweep_t<R>(ctx, g, p, dir, dt, cur, dst, w->cc, fuse_xy ? wrap : 0, img,
+                         dir == 0 && fuse_cfl ? ctx->d_slot : nullptr);
     }
     if (rc) return rc;
     // after the x-y walk only the z walk reads the state, along z alone; the
@@ -404,7 +414,7 @@ int update_t(misohip_ctx *ctx, const misohip_grid *g, const misohip_params *p,
     // their sources, so a run fills them after its last step only
     const int axes = last ? (fill_periodic ? 7 : 7 & ~wrap)
                           : (dir == 0 && fuse_xy && wrap) ? 4 & ~wrap : 7;
-    rc = ghost_t<R>(ctx, dst, sh, b, axes);
+    rc = ghost_t<R>(ctx, dst, sh, b, img.on ? 0 : axes);
     if (rc) return rc;
     if (dir == 1 && fuse_z) break;
     other = cur;

@@ -218,6 +218,46 @@ struct Shape {
   }
 };
 
+// Boundaries of an x-y run (periodic or mirrored axes) for the passes that
+// store ghost cells themselves: a fill of its own costs a run more in its
+// launch than in bytes.  A step of 256^2 in FP64 96 -> 58 us (six fills of 6
+// us), of 1131 x 757 in FP32 196 -> 166; the passes take up to 1 us longer, or
+// 4 % where they are large: in a batch, whose fills are one launch for all
+// runs, that is what the fills cost (17.6 ms either way for four steps of 64
+// runs of 128^2 .. 1024^2).
+struct GhostImg {
+  int on = 0;
+  int periodic[2] = {0, 0};     // x, y; else mirrored
+  unsigned flip[2] = {0u, 0u};  // bit f: field f changes sign across a mirrored axis
+};
+
+// The ghost cells whose source is interior cell (i, j), from its nine values:
+// what the ghost fill would copy there, each coordinate mapped on its own.
+template <typename R>
+__device__ __forceinline__ void ghost_images(const Fld<R> &out, const Shape &sh,
+                                             const GhostImg &im, int i, int j, const R (&v)[9]) {
+  const bool xl = i < 2 * sh.mi, xh = i >= sh.It - 2 * sh.mi;
+  const bool yl = j < 2 * sh.mj, yh = j >= sh.Jt - 2 * sh.mj;
+  if (!(xl || xh || yl || yh)) return;
+  const int ni = sh.It - 2 * sh.mi, nj = sh.Jt - 2 * sh.mj;
+#pragma unroll 1
+  for (int n = 1; n < 9; ++n) {  // per axis: 0 the cell's own coordinate, 1, 2 the images of
+    const int a = n % 3, b = n / 3;  // the cells at the low and at the high end
+    if ((a == 1 && !xl) || (a == 2 && !xh) || (b == 1 && !yl) || (b == 2 && !yh)) continue;
+    const int gi = a == 0 ? i
+                 : im.periodic[0] ? (a == 1 ? i + ni : i - ni)
+                                  : 2 * (a == 1 ? sh.mi : sh.It - sh.mi) - 1 - i;
+    const int gj = b == 0 ? j
+                 : im.periodic[1] ? (b == 1 ? j + nj : j - nj)
+                                  : 2 * (b == 1 ? sh.mj : sh.Jt - sh.mj) - 1 - j;
+    const unsigned flip = (a && !im.periodic[0] ? im.flip[0] : 0u) ^
+                          (b && !im.periodic[1] ? im.flip[1] : 0u);
+    const int g = sh.idx(gi, gj, 0);
+#pragma unroll
+    for (int f = 0; f < 9; ++f) out.q[f][g] = (flip >> f) & 1u ? -v[f] : v[f];
+  }
+}
+
 // Generalised minmod slope, limiter.hpp:10-22.  The two terms of the final
 // sum, min(0, max) and max(0, min) with min <= max, are float-narrowed and
 // at least one of them is a zero, so their sum is exact in float: it is
@@ -258,6 +298,8 @@ __device__ __forceinline__ float cfl_candidate_v(R ro, R vx, R vy, R vz, R bx, R
   const R total_vel = cs + vv + ca;
   return static_cast<float>(cfl * hmin / total_vel);
 }
+
+constexpr unsigned CFL_NONE = 0x501502f9u;  // 1e10f: a CFL reduction's start
 
 // slot = min(slot, v).  The load lets most of a launch's waves do without the
 // atomic (a value read too early is only larger): all of them on one word

@@ -105,7 +105,7 @@ hipError_t launch_ghost_fill(hipStream_t st, const Fld<R> &q, const Shape &sh, c
 
 // ---------------------------------------------------------------- CFL
 __global__ void cfl_init_kernel(unsigned *slot) {
-  if (threadIdx.x == 0) slot[0] = __float_as_uint(1.e10f);
+  if (threadIdx.x == 0) slot[0] = CFL_NONE;
 }
 
 template <typename R>

@@ -22,6 +22,7 @@ struct RkScalars {
   // src_kind 2: src.vx, src.vy, src.vz, src.ei of the stage's argm (fields
   // of the grid's shape, the run's Real)
   const void *src_arr[4];
+  GhostImg img;  // x-y runs: ghost cells stored with their sources
 };
 
 // Scalars of one AV sweep (ArtificialViscosity members plus dt).
@@ -36,6 +37,10 @@ struct AvScalars {
   // nparts), the x-y walk's planes part0, part0 + 1, ... (nparts of them; a
   // range past the top z ring plane continues at the bottom one); 0: all
   int part0 = 0, nparts = 0;
+  GhostImg img;  // x-y runs: ghost cells stored with their sources
+  // x sweep, x-y walk: the CFL slot that this step's last sweep reduces into,
+  // cleared on the way (none: null)
+  unsigned *clear = nullptr;
 };
 
 // Boundary description on the device: axis kind (0 mirror, 1 periodic,
@@ -45,6 +50,19 @@ struct BcDev {
   float sign[3][9];
   const void *fixed[9];
 };
+
+// the ghost cells of an x-y run that its passes can store themselves
+inline GhostImg ghost_img(const Shape &sh, const BcDev &b) {
+  GhostImg m;
+  m.on = sh.is && sh.js && !sh.ks && b.periodic[0] < 2 && b.periodic[1] < 2 &&
+         sh.It >= 3 * sh.mi && sh.Jt >= 3 * sh.mj;  // every image is a ghost cell
+  for (int a = 0; a < 2; ++a) {
+    m.periodic[a] = b.periodic[a];
+    for (int f = 0; f < 9; ++f)
+      if (b.sign[a][f] < 0.f) m.flip[a] |= 1u << f;
+  }
+  return m;
+}
 
 // one ray of the sweep, everything the plane kernel needs
 struct RtRay {

@@ -151,7 +151,7 @@ __device__ __forceinline__ void rk_update(const R o[9], const Fld<R> &rslt, int 
                                           const R damp, R a_ro, R a_vx, R d4x, R d5x, R t_vx,
                                           R a_vy, R d4y, R d5y, R t_vy, R a_vz, R d4z, R d5z,
                                           R t_vz, R a_bx, R a_by, R a_bz, R a_ph, R a_ei,
-                                          R t_ei) {
+                                          R t_ei, R *stored = nullptr) {
   const R pii4 = Const<R>::pii4, pii8 = Const<R>::pii8;
   const R o_ro = o[0], o_vx = o[1], o_vy = o[2], o_vz = o[3];
   const R o_bx = o[4], o_by = o[5], o_bz = o[6];
@@ -200,6 +200,10 @@ __device__ __forceinline__ void rk_update(const R o[9], const Fld<R> &rslt, int 
   rslt.q[6][c] = bz;
   rslt.q[7][c] = R(ei);
   rslt.q[8][c] = ph;
+  if (stored) {
+    stored[0] = ro; stored[1] = vx; stored[2] = vy; stored[3] = vz; stored[4] = bx;
+    stored[5] = by; stored[6] = bz; stored[7] = R(ei); stored[8] = ph;
+  }
 }
 
 // Energy recovery is carried in double for both storage types ("pressure
@@ -312,8 +316,12 @@ __device__ __forceinline__ void rk_block(const Fld<const R> &orgn, const Fld<con
 #pragma unroll
   for (int m = 0; m < 9; ++m) o[m] = orgn.q[m][c];
   const R gro = sc.src_kind == 1 ? argm.q[0][c] : R(0);
+  R st[9];
   rk_update<R>(o, rslt, c, gro, sc, dt, ch2, damp, a_ro, a_vx, d4x, d5x, t_vx, a_vy, d4y_,
-               d5y_, t_vy, a_vz, d4z, d5z, t_vz, a_bx, a_by, a_bz, a_ph, a_ei, t_ei);
+               d5y_, t_vy, a_vz, d4z, d5z, t_vz, a_bx, a_by, a_bz, a_ph, a_ei, t_ei, st);
+  if constexpr (HX && HY && !HZ) {
+    if (sc.img.on) ghost_images(rslt, sh, sc.img, i, j, st);
+  }
 }
 
 template <typename R, bool HX, bool HY, bool HZ, int SPLIT>
@@ -838,8 +846,10 @@ __device__ __forceinline__ void rk_ywalk_wave(const Fld<const R> &orgn, const Fl
     t_ei = t_ei + S[16];
     if (out) {
       const R gro = sc.src_kind == 1 ? w[2][0] : R(0);
+      R st[9];
       rk_update<R>(o, rslt, c, gro, sc, dt, ch2, damp, a_ro, a_vx, d4x, d5x, t_vx, a_vy, d4y,
-                   d5y, t_vy, a_vz, d4z, d5z, t_vz, a_bx, a_by, a_bz, a_ph, a_ei, t_ei);
+                   d5y, t_vy, a_vz, d4z, d5z, t_vz, a_bx, a_by, a_bz, a_ph, a_ei, t_ei, st);
+      if (sc.img.on) ghost_images(rslt, sh, sc.img, i, j, st);
     }
     // the window moves up a row; row j+4 is loaded for the step after next
 #pragma unroll
@@ -982,6 +992,7 @@ __global__ __launch_bounds__(256) void batch_rk_ywalk_kernel(const BatchInst<R> 
                                                              const int *__restrict__ start, int n,
                                                              int total, int stage, int in_set,
                                                              int out_set, RkScalars sc) {
+  sc.img.on = 0;  // a batch fills the ghost cells of all runs in one launch
   const int V = xcd_virtual_block(blockIdx.x, total);
   const int m = batch_find(start, n, V);
   const BatchInst<R> &I = inst[m];
@@ -1005,6 +1016,7 @@ __global__ __launch_bounds__(256) void batch_rk_kernel(const BatchInst<R> *__res
                                                        const int *__restrict__ start, int n,
                                                        int total, int stage, int in_set,
                                                        int out_set, RkScalars sc) {
+  sc.img.on = 0;
   const int V = xcd_virtual_block(blockIdx.x, total);
   const int m = batch_find(start, n, V);
   const int b = V - start[m];

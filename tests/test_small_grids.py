@@ -1,0 +1,51 @@
+"""Small and ragged grids against the oracle, bit for bit: launches cut into
+chunks of one cell or plane, and the ghost cells that the passes of an x-y
+run store beside their sources (whole arrays, corners included)."""
+import numpy as np
+import pytest
+
+from tests.parity_util import assert_bitwise, random_state
+
+# components that change sign across a wall of each axis
+SIGNS = tuple(tuple(-1 if f in (1 + a, 4 + a) else 1 for f in range(9)) for a in range(3))
+
+
+def _both(ctx, sizes, periodic, nsteps, use_run):
+    from miso_amd import mhd
+    from oracle import oracle as O
+    og = O.make_grid(sizes, 2, dtype=np.float64)
+    op = O.Params(cfl_number=0.4, periodic=periodic, sym_sign=SIGNS)
+    g = mhd.Grid(*sizes, 2, dtype=np.float64, device="cuda:0")
+    ref = random_state((g.i_total, g.j_total, g.k_total), 3, amp=0.05)
+    O.ghost_fill(og, op, ref)
+    q0 = ref.copy()
+    ref_dts = O.run(og, op, ref, nsteps)
+    O.ghost_fill(og, op, ref)
+    m = mhd.MHD(mhd.Config({"mhd": {"cfl_number": 0.4}}), g, ctx, gm=5.0 / 3.0)
+    bc = mhd.BoundaryCondition(periodic, SIGNS)
+    m.apply_initial_condition(q0, bc)
+    if use_run:
+        dts = m.integrator.run(bc, m.qq, nsteps)
+    else:
+        dts = [m.integrator.step(bc, m.qq) for _ in range(nsteps)]
+    return m.qq.to_host(ctx), ref, np.array(dts), ref_dts
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", [(2, 2, 1), (3, 5, 1), (64, 4, 1), (7, 61, 1), (129, 66, 1)])
+@pytest.mark.parametrize("periodic", [(1, 1, 1), (0, 1, 1), (1, 0, 1), (0, 0, 1)])
+@pytest.mark.parametrize("use_run", [False, True])
+def test_xy_runs_with_their_ghost_cells(ctx, sizes, periodic, use_run):
+    out, ref, dts, ref_dts = _both(ctx, sizes, periodic, 3, use_run)
+    assert np.array_equal(dts, ref_dts), (dts, ref_dts)
+    assert_bitwise(out, ref, f"{sizes} {periodic}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", [(4, 3, 2), (65, 2, 3), (61, 9, 1 + 64), (6, 131, 5)])
+@pytest.mark.parametrize("periodic", [(1, 1, 1), (0, 0, 0), (1, 0, 1)])
+def test_3d_runs_in_the_shortest_chunks(ctx, sizes, periodic):
+    out, ref, dts, ref_dts = _both(ctx, sizes, periodic, 3, True)
+    assert np.array_equal(dts, ref_dts), (dts, ref_dts)
+    sl = (slice(None),) + (slice(2, -2),) * 3  # the oracle's 3D edges keep what was there
+    assert_bitwise(out[sl], ref[sl], f"{sizes} {periodic}")
