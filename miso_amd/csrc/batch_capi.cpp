@@ -9,6 +9,7 @@
 // single-run kernels' block functions, the per-instance scalars are formed
 // with the host path's arithmetic (batch_params_kernel), and exp(-dt_s/tau)
 // is taken from a table of host-library values.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <new>
@@ -179,11 +180,20 @@ int create_t(misohip_ctx *ctx, int n, const misohip_grid *grids, const misohip_f
     I.dyi = static_cast<const R *>(g->dyi); I.dzi = static_cast<const R *>(g->dzi);
     I.sh = shape_of(g);
     I.min_dxyz = g->min_dxyz;
-    // this run's y walk alone decides (the tuner's per-run choice replaces it)
-    int nch = 0;
-    walk_split(g->j_size, 64L * ((g->i_size + 63) / 64) * (g->ks ? g->k_size : 1), chunk, I.chunk,
-               nch);
   }
+  // The walks' length, one for all runs (the tuner's per-run choice replaces
+  // it).  With A rows for each of the waves that run at a time, walks of c
+  // rows take about A / c rounds, half a round more at the end, of c rows and
+  // the four each walk reads besides: least at c = sqrt(8 A).  64 runs of
+  // 128^2 .. 1024^2 in FP32 walk 32 rows: y sweep 773 -> 692 us a step
+  // against lengths that filled the chip with each run alone (4 rows for most).
+  double rows = 0.0;
+  for (int m = 0; m < n; ++m)
+    rows += (double)((grids[m].i_size + 63) / 64) * grids[m].j_size *
+            (grids[m].ks ? grids[m].k_size : 1);
+  const double at_a_time = 1024.0 * (sizeof(R) == 8 ? 1 : 3);
+  const int c = (int)std::sqrt(8.0 * rows / at_a_time);
+  for (BatchInst<R> &I : inst) I.chunk = std::max(4, std::min(c, chunk));
   fill_table(b->tab);
   hipError_t e = hipMalloc(reinterpret_cast<void **>(&b->d_inst), sizeof(BatchInst<R>) * n);
   if (e == hipSuccess) e = hipMalloc(reinterpret_cast<void **>(&b->d_dyn), sizeof(BatchDyn<R>) * n);

@@ -160,19 +160,6 @@ hipError_t launch_stream(hipStream_t, const void *, void *, size_t, int, double 
 // waves then take four rows of that axis).
 __host__ __device__ inline int walk_waves_x(int n_other) { return n_other < 4 ? 4 : 1; }
 
-// Chunks of a walk over n_dir cells in a batch: the requested length (at
-// least 4), halved while the launch would have fewer than 2^18 threads, then
-// evened out.  Every chunk recomputes its first slopes and flux from the
-// fields, so the results do not depend on the split.
-inline void walk_split(int n_dir, long threads_per_chunk, int chunk_req, int &chunk,
-                       int &nchunks) {
-  int c = chunk_req < 4 ? 4 : chunk_req;
-  while (c > 4 && (long)((n_dir + c - 1) / c) * threads_per_chunk < (1L << 18)) c = (c + 1) / 2;
-  if (c < 4) c = 4;
-  nchunks = (n_dir + c - 1) / c;
-  chunk = (n_dir + nchunks - 1) / nchunks;
-}
-
 // ---------------------------------------------------------------- batches
 // One instance of a batched launch: its three field sets (0 = qq, 1 = argm,
 // 2 = rslt), frozen AV speed, metric and shape.  Stored in device memory;
