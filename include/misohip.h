@@ -414,6 +414,19 @@ int misohip_mlp_features(misohip_ctx *ctx, misohip_mlp *m, const misohip_grid *g
 int misohip_mlp_qrad(misohip_ctx *ctx, misohip_mlp *m, const misohip_grid *g, const void *X,
                      float *Y, const int *flags, const void *q_rt, const void *corr,
                      void *qrad);
+/* Training data, row-major [..][width] in dt, on the given stream of the
+ * current device (NULL = the null stream).  Moments of the n rows listed, by
+ * column, in FP64: mean, standard deviation (n - 1), mean magnitude; work is
+ * scratch of 2 x MISOHIP_MOMENT_SHARES x width doubles.  Normalize: out =
+ * (x - mean) / sd of the first n rows, formed in FP64, as FP32 or bf16; width
+ * a multiple of 4, out on a 16-byte boundary. */
+#define MISOHIP_MOMENT_SHARES 64
+int misohip_column_moments(misohip_dtype dt, const void *x, const long long *rows, long n,
+                           int width, double *mean, double *sd, double *mean_abs, double *work,
+                           void *stream);
+int misohip_column_normalize(misohip_dtype dt, const void *x, long n, int width,
+                             const double *mean, const double *sd, int bf16, void *out,
+                             void *stream);
 /* residual indicator of the last network output Y against a plain solve
  * q_rt: flag columns whose relative L2 error over the column exceeds tol;
  * corr (optional) receives q_rt - network on every interior cell, the

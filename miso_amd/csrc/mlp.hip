@@ -40,6 +40,19 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// A barrier for what the workgroup's waves exchange through LDS alone: global
+// loads and stores stay in flight across it (147456 columns of inference 635 ->
+// 622 us).  WIDE: they exchange through global memory too.
+template <bool WIDE> __device__ __forceinline__ void chain_barrier() {
+  if (WIDE) {
+    __syncthreads();
+    return;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // features of X that a workgroup of 64 columns takes at a time
 constexpr int MLP_X_TALL = 128;
 
@@ -70,7 +83,7 @@ constexpr int MLP_X_TALL = 128;
 // At that size and a batch of 1024 a training step's chain takes 37 us, where
 // a launch per layer, product and elementwise step (128 x 128 tiles: 16
 // workgroups) took 232; 147456 columns of inference, their Q_rad field
-// included, 635 us for 957 (without
+// included, 622 us for 957 (without
 // its 1.1 GB of Y, corrections and Q_rad it would take 363).  Every sum is
 // taken in the order of k, 32 at a time, as those took it: the same bits.
 template <int NT, int WAVES, int RT, int PD, bool TRAIN, bool WIDE>
@@ -130,7 +143,7 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
   // features [f0, f0 + cw) of the workgroup's columns into xbuf
   auto stage = [&](int f0) {
     const int cw = min(xw, n_in - f0), per = cw >> 3, n = NS * per;
-    __syncthreads();
+    chain_barrier<WIDE>();
     for (int t = tid; t < n; t += 4 * NTHR) {
       uint4 v[4];
 #pragma unroll
@@ -146,7 +159,7 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
         if (q < n) *reinterpret_cast<uint4 *>(xbuf + r * xpitch + 8 * c) = v[e];
       }
     }
-    __syncthreads();
+    chain_barrier<WIDE>();
     return cw;
   };
   // NT > 1: the thread's part of XW features of the workgroup's columns, in
@@ -203,10 +216,10 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
       steps(b + col * pitch + kq * 8, 16 * pitch, 0, KT);
     } else if constexpr (NT > 1) {
       fetch(0);
-      if (base) __syncthreads();
+      if (base) chain_barrier<WIDE>();
       put(xbuf);
       for (int k0 = 0, h = 0; k0 < KT; k0 += XW / 32, h ^= 1) {
-        __syncthreads();
+        chain_barrier<WIDE>();
         if (k0 + XW / 32 < KT) fetch(k0 * 32 + XW);
         steps(xbuf + (h * NS + col) * xpitch + kq * 8, 16 * xpitch, k0, min(XW / 32, KT - k0));
         if (k0 + XW / 32 < KT) put(xbuf + (h ^ 1) * NS * xpitch);
@@ -325,7 +338,7 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
     else if (TRAIN && l > 0)
       preload(L[l].wtp, L[l].out / 32, L[l].in / 16, 0, tiles_of(L[l].in / 16));
     if (!last || TRAIN) {
-      __syncthreads();
+      chain_barrier<WIDE>();
       if (TRAIN) pack(nxt, pitch, L[l].out, last ? L[l].dT : L[l + 1].aT, 0);
       uint16_t *t = cur;
       cur = nxt;
@@ -357,7 +370,7 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
       }
       if (l > 1)
         preload(L[l - 1].wtp, L[l - 1].out / 32, L[l - 1].in / 16, 0, tiles_of(L[l - 1].in / 16));
-      __syncthreads();
+      chain_barrier<WIDE>();
       pack(nxt, pitch, L[l].in, L[l - 1].dT, 0);
       uint16_t *t = cur;
       cur = nxt;
@@ -634,6 +647,90 @@ __global__ __launch_bounds__(256) void column_features_kernel(
   }
 }
 
+// Sums over chosen rows of a row-major [..][W] array, by column, in FP64: of
+// the values and of their magnitudes, or (SQ) of the squared distances from
+// the mean.  A block takes 64 columns and a share of the rows; its sums go to
+// p0 (p1) [share][column].
+// Bound by HBM: the rows are read twice (the mean first, so that no digits
+// cancel).  14746 x 1536 and their targets: 0.2 ms, where FP64 copies of the
+// rows and library reductions took 1.1.
+template <typename T, bool SQ>
+__global__ __launch_bounds__(256) void moments_kernel(const T *__restrict__ x,
+                                                      const long long *__restrict__ rows, long n,
+                                                      int W, const double *__restrict__ mean,
+                                                      double *__restrict__ p0,
+                                                      double *__restrict__ p1, long share) {
+  __shared__ double red[2][4][64];
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = blockIdx.x * 64 + lane, c = min(col, W - 1);
+  const long r1 = min(n, (blockIdx.y + 1) * share);
+  const double m = SQ ? mean[c] : 0.0;
+  double a = 0.0, b = 0.0;
+#pragma unroll 8
+  for (long r = blockIdx.y * share + wv; r < r1; r += 4) {
+    const double v = (double)x[rows[r] * W + c];
+    if (SQ) {
+      a += (v - m) * (v - m);
+    } else {
+      a += v;
+      b += fabs(v);
+    }
+  }
+  red[0][wv][lane] = a;
+  red[1][wv][lane] = b;
+  __syncthreads();
+  if (wv == 0 && col < W) {
+    const long at = (long)blockIdx.y * W + col;
+    p0[at] = (red[0][0][lane] + red[0][1][lane]) + (red[0][2][lane] + red[0][3][lane]);
+    if (!SQ) p1[at] = (red[1][0][lane] + red[1][1][lane]) + (red[1][2][lane] + red[1][3][lane]);
+  }
+}
+
+// mean and mean magnitude, or (SQ) the standard deviation, from the shares
+template <bool SQ>
+__global__ __launch_bounds__(64) void moments_final_kernel(const double *__restrict__ p0,
+                                                           const double *__restrict__ p1, long n,
+                                                           int W, int shares,
+                                                           double *__restrict__ o0,
+                                                           double *__restrict__ o1) {
+  const int col = blockIdx.x * 64 + threadIdx.x;
+  if (col >= W) return;
+  double a = 0.0, b = 0.0;
+#pragma unroll 16
+  for (int s = 0; s < shares; ++s) {
+    a += p0[(long)s * W + col];
+    if (!SQ) b += p1[(long)s * W + col];
+  }
+  if (SQ) {
+    o0[col] = sqrt(a / (n ? (double)(n - 1) : 0.0));
+  } else {
+    o0[col] = a / (double)n;
+    o1[col] = b / (double)n;
+  }
+}
+
+// (x - mean) / sd in FP64, four columns a thread, to bf16 (by way of FP32) or
+// FP32
+template <typename T, bool BF>
+__global__ __launch_bounds__(256) void normalize_kernel(const T *__restrict__ x, long n4, int W,
+                                                        const double *__restrict__ mean,
+                                                        const double *__restrict__ sd,
+                                                        void *__restrict__ out) {
+  typedef T x4 __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+  const long t = (long)blockIdx.x * 256 + threadIdx.x;
+  if (t >= n4) return;
+  const int c = (int)(4 * t % W);
+  const x4 v = reinterpret_cast<const x4 *>(x)[t];
+  f32x4 y;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) y[e] = (float)(((double)v[e] - mean[c + e]) / sd[c + e]);
+  if (BF)
+    reinterpret_cast<uint2 *>(out)[t] = f2bf4(y);
+  else
+    reinterpret_cast<f32x4 *>(out)[t] = y;
+}
+
 // residual indicator per column: relative L2 of (mlp - rt) over the column
 // above `tol` -> flag = 1; corr (optional) receives rt - mlp on every cell
 __global__ void column_residual_kernel(const float *__restrict__ Y, Shape sh,
@@ -758,6 +855,47 @@ hipError_t launch_column_features(hipStream_t st, const Fld<const double> &q, co
   if (nb > 2147483647L) return hipErrorInvalidValue;
   hipLaunchKernelGGL(column_features_kernel, dim3((unsigned)nb), dim3(256), 0, st, q, sh, gm, mu,
                      sd, X, Xf, nfeat, nbx, (int)nb);
+  return hipGetLastError();
+}
+
+template <typename T>
+static hipError_t moments(hipStream_t st, const T *x, const long long *rows, long n, int W,
+                          double *mean, double *sd, double *mean_abs, double *work) {
+  const dim3 grid((W + 63) / 64, MLP_SHARES), one((W + 63) / 64);
+  const long share = (n + MLP_SHARES - 1) / MLP_SHARES;
+  double *p1 = work + (long)MLP_SHARES * W;
+  hipLaunchKernelGGL((moments_kernel<T, false>), grid, dim3(256), 0, st, x, rows, n, W, nullptr,
+                     work, p1, share);
+  hipLaunchKernelGGL((moments_final_kernel<false>), one, dim3(64), 0, st, work, p1, n, W,
+                     MLP_SHARES, mean, mean_abs);
+  hipLaunchKernelGGL((moments_kernel<T, true>), grid, dim3(256), 0, st, x, rows, n, W, mean, work,
+                     nullptr, share);
+  hipLaunchKernelGGL((moments_final_kernel<true>), one, dim3(64), 0, st, work, nullptr, n, W,
+                     MLP_SHARES, sd, nullptr);
+  return hipGetLastError();
+}
+
+hipError_t launch_moments(hipStream_t st, const void *x, bool f64, const long long *rows, long n,
+                          int W, double *mean, double *sd, double *mean_abs, double *work) {
+  if (f64)
+    return moments(st, static_cast<const double *>(x), rows, n, W, mean, sd, mean_abs, work);
+  return moments(st, static_cast<const float *>(x), rows, n, W, mean, sd, mean_abs, work);
+}
+
+hipError_t launch_normalize(hipStream_t st, const void *x, bool f64, long n, int W,
+                            const double *mean, const double *sd, void *out, bool bf16) {
+  const long n4 = n * W / 4;
+  const dim3 grid((unsigned)((n4 + 255) / 256));
+  const double *xd = static_cast<const double *>(x);
+  const float *xf = static_cast<const float *>(x);
+  if (f64 && bf16)
+    hipLaunchKernelGGL((normalize_kernel<double, true>), grid, dim3(256), 0, st, xd, n4, W, mean, sd, out);
+  else if (f64)
+    hipLaunchKernelGGL((normalize_kernel<double, false>), grid, dim3(256), 0, st, xd, n4, W, mean, sd, out);
+  else if (bf16)
+    hipLaunchKernelGGL((normalize_kernel<float, true>), grid, dim3(256), 0, st, xf, n4, W, mean, sd, out);
+  else
+    hipLaunchKernelGGL((normalize_kernel<float, false>), grid, dim3(256), 0, st, xf, n4, W, mean, sd, out);
   return hipGetLastError();
 }
 

@@ -1,6 +1,7 @@
 // What the surrogate's kernels (mlp.hip) and its C ABI (mlp_capi.cpp) share.
 #pragma once
 
+#include "../../include/misohip.h"
 #include "launch.hpp"
 
 namespace misohip {
@@ -54,6 +55,11 @@ hipError_t launch_mlp_adam(hipStream_t, const MlpLayer *, int nl, int tiles, con
 hipError_t launch_mlp_pack(hipStream_t, const MlpLayer *, int nl, int layer, int tiles);
 hipError_t launch_column_features(hipStream_t, const Fld<const double> &, const Shape &, double,
                                   const float *, const float *, uint16_t *, float *, int);
+constexpr int MLP_SHARES = MISOHIP_MOMENT_SHARES;
+hipError_t launch_moments(hipStream_t, const void *x, bool f64, const long long *rows, long n,
+                          int W, double *mean, double *sd, double *mean_abs, double *work);
+hipError_t launch_normalize(hipStream_t, const void *x, bool f64, long n, int W,
+                            const double *mean, const double *sd, void *out, bool bf16);
 hipError_t launch_column_residual(hipStream_t, const float *, const Shape &, const float *,
                                   const float *, const double *, int *, float, double *);
 

@@ -282,6 +282,29 @@ int misohip_mlp_qrad(misohip_ctx *ctx, misohip_mlp *m, const misohip_grid *g, co
   return MISOHIP_OK;
 }
 
+int misohip_column_moments(misohip_dtype dt, const void *x, const long long *rows, long n,
+                           int width, double *mean, double *sd, double *mean_abs, double *work,
+                           void *stream) {
+  if (!x || !rows || !mean || !sd || !mean_abs || !work || n < 0 || width < 1)
+    return MISOHIP_E_ARG;
+  if (dt != MISOHIP_F64 && dt != MISOHIP_F32) return MISOHIP_E_DTYPE;
+  MISOHIP_TRY(launch_moments(static_cast<hipStream_t>(stream), x, dt == MISOHIP_F64, rows, n,
+                             width, mean, sd, mean_abs, work));
+  return MISOHIP_OK;
+}
+
+int misohip_column_normalize(misohip_dtype dt, const void *x, long n, int width,
+                             const double *mean, const double *sd, int bf16, void *out,
+                             void *stream) {
+  if (!x || !mean || !sd || !out || n < 0 || width < 4 || width % 4) return MISOHIP_E_ARG;
+  if (dt != MISOHIP_F64 && dt != MISOHIP_F32) return MISOHIP_E_DTYPE;
+  if ((double)n * width / 1024.0 >= 4294967295.0) return MISOHIP_E_RANGE;
+  if (n == 0) return MISOHIP_OK;
+  MISOHIP_TRY(launch_normalize(static_cast<hipStream_t>(stream), x, dt == MISOHIP_F64, n, width,
+                               mean, sd, out, bf16 != 0));
+  return MISOHIP_OK;
+}
+
 // residual indicator: flag columns whose network Q_rad (from Y) differs from
 // the plain-RT q_rt by more than tol in relative L2 over the column; corr
 // (optional) receives q_rt - network on every interior cell

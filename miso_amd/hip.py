@@ -14,6 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "lib", "libmisohip.so")
 
 F64, F32 = 0, 1
+MOMENT_SHARES = 64  # MISOHIP_MOMENT_SHARES
 
 FIELD_NAMES = ("ro", "vx", "vy", "vz", "bx", "by", "bz", "ei", "ph")
 
@@ -140,6 +141,10 @@ SIGNATURES = {
                              C.c_double, C.c_void_p, C.c_void_p],
     "misohip_mlp_qrad": [C.c_void_p, C.c_void_p, _P(MisohipGrid), C.c_void_p, C.c_void_p,
                          C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p],
+    "misohip_column_moments": [C.c_int, C.c_void_p, C.c_void_p, C.c_long, C.c_int, C.c_void_p,
+                               C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p],
+    "misohip_column_normalize": [C.c_int, C.c_void_p, C.c_long, C.c_int, C.c_void_p, C.c_void_p,
+                                 C.c_int, C.c_void_p, C.c_void_p],
     "misohip_mlp_residual": [C.c_void_p, C.c_void_p, _P(MisohipGrid), C.c_void_p, C.c_void_p,
                              C.c_void_p, C.c_double, C.c_void_p],
     "misohip_run": [C.c_void_p, _P(MisohipGrid), C.c_int, _P(MisohipParams), _P(MisohipBc),

@@ -33,6 +33,47 @@ def interior_columns(field, grid):
     return sub.permute(1, 2, 0).reshape(grid.i_size * grid.j_size, grid.k_size)
 
 
+def _rows(x):
+    """(N, W) as the column kernels read it: row-major, FP32 or FP64."""
+    import torch
+    if x.dtype not in (torch.float32, torch.float64):
+        x = x.double()
+    x = x.contiguous()
+    return x, hip.F64 if x.dtype == torch.float64 else hip.F32
+
+
+def _stream(x):
+    import torch
+    return C.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)
+
+
+def _moments(x, rows):
+    """FP64 mean, standard deviation (n - 1) and mean magnitude of x[rows] by
+    column."""
+    import torch
+    x, dt = _rows(x)
+    out = [torch.empty(x.shape[1], dtype=torch.float64, device=x.device) for _ in range(3)]
+    work = torch.empty(2 * hip.MOMENT_SHARES * x.shape[1], dtype=torch.float64, device=x.device)
+    with torch.cuda.device(x.device):
+        hip.call("misohip_column_moments", dt, C.c_void_p(x.data_ptr()),
+                 C.c_void_p(rows.data_ptr()), rows.shape[0], x.shape[1],
+                 *(C.c_void_p(t.data_ptr()) for t in out), C.c_void_p(work.data_ptr()),
+                 _stream(x))
+    return out
+
+
+def _normalized(x, mean, sd, dtype):
+    """(x - mean) / sd, formed in FP64, as bf16 or FP32."""
+    import torch
+    x, dt = _rows(x)
+    out = torch.empty(x.shape, dtype=dtype, device=x.device)
+    with torch.cuda.device(x.device):
+        hip.call("misohip_column_normalize", dt, C.c_void_p(x.data_ptr()), x.shape[0], x.shape[1],
+                 C.c_void_p(mean.data_ptr()), C.c_void_p(sd.data_ptr()),
+                 int(dtype == torch.bfloat16), C.c_void_p(out.data_ptr()), _stream(x))
+    return out
+
+
 class ColumnSurrogate:
     def __init__(self, ctx, nz: int, hidden: int = 256, hidden_layers: int = 3,
                  max_batch: int = 4096, seed: int = 0, device="cuda", features: int = 3):
@@ -136,17 +177,14 @@ class ColumnSurrogate:
         nval = max(batch, int(n * val_frac)) if n > 2 * batch else 0
         tr, va = perm[nval:], perm[:nval]
         ntr = (len(tr) // batch) * batch
-        f64 = feats[tr].double()
-        t64 = targets[tr].double()
-        mu_in = f64.mean(0)
-        sd_in = torch.maximum(f64.std(0), 1e-6 * f64.abs().mean(0)).clamp_min(1e-12)
-        mu_out = t64.mean(0)
-        sd_out = t64.std(0).clamp_min(1e-12)
+        mu_in, sd_in, mean_abs = _moments(feats, tr)
+        sd_in = torch.maximum(sd_in, 1e-6 * mean_abs).clamp_min(1e-12)
+        mu_out, sd_out, _ = _moments(targets, tr)
+        sd_out = sd_out.clamp_min(1e-12)
         self.set_normalization(mu_in.cpu().numpy(), sd_in.cpu().numpy(), mu_out.cpu().numpy(),
                                sd_out.cpu().numpy())
-        Xn = ((feats.double() - mu_in) / sd_in).to(torch.bfloat16)
-        Yn = ((targets.double() - mu_out) / sd_out).float()
-        del f64, t64
+        Xn = _normalized(feats, mu_in, sd_in, torch.bfloat16)
+        Yn = _normalized(targets, mu_out, sd_out, torch.float32)
         steps = epochs * (ntr // batch)
         k = 0
         last = 0.0

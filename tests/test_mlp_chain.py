@@ -129,3 +129,33 @@ def test_qrad_field_is_the_scaled_output(ctx, ni, nj, nz, n_hidden):
         want[inner] = ref
         assert torch.equal(q, want)
     net.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", ["float32", "float64"])
+@pytest.mark.parametrize("n,width,chosen", [(1, 4, 1), (7, 60, 3), (300, 64, 257), (5, 1536, 2),
+                                            (4100, 132, 4097)])
+def test_training_data_moments_and_scaling(dtype, n, width, chosen):
+    """Column moments of chosen rows and the scaled columns against torch in
+    64 bits; the scaled values are the same bits."""
+    import torch
+    from miso_amd import surrogate
+    g = torch.Generator().manual_seed(n)
+    x = (torch.randn((n, width), generator=g, dtype=torch.float64) * 0.1 - 1.0).to("cuda:0")
+    x = x.to(getattr(torch, dtype))
+    rows = torch.randperm(n, generator=g)[:chosen].to("cuda:0")
+    mean, sd, mean_abs = surrogate._moments(x, rows)
+    ref = x[rows].double()
+    eps = 2.0 ** -52 * chosen  # a sum's rounding, of values of magnitude one
+    assert (mean - ref.mean(0)).abs().max() <= eps
+    assert (mean_abs - ref.abs().mean(0)).abs().max() <= eps
+    if chosen > 1:
+        assert ((sd - ref.std(0)).abs() <= 1e3 * eps * ref.std(0)).all()
+    else:
+        assert torch.isnan(sd).all()
+    sd = sd.nan_to_num(nan=0.1).clamp_min(1e-12)
+    want = (x.double() - mean) / sd
+    assert torch.equal(surrogate._normalized(x, mean, sd, torch.bfloat16), want.to(torch.bfloat16))
+    assert torch.equal(surrogate._normalized(x, mean, sd, torch.float32), want.float())
+    odd = torch.cat([x[:1], x])[1:]  # rows from an odd offset on
+    assert torch.equal(surrogate._normalized(odd, mean, sd, torch.float32), want.float())
