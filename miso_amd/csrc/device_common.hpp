@@ -84,6 +84,15 @@ __device__ __forceinline__ R lane_dn(R v) {  // value of lane + 1
   return dpp_move<0x130>(v);
 }
 
+// A barrier for what a workgroup's waves exchange through LDS alone: global
+// loads and stores stay in flight across it (__syncthreads waits for all of
+// them).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Workgroups are dispatched round-robin over the 8 XCDs (linear block L runs
 // on XCD L % 8, and each XCD takes its blocks in increasing L).  Mapping L to
 // the virtual block V below gives every XCD one contiguous range of V, i.e. a

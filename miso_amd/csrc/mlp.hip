@@ -40,17 +40,14 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// A barrier for what the workgroup's waves exchange through LDS alone: global
-// loads and stores stay in flight across it (147456 columns of inference 635 ->
-// 622 us).  WIDE: they exchange through global memory too.
+// The waves of a workgroup exchange activations through LDS (147456 columns of
+// inference 635 -> 622 us with loads and stores in flight across it); WIDE:
+// through global memory.
 template <bool WIDE> __device__ __forceinline__ void chain_barrier() {
-  if (WIDE) {
+  if (WIDE)
     __syncthreads();
-    return;
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  else
+    lds_barrier();
 }
 
 // features of X that a workgroup of 64 columns takes at a time

@@ -208,7 +208,7 @@ __global__ __launch_bounds__(64 * W) void rt_sweep_tile_kernel(
   };
   auto exchange = [&](RtTilePlane<R> &x, int p) {
     edge[p & 1][w][lane] = x.i[R - 1];
-    __syncthreads();
+    lds_barrier();
     x.ih = edge[p & 1][w ? w - 1 : 0][lane];
   };
   RtTilePlane<R> x0, x1, x2;
@@ -253,8 +253,14 @@ __global__ __launch_bounds__(64 * W) void rt_sweep_tile_kernel(
   rt_block_max(best, part);
 }
 
-// rows a wave holds, in patches of RT_ROWS and of RT_ROWS_SMALL rows
-constexpr int RT_R = 4, RT_R_SMALL = 5;
+// Rows a wave holds, in patches of RT_ROWS and of RT_ROWS_SMALL rows.  Full
+// launches read least with four (two: radiative step of 256^3 15.8 -> 17.2 ms,
+// cold solve of 211 x 150 x 187 7.2 -> 7.9).  The short patches' launches leave
+// most of the chip idle and run at the length of a plane's FP64 chain: ten
+// waves of two rows instead of four of five hide more of it (slab solve of
+// 384^2 x 27 3.21 -> 3.01 ms; five of four, uneven over the SIMDs, 3.31; loads
+// two planes ahead 3.07).
+constexpr int RT_R = 4, RT_R_SMALL = 2;
 
 hipError_t launch_rt_sweep_tiles(hipStream_t st, double *I, const double *kap, const double *S,
                                  const double *kap_y, const double *S_y, const RtRays &rays,
