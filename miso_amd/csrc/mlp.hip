@@ -77,19 +77,20 @@ constexpr int MLP_X_TALL = 128;
 // batches of inference (NT = 2: 736 us for 635 at 147456 columns; four waves
 // of twice the row tiles 680; three row tiles a wave spill: 994; features of
 // X by 256, one workgroup a CU: 850).
-// At that size and a batch of 1024 a training step's chain takes 37 us, where
+// At that size and a batch of 1024 a training step's chain takes 34 us, where
 // a launch per layer, product and elementwise step (128 x 128 tiles: 16
 // workgroups) took 232; 147456 columns of inference, their Q_rad field
-// included, 622 us for 957 (without
+// included, 640 us for 957 (without
 // its 1.1 GB of Y, corrections and Q_rad it would take 363).  Every sum is
 // taken in the order of k, 32 at a time, as those took it: the same bits.
 template <int NT, int WAVES, int RT, int PD, bool TRAIN, bool WIDE>
 __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
-    const MlpLayer *__restrict__ L, int nl, const uint16_t *__restrict__ X, int M,
+    MlpNet net, const uint16_t *__restrict__ X, int M,
     float *__restrict__ Y, MlpLoss ls, MlpField fo, uint16_t *g0, uint16_t *g1, int bw, int xoff,
     int xw) {
   constexpr int NS = 16 * NT, NTHR = 64 * WAVES;
   static_assert(RT <= 3, "product()");
+  static_assert(NT > 1 || RT == 1, "one row tile a wave");
   static_assert(NT == 1 || !TRAIN, "the packed columns of a training tile are 16");
   extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -101,7 +102,7 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
   uint16_t *nxt = WIDE ? g0 + (long)s0 * pitch : lds;
   uint16_t *cur = WIDE ? g1 + (long)s0 * pitch : lds + NS * pitch;
   uint16_t *xbuf = lds + xoff;
-  const int n_in = L[0].in;
+  const int n_in = net.n_in, nl = net.nl;
 
   bf16x8 a[PD][RT];
   f32x4 acc[RT][NT];
@@ -190,23 +191,35 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
     for (int r = 0; r < cnt; ++r)
 #pragma unroll
       for (int n = 0; n < NT; ++n) acc[r][n] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    // k-steps k0 .. k0 + ke - 1, their B operand from `row` on
+    // K-steps k0 .. k0 + ke - 1, their B operand from `row` on.  Whole rounds
+    // of the PD k-steps in flight have no branch inside: past one the compiler
+    // would wait for all loads in flight at the start of every round (38 us a
+    // training step's chain for 34; with 8 in flight 35, with 2 37.5).
     auto steps = [&](const uint16_t *row, int rp, int k0, int ke) {
-      for (int k = 0; k < ke; k += PD) {
+      auto one = [&](int p, int k) {
+        bf16x8 bv[NT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+          bv[n] = *reinterpret_cast<const bf16x8 *>(row + n * rp + k * 32);
+#pragma unroll
+        for (int r = 0; r < cnt; ++r)
+#pragma unroll
+          for (int n = 0; n < NT; ++n) acc[r][n] = mfma(a[p][r], bv[n], acc[r][n]);
+      };
+      int k = 0;
+      for (; k + PD <= ke && k0 + k + PD < KT; k += PD) {
 #pragma unroll
         for (int p = 0; p < PD; ++p) {
-          if (k + p >= ke) break;
-          bf16x8 bv[NT];
+          one(p, k + p);
 #pragma unroll
-          for (int n = 0; n < NT; ++n)
-            bv[n] = *reinterpret_cast<const bf16x8 *>(row + n * rp + (k + p) * 32);
-#pragma unroll
-          for (int r = 0; r < cnt; ++r) {
-#pragma unroll
-            for (int n = 0; n < NT; ++n) acc[r][n] = mfma(a[p][r], bv[n], acc[r][n]);
+          for (int r = 0; r < cnt; ++r)
             a[p][r] = frag(wp, KT, tile[r], min(k0 + k + p + PD, KT - 1));
-          }
         }
+      }
+#pragma unroll
+      for (int p = 0; p < PD; ++p) {  // the last PD k-steps at most
+        if (k + p >= ke) break;
+        one(p, k + p);
       }
     };
     if (!input) {
@@ -224,7 +237,7 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
     } else {
       for (int k0 = 0; k0 < KT; k0 += xw >> 5) {
         const int cw = stage(k0 * 32);
-        if (TRAIN && keep) pack(xbuf, xpitch, cw, L[0].aT, k0 * 32);
+        if (TRAIN && keep) pack(xbuf, xpitch, cw, net.aT, k0 * 32);
         steps(xbuf + col * xpitch + kq * 8, 16 * xpitch, k0, cw >> 5);
       }
     }
@@ -244,7 +257,7 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
   // for possible aliases
   auto store_output = [&](int r, int o, f32x4 bias) {
     constexpr int H = NT < 2 ? NT : 2;
-    const int no = L[nl - 1].out, st = fo.sh.It * fo.sh.Jt;
+    const int no = net.n_out, st = fo.sh.It * fo.sh.Jt;
     f32x4 mu, sd;
     if (fo.qrad) {
       mu = *reinterpret_cast<const f32x4 *>(fo.mu + o);
@@ -287,12 +300,14 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
     }
   };
 
+  auto load4 = [](const float *q) { return *reinterpret_cast<const f32x4u *>(q); };
   // ---- forward
-  preload(L[0].wp, n_in / 32, L[0].out / 16, 0, tiles_of(L[0].out / 16));
+  preload(net.wp, n_in / 32, net.out(0) / 16, 0, tiles_of(net.out(0) / 16));
   for (int l = 0; l < nl; ++l) {
     const bool last = l == nl - 1;
-    const int KT = L[l].in / 32, OT = L[l].out / 16, cnt = tiles_of(OT);
-    const uint16_t *wp = L[l].wp;
+    const int KT = net.in(l) / 32, O = net.out(l), OT = O / 16, cnt = tiles_of(OT);
+    const uint16_t *wp = net.wp + net.w_at(l);
+    const float *b = net.b + net.b_at(l);
     for (int base = 0; base < OT; base += WAVES * cnt) {
       if (base) preload(wp, KT, OT, base, cnt);
       product(cnt, wp, KT, OT, base, cur, l == 0, base == 0);
@@ -301,77 +316,77 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
         const int tile = base + wave * cnt + r;
         if (r >= cnt || tile >= OT) break;
         const int o = tile * 16 + 4 * kq;
-        const f32x4 bias = *reinterpret_cast<const f32x4 *>(L[l].b + o);
+        const f32x4 bias = load4(b + o);
+        if (!TRAIN && last) {
+          store_output(r, o, bias);
+          continue;
+        }
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
-          const int sl = 16 * n + col, s = s0 + sl;
-          f32x4 x = acc[r][n] + bias;
-          if (!TRAIN && last) break;
+          const int sl = 16 * n + col;
+          const f32x4 x = acc[r][n] + bias;
+          f32x4 h;
           if (!last) {
             if (TRAIN)
-              *reinterpret_cast<f32x4 *>(L[l].pre + ((long)blockIdx.x * OT + tile) * 256 +
-                                         lane * 4) = x;
-            f32x4 h;
+              *reinterpret_cast<f32x4 *>(net.pre + net.d_at(l) +
+                                         ((long)blockIdx.x * OT + tile) * 256 + lane * 4) = x;
 #pragma unroll
             for (int v = 0; v < 4; ++v) h[v] = x[v] / (1.f + expf(-x[v]));
-            *reinterpret_cast<uint2 *>(nxt + sl * pitch + o) = f2bf4(h);
-          } else if (TRAIN) {
-            const f32x4 t = *reinterpret_cast<const f32x4u *>(ls.T + (long)s * L[l].out + o);
-            f32x4 g;
+          } else {
+            const f32x4 t = load4(ls.T + (long)(s0 + sl) * O + o);
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
               const float d = x[v] - t[v];
-              g[v] = 2.f * d * ls.scale;
+              h[v] = 2.f * d * ls.scale;
             }
-            *reinterpret_cast<uint2 *>(nxt + sl * pitch + o) = f2bf4(g);
-            if (Y) *reinterpret_cast<f32x4u *>(Y + (long)s * L[l].out + o) = x;
+            if (Y) *reinterpret_cast<f32x4u *>(Y + (long)(s0 + sl) * O + o) = x;
           }
+          *reinterpret_cast<uint2 *>(nxt + sl * pitch + o) = f2bf4(h);
         }
-        if (!TRAIN && last) store_output(r, o, bias);
       }
     }
     if (!last)
-      preload(L[l + 1].wp, L[l + 1].in / 32, L[l + 1].out / 16, 0, tiles_of(L[l + 1].out / 16));
-    else if (TRAIN && l > 0)
-      preload(L[l].wtp, L[l].out / 32, L[l].in / 16, 0, tiles_of(L[l].in / 16));
+      preload(net.wp + net.w_at(l + 1), O / 32, net.out(l + 1) / 16, 0,
+              tiles_of(net.out(l + 1) / 16));
+    else if (TRAIN)
+      preload(net.wtp + net.w_at(l), O / 32, net.in(l) / 16, 0, tiles_of(net.in(l) / 16));
     if (!last || TRAIN) {
       chain_barrier<WIDE>();
-      if (TRAIN) pack(nxt, pitch, L[l].out, last ? L[l].dT : L[l + 1].aT, 0);
-      uint16_t *t = cur;
+      if (TRAIN) pack(nxt, pitch, O, last ? net.dT + net.d_at(l) : net.aT + net.a_at(l + 1), 0);
+      uint16_t *swap = cur;
       cur = nxt;
-      nxt = t;
+      nxt = swap;
     }
   }
   if constexpr (TRAIN) {
     // ---- back: the gradient of layer l's input, times silu' of layer l - 1
     for (int l = nl - 1; l > 0; --l) {
-      const int KT = L[l].out / 32, OT = L[l].in / 16, cnt = tiles_of(OT);
-      const uint16_t *wp = L[l].wtp;
+      const int KT = net.out(l) / 32, I = net.in(l), OT = I / 16, cnt = tiles_of(OT);
+      const uint16_t *wp = net.wtp + net.w_at(l);
       for (int base = 0; base < OT; base += WAVES * cnt) {
         if (base) preload(wp, KT, OT, base, cnt);
         product(cnt, wp, KT, OT, base, cur, false, false);
-#pragma unroll
-        for (int r = 0; r < RT; ++r) {
-          const int tile = base + wave * cnt + r;
-          if (r >= cnt || tile >= OT) break;
+        const int tile = base + wave;
+        if (tile < OT) {
           const f32x4 x = *reinterpret_cast<const f32x4 *>(
-              L[l - 1].pre + ((long)blockIdx.x * OT + tile) * 256 + lane * 4);
+              net.pre + net.d_at(l - 1) + ((long)blockIdx.x * OT + tile) * 256 + lane * 4);
           f32x4 g;
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
             const float sg = 1.f / (1.f + expf(-x[v]));
-            g[v] = acc[r][0][v] * sg * (1.f + x[v] * (1.f - sg));
+            g[v] = acc[0][0][v] * sg * (1.f + x[v] * (1.f - sg));
           }
           *reinterpret_cast<uint2 *>(nxt + col * pitch + tile * 16 + 4 * kq) = f2bf4(g);
         }
       }
       if (l > 1)
-        preload(L[l - 1].wtp, L[l - 1].out / 32, L[l - 1].in / 16, 0, tiles_of(L[l - 1].in / 16));
+        preload(net.wtp + net.w_at(l - 1), I / 32, net.in(l - 1) / 16, 0,
+                tiles_of(net.in(l - 1) / 16));
       chain_barrier<WIDE>();
-      pack(nxt, pitch, L[l].in, L[l - 1].dT, 0);
-      uint16_t *t = cur;
+      pack(nxt, pitch, I, net.dT + net.d_at(l - 1), 0);
+      uint16_t *swap = cur;
       cur = nxt;
-      nxt = t;
+      nxt = swap;
     }
   }
 }
@@ -383,18 +398,19 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
 // additions grows with the batch, and these sums are added in order; a bias
 // is 16 sums, of every 16th column each, added in order.
 // Bound by the operands' way from L2 (64 bytes a clock and CU): 80 MB at a
-// batch of 1024 and 1536-256-256-256-384: 10.5 us, where a launch per layer
+// batch of 1024 and 1536-256-256-256-384: 8.2 us, where a launch per layer
 // that transposed through LDS, its partial sums in memory and column sums by
 // four workgroups took 134.
-__global__ __launch_bounds__(64) void mlp_wgrad_kernel(const MlpLayer *__restrict__ L, int nl,
-                                                       int SB, int per, int tiles) {
+__global__ __launch_bounds__(64) void mlp_wgrad_kernel(MlpNet net, int SB, int per,
+                                                       int tiles) {
   const int lane = threadIdx.x, row = lane & 15, kq = lane >> 4;
-  int blk = blockIdx.x, l = 0;
+  int blk = blockIdx.x;
   if (blk >= tiles) {  // lane: bias o, octets of columns of one parity
     blk -= tiles;
-    while (blk >= L[l].out / 32) blk -= L[l++].out / 32;
+    const int l = min(blk / (net.n_hidden / 32), net.nl - 1);
+    blk -= l * (net.n_hidden / 32);
     const int o = lane & 31, par = lane >> 5;
-    const uint16_t *d = L[l].dT + ((long)(2 * blk + (o >> 4)) * SB * 64 + (o & 15)) * 8;
+    const uint16_t *d = net.dT + net.d_at(l) + ((long)(2 * blk + (o >> 4)) * SB * 64 + (o & 15)) * 8;
     float s[8] = {};
 #pragma unroll 8
     for (int q = par; q < 4 * SB; q += 2) {
@@ -409,17 +425,16 @@ __global__ __launch_bounds__(64) void mlp_wgrad_kernel(const MlpLayer *__restric
     for (int e = 1; e < 8; ++e) t += s[e];
 #pragma unroll
     for (int e = 0; e < 8; ++e) t += __shfl(s[e], lane | 32, 64);
-    if (par == 0) L[l].gb[32 * blk + o] = t;
+    if (par == 0) net.gb[net.b_at(l) + 32 * blk + o] = t;
     return;
   }
-  while (l + 1 < nl && blk >= L[l + 1].tile0) ++l;
-  const int I = L[l].in, nti = I / 32;
-  const int t = blk - L[l].tile0, to = t / nti, ti = t - to * nti;
+  const int l = net.layer_of(blk), I = net.in(l), nti = I / 32;
+  const int t = blk - net.tile_at(l), to = t / nti, ti = t - to * nti;
   const uint16_t *pa[2], *pb[2];
 #pragma unroll
   for (int x = 0; x < 2; ++x) {
-    pa[x] = L[l].dT + (long)(to * 2 + x) * SB * 512 + lane * 8;
-    pb[x] = L[l].aT + (long)(ti * 2 + x) * SB * 512 + lane * 8;
+    pa[x] = net.dT + net.d_at(l) + (long)(to * 2 + x) * SB * 512 + lane * 8;
+    pb[x] = net.aT + net.a_at(l) + (long)(ti * 2 + x) * SB * 512 + lane * 8;
   }
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   f32x4 acc[2][2], sum[2][2];
@@ -440,32 +455,40 @@ __global__ __launch_bounds__(64) void mlp_wgrad_kernel(const MlpLayer *__restric
 #pragma unroll
   for (int p = 0; p < PD; ++p) load(p, p);
   int c = 0;
-  for (int s = 0; s < SB; s += PD)
+  auto one = [&](int p) {
 #pragma unroll
-    for (int p = 0; p < PD; ++p) {
-      if (s + p >= SB) break;
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y) acc[x][y] = mfma(a[p][x], b[p][y], acc[x][y]);
+    if (++c == per && per < SB) {
+      c = 0;
 #pragma unroll
       for (int x = 0; x < 2; ++x)
 #pragma unroll
-        for (int y = 0; y < 2; ++y) acc[x][y] = mfma(a[p][x], b[p][y], acc[x][y]);
-      load(p, s + p + PD);
-      if (++c == per && per < SB) {
-        c = 0;
-#pragma unroll
-        for (int x = 0; x < 2; ++x)
-#pragma unroll
-          for (int y = 0; y < 2; ++y) {
-            sum[x][y] += acc[x][y];
-            acc[x][y] = zero;
-          }
-      }
+        for (int y = 0; y < 2; ++y) {
+          sum[x][y] += acc[x][y];
+          acc[x][y] = zero;
+        }
     }
+  };
+  int s = 0;
+  for (; s + PD < SB; s += PD)  // no branch past a load: see the chain's steps
+#pragma unroll
+    for (int p = 0; p < PD; ++p) {
+      one(p);
+      load(p, s + p + PD);
+    }
+#pragma unroll
+  for (int p = 0; p < PD; ++p) {
+    if (s + p >= SB) break;
+    one(p);
+  }
 #pragma unroll
   for (int x = 0; x < 2; ++x)
 #pragma unroll
     for (int y = 0; y < 2; ++y) {
       const f32x4 g = per < SB ? sum[x][y] : acc[x][y];
-      float *gw = L[l].gw + (long)(to * 32 + x * 16 + 4 * kq) * I + ti * 32 + y * 16 + row;
+      float *gw = net.gw + net.w_at(l) + (long)(to * 32 + x * 16 + 4 * kq) * I + ti * 32 + y * 16 + row;
 #pragma unroll
       for (int v = 0; v < 4; ++v) gw[(long)v * I] = g[v];
     }
@@ -506,40 +529,37 @@ __device__ __forceinline__ float adam_step(float &w, float g, float &m1, float &
 // Bound by HBM or the last-level cache, 32 bytes a weight: 6.2 us for 622592
 // weights (28 as eight launches).
 template <bool UPDATE>
-__global__ __launch_bounds__(256) void mlp_adam_kernel(const MlpLayer *__restrict__ L, int nl,
-                                                       int l0, MlpAdam p) {
+__global__ __launch_bounds__(256) void mlp_adam_kernel(MlpNet net, int l0, MlpAdam p) {
   __shared__ __attribute__((aligned(16))) uint16_t tile[32][40];
-  const int blk = blockIdx.x + L[l0].tile0;
-  int l = l0;
-  while (l + 1 < nl && blk >= L[l + 1].tile0) ++l;
-  const int I = L[l].in, O = L[l].out, nti = I / 32;
-  const int t = blk - L[l].tile0, to = t / nti, ti = t - to * nti;
+  const int blk = blockIdx.x + net.tile_at(l0), l = net.layer_of(blk);
+  const int I = net.in(l), O = net.out(l), nti = I / 32;
+  const int t = blk - net.tile_at(l), to = t / nti, ti = t - to * nti;
   const int tid = threadIdx.x, r = tid >> 3, c = 4 * (tid & 7);
-  const long at = (long)(to * 32 + r) * I + ti * 32 + c;
-  f32x4 w = *reinterpret_cast<const f32x4 *>(L[l].w + at);
+  const long at = net.w_at(l) + (long)(to * 32 + r) * I + ti * 32 + c;
+  f32x4 w = *reinterpret_cast<const f32x4 *>(net.w + at);
   if (UPDATE) {
-    const f32x4 g = *reinterpret_cast<const f32x4 *>(L[l].gw + at);
-    f32x4 m1 = *reinterpret_cast<const f32x4 *>(L[l].mw + at);
-    f32x4 m2 = *reinterpret_cast<const f32x4 *>(L[l].vw + at);
+    const f32x4 g = *reinterpret_cast<const f32x4 *>(net.gw + at);
+    f32x4 m1 = *reinterpret_cast<const f32x4 *>(net.mw + at);
+    f32x4 m2 = *reinterpret_cast<const f32x4 *>(net.vw + at);
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       float x = w[v], y = m1[v], z = m2[v];
       adam_step(x, g[v], y, z, p, p.wd);
       w[v] = x; m1[v] = y; m2[v] = z;
     }
-    *reinterpret_cast<f32x4 *>(L[l].w + at) = w;
-    *reinterpret_cast<f32x4 *>(L[l].mw + at) = m1;
-    *reinterpret_cast<f32x4 *>(L[l].vw + at) = m2;
+    *reinterpret_cast<f32x4 *>(net.w + at) = w;
+    *reinterpret_cast<f32x4 *>(net.mw + at) = m1;
+    *reinterpret_cast<f32x4 *>(net.vw + at) = m2;
     if (ti == 0 && tid < 32) {
-      const int o = to * 32 + tid;
-      adam_step(L[l].b[o], L[l].gb[o], L[l].mb[o], L[l].vb[o], p, 0.f);
+      const long o = net.b_at(l) + to * 32 + tid;
+      adam_step(net.b[o], net.gb[o], net.mb[o], net.vb[o], p, 0.f);
     }
   }
   *reinterpret_cast<uint2 *>(&tile[r][c]) = f2bf4(w);
   __syncthreads();
   const int lane = tid & 63, row = lane & 15, k = 8 * (lane >> 4), h = (tid >> 6) & 1;
   if (tid < 128) {
-    *reinterpret_cast<uint4 *>(L[l].wp + ((long)(to * 2 + h) * nti + ti) * 512 + lane * 8) =
+    *reinterpret_cast<uint4 *>(net.wp + net.w_at(l) + ((long)(to * 2 + h) * nti + ti) * 512 + lane * 8) =
         *reinterpret_cast<const uint4 *>(&tile[16 * h + row][k]);
   } else {
     uint32_t v[4];
@@ -547,7 +567,7 @@ __global__ __launch_bounds__(256) void mlp_adam_kernel(const MlpLayer *__restric
     for (int e = 0; e < 4; ++e)
       v[e] = (uint32_t)tile[k + 2 * e][16 * h + row] |
              (uint32_t)tile[k + 2 * e + 1][16 * h + row] << 16;
-    *reinterpret_cast<uint4 *>(L[l].wtp + ((long)(ti * 2 + h) * (O / 32) + to) * 512 + lane * 8) =
+    *reinterpret_cast<uint4 *>(net.wtp + net.w_at(l) + ((long)(ti * 2 + h) * (O / 32) + to) * 512 + lane * 8) =
         make_uint4(v[0], v[1], v[2], v[3]);
   }
 }
@@ -765,7 +785,7 @@ size_t chain_lds(int ns, int bw, int xw) {
 }
 
 template <int NT, int WAVES, int RT, int PD, bool TRAIN, bool WIDE>
-hipError_t chain(hipStream_t st, const MlpLayer *L, int nl, const uint16_t *X, int M, float *Y,
+hipError_t chain(hipStream_t st, const MlpNet &net, const uint16_t *X, int M, float *Y,
                  const MlpLoss &ls, const MlpField &fo, uint16_t *g0, uint16_t *g1, int bw,
                  int xoff, int xw, size_t bytes) {
   auto k = mlp_chain_kernel<NT, WAVES, RT, PD, TRAIN, WIDE>;
@@ -774,7 +794,7 @@ hipError_t chain(hipStream_t st, const MlpLayer *L, int nl, const uint16_t *X, i
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(k, dim3((M + 16 * NT - 1) / (16 * NT)), dim3(64 * WAVES), bytes, st, L, nl,
+  hipLaunchKernelGGL(k, dim3((M + 16 * NT - 1) / (16 * NT)), dim3(64 * WAVES), bytes, st, net,
                      X, M, Y, ls, fo, g0, g1, bw, xoff, xw);
   return hipGetLastError();
 }
@@ -785,9 +805,10 @@ bool mlp_is_wide(int n_in, int maxw) {
   return chain_lds(16, maxw, x_width(n_in)) + 1024 > (size_t)LDS_BYTES;
 }
 
-hipError_t launch_mlp_forward(hipStream_t st, const MlpLayer *L, int nl, int n_in, int n_hidden,
-                              bool wide, int maxw, const uint16_t *X, int M, float *Y,
-                              const MlpField &fo, uint16_t *g0, uint16_t *g1) {
+hipError_t launch_mlp_forward(hipStream_t st, const MlpNet &net, bool wide, int maxw,
+                              const uint16_t *X, int M, float *Y, const MlpField &fo,
+                              uint16_t *g0, uint16_t *g1) {
+  const int n_in = net.n_in, n_hidden = net.n_hidden;
   const MlpLoss none{};
   // X passes through the place of the second buffer, two chunks of it (the
   // input layer writes the first buffer)
@@ -795,31 +816,31 @@ hipError_t launch_mlp_forward(hipStream_t st, const MlpLayer *L, int nl, int n_i
   const size_t tall = sizeof(uint16_t) * NS *
                       (n_hidden + 8 + std::max(n_hidden + 8, 2 * (MLP_X_TALL + 8)));
   if (M >= MLP_TALL && tall <= (size_t)LDS_BYTES)
-    return chain<NT, 8, 2, 2, false, false>(st, L, nl, X, M, Y, none, fo, g0, g1, n_hidden,
+    return chain<NT, 8, 2, 2, false, false>(st, net, X, M, Y, none, fo, g0, g1, n_hidden,
                                             NS * (n_hidden + 8), MLP_X_TALL, tall);
   const int xw = x_width(n_in);
   if (wide)
-    return chain<1, 16, 1, 8, false, true>(st, L, nl, X, M, Y, none, fo, g0, g1, maxw, 0, xw,
+    return chain<1, 16, 1, 4, false, true>(st, net, X, M, Y, none, fo, g0, g1, maxw, 0, xw,
                                            chain_lds(16, 0, xw));
-  return chain<1, 16, 1, 8, false, false>(st, L, nl, X, M, Y, none, fo, g0, g1, maxw,
+  return chain<1, 16, 1, 4, false, false>(st, net, X, M, Y, none, fo, g0, g1, maxw,
                                           32 * (maxw + 8), xw, chain_lds(16, maxw, xw));
 }
 
-hipError_t launch_mlp_grad(hipStream_t st, const MlpLayer *L, int nl, int n_in, bool wide,
-                           int maxw, int tiles, int bias_tiles, const uint16_t *X, int M,
-                           const MlpLoss &ls, float *Y, uint16_t *g0, uint16_t *g1) {
+hipError_t launch_mlp_grad(hipStream_t st, const MlpNet &net, bool wide, int maxw,
+                           const uint16_t *X, int M, const MlpLoss &ls, float *Y, uint16_t *g0,
+                           uint16_t *g1) {
   const MlpField none{};
-  const int xw = x_width(n_in);
+  const int xw = x_width(net.n_in);
   hipError_t e =
-      wide ? chain<1, 16, 1, 8, true, true>(st, L, nl, X, M, Y, ls, none, g0, g1, maxw, 0, xw,
+      wide ? chain<1, 16, 1, 4, true, true>(st, net, X, M, Y, ls, none, g0, g1, maxw, 0, xw,
                                             chain_lds(16, 0, xw))
-           : chain<1, 16, 1, 8, true, false>(st, L, nl, X, M, Y, ls, none, g0, g1, maxw,
+           : chain<1, 16, 1, 4, true, false>(st, net, X, M, Y, ls, none, g0, g1, maxw,
                                              32 * (maxw + 8), xw, chain_lds(16, maxw, xw));
   if (e != hipSuccess) return e;
   int splits = 16;  // equal sums of whole k-steps
   while (M % (32 * splits)) --splits;
-  hipLaunchKernelGGL(mlp_wgrad_kernel, dim3(tiles + bias_tiles), dim3(64), 0, st, L, nl, M / 32,
-                     M / 32 / splits, tiles);
+  hipLaunchKernelGGL(mlp_wgrad_kernel, dim3(net.tiles() + net.bias_tiles()), dim3(64), 0, st,
+                     net, M / 32, M / 32 / splits, net.tiles());
   return hipGetLastError();
 }
 
@@ -830,14 +851,14 @@ hipError_t launch_mlp_loss(hipStream_t st, const float *Y, const float *T, float
   return hipGetLastError();
 }
 
-hipError_t launch_mlp_adam(hipStream_t st, const MlpLayer *L, int nl, int tiles,
-                           const MlpAdam &p) {
-  hipLaunchKernelGGL((mlp_adam_kernel<true>), dim3(tiles), dim3(256), 0, st, L, nl, 0, p);
+hipError_t launch_mlp_adam(hipStream_t st, const MlpNet &net, const MlpAdam &p) {
+  hipLaunchKernelGGL((mlp_adam_kernel<true>), dim3(net.tiles()), dim3(256), 0, st, net, 0, p);
   return hipGetLastError();
 }
 
-hipError_t launch_mlp_pack(hipStream_t st, const MlpLayer *L, int nl, int layer, int tiles) {
-  hipLaunchKernelGGL((mlp_adam_kernel<false>), dim3(tiles), dim3(256), 0, st, L, nl, layer,
+hipError_t launch_mlp_pack(hipStream_t st, const MlpNet &net, int layer) {
+  const int tiles = net.in(layer) / 32 * (net.out(layer) / 32);
+  hipLaunchKernelGGL((mlp_adam_kernel<false>), dim3(tiles), dim3(256), 0, st, net, layer,
                      MlpAdam{});
   return hipGetLastError();
 }

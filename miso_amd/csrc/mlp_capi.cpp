@@ -16,10 +16,8 @@ struct misohip_mlp {
   int max_batch;
   int maxw;    // the widest activation
   bool wide;   // activations in g0, g1 instead of LDS
-  int tiles, bias_tiles;
   long t;  // Adam step
-  std::vector<MlpLayer> layer;
-  MlpLayer *d_layer = nullptr;   // the same, on the device
+  MlpNet net;
   uint16_t *g0 = nullptr, *g1 = nullptr;
   float *y = nullptr;            // the network's output where the loss is asked for
   float *loss_part = nullptr;
@@ -42,8 +40,8 @@ template <typename T> hipError_t alloc(misohip_mlp *m, T **p, size_t n) {
 
 int forward(misohip_ctx *ctx, misohip_mlp *m, const uint16_t *X, int batch, float *Y,
             const MlpField &field) {
-  MISOHIP_TRY(launch_mlp_forward(ctx->stream, m->d_layer, m->n_layers, m->n_in, m->n_hidden,
-                                 m->wide, m->maxw, X, batch, Y, field, m->g0, m->g1));
+  MISOHIP_TRY(launch_mlp_forward(ctx->stream, m->net, m->wide, m->maxw, X, batch, Y, field, m->g0,
+                                 m->g1));
   return MISOHIP_OK;
 }
 
@@ -82,34 +80,25 @@ int misohip_mlp_create(misohip_ctx *ctx, int n_in, int n_hidden, int n_hidden_la
   m->t = 0;
   m->maxw = n_hidden > n_out ? n_hidden : n_out;
   m->wide = mlp_is_wide(n_in, m->maxw);
-  m->tiles = m->bias_tiles = 0;
   hipError_t e = hipSuccess;
-  for (int l = 0; l < m->n_layers && e == hipSuccess; ++l) {
-    const bool last = l == m->n_layers - 1;
-    const int I = l == 0 ? n_in : n_hidden;
-    const int O = last ? n_out : n_hidden;
-    const size_t nw = (size_t)O * I;
-    MlpLayer y{};
-    y.in = I;
-    y.out = O;
-    y.tile0 = m->tiles;
-    m->tiles += (O / 32) * (I / 32);
-    m->bias_tiles += O / 32;
-    for (float **p : {&y.w, &y.gw, &y.mw, &y.vw})
-      if (e == hipSuccess) e = alloc(m, p, nw);
-    for (float **p : {&y.b, &y.gb, &y.mb, &y.vb})
-      if (e == hipSuccess) e = alloc(m, p, O);
-    for (uint16_t **p : {&y.wp, &y.wtp})
-      if (e == hipSuccess) e = alloc(m, p, nw);
-    if (e == hipSuccess && !last) e = alloc(m, &y.pre, (size_t)max_batch * O);
-    if (e == hipSuccess) e = alloc(m, &y.aT, (size_t)max_batch * I);
-    if (e == hipSuccess) e = alloc(m, &y.dT, (size_t)max_batch * O);
-    m->layer.push_back(y);
-  }
-  if (e == hipSuccess) e = alloc(m, &m->d_layer, m->layer.size());
+  MlpNet &net = m->net;
+  net.n_in = n_in;
+  net.n_hidden = n_hidden;
+  net.n_out = n_out;
+  net.nl = m->n_layers;
+  net.rows = max_batch;
+  const size_t nw = (size_t)net.w_at(m->n_layers - 1) + (size_t)n_hidden * n_out;
+  const size_t nb = (size_t)net.b_at(m->n_layers - 1) + n_out;
+  for (float **p : {&net.w, &net.gw, &net.mw, &net.vw})
+    if (e == hipSuccess) e = alloc(m, p, nw);
+  for (float **p : {&net.b, &net.gb, &net.mb, &net.vb})
+    if (e == hipSuccess) e = alloc(m, p, nb);
+  for (uint16_t **p : {&net.wp, &net.wtp})
+    if (e == hipSuccess) e = alloc(m, p, nw);
+  if (e == hipSuccess) e = alloc(m, &net.pre, (size_t)net.d_at(m->n_layers - 1));
+  if (e == hipSuccess) e = alloc(m, &net.aT, (size_t)net.a_at(m->n_layers));
   if (e == hipSuccess)
-    e = hipMemcpy(m->d_layer, m->layer.data(), sizeof(MlpLayer) * m->layer.size(),
-                  hipMemcpyHostToDevice);
+    e = alloc(m, &net.dT, (size_t)net.d_at(m->n_layers - 1) + (size_t)max_batch * n_out);
   if (m->wide) {
     if (e == hipSuccess) e = alloc(m, &m->g0, (size_t)max_batch * (m->maxw + 8));
     if (e == hipSuccess) e = alloc(m, &m->g1, (size_t)max_batch * (m->maxw + 8));
@@ -144,15 +133,16 @@ int misohip_mlp_set_layer(misohip_ctx *ctx, misohip_mlp *m, int layer, const flo
                           const float *b_host) {
   if (!ctx || !m || layer < 0 || layer >= m->n_layers || !w_host || !b_host) return MISOHIP_E_ARG;
   MISOHIP_TRY(hipSetDevice(ctx->device));
-  const MlpLayer &y = m->layer[layer];
-  const size_t nw = (size_t)y.out * y.in;
-  MISOHIP_TRY(hipMemcpy(y.w, w_host, sizeof(float) * nw, hipMemcpyHostToDevice));
-  MISOHIP_TRY(hipMemcpy(y.b, b_host, sizeof(float) * y.out, hipMemcpyHostToDevice));
-  MISOHIP_TRY(launch_mlp_pack(ctx->stream, m->d_layer, m->n_layers, layer, (int)(nw / 1024)));
-  MISOHIP_TRY(hipMemsetAsync(y.mw, 0, sizeof(float) * nw, ctx->stream));
-  MISOHIP_TRY(hipMemsetAsync(y.vw, 0, sizeof(float) * nw, ctx->stream));
-  MISOHIP_TRY(hipMemsetAsync(y.mb, 0, sizeof(float) * y.out, ctx->stream));
-  MISOHIP_TRY(hipMemsetAsync(y.vb, 0, sizeof(float) * y.out, ctx->stream));
+  const MlpNet &y = m->net;
+  const long w0 = y.w_at(layer), b0 = y.b_at(layer);
+  const size_t nw = sizeof(float) * y.out(layer) * y.in(layer), nb = sizeof(float) * y.out(layer);
+  MISOHIP_TRY(hipMemcpy(y.w + w0, w_host, nw, hipMemcpyHostToDevice));
+  MISOHIP_TRY(hipMemcpy(y.b + b0, b_host, nb, hipMemcpyHostToDevice));
+  MISOHIP_TRY(launch_mlp_pack(ctx->stream, y, layer));
+  MISOHIP_TRY(hipMemsetAsync(y.mw + w0, 0, nw, ctx->stream));
+  MISOHIP_TRY(hipMemsetAsync(y.vw + w0, 0, nw, ctx->stream));
+  MISOHIP_TRY(hipMemsetAsync(y.mb + b0, 0, nb, ctx->stream));
+  MISOHIP_TRY(hipMemsetAsync(y.vb + b0, 0, nb, ctx->stream));
   MISOHIP_TRY(hipStreamSynchronize(ctx->stream));
   m->t = 0;
   return MISOHIP_OK;
@@ -164,10 +154,11 @@ int misohip_mlp_get_layer(misohip_ctx *ctx, misohip_mlp *m, int layer, int which
     return MISOHIP_E_ARG;
   MISOHIP_TRY(hipSetDevice(ctx->device));
   MISOHIP_TRY(hipStreamSynchronize(ctx->stream));
-  const MlpLayer &y = m->layer[layer];
-  const size_t nw = (size_t)y.out * y.in;
-  const float *src = which == 0 ? y.w : which == 1 ? y.b : which == 2 ? y.gw : y.gb;
-  const size_t n = (which == 0 || which == 2) ? nw : (size_t)y.out;
+  const MlpNet &y = m->net;
+  const bool bias = which == 1 || which == 3;
+  const float *src = (which == 0 ? y.w : which == 1 ? y.b : which == 2 ? y.gw : y.gb) +
+                     (bias ? y.b_at(layer) : y.w_at(layer));
+  const size_t n = bias ? (size_t)y.out(layer) : (size_t)y.out(layer) * y.in(layer);
   MISOHIP_TRY(hipMemcpy(host, src, sizeof(float) * n, hipMemcpyDeviceToHost));
   return MISOHIP_OK;
 }
@@ -204,9 +195,9 @@ int misohip_mlp_grad(misohip_ctx *ctx, misohip_mlp *m, const void *X, const floa
     MlpLoss ls;
     ls.T = T;
     ls.scale = 1.f / (float)n;
-    MISOHIP_TRY(launch_mlp_grad(ctx->stream, m->d_layer, m->n_layers, m->n_in, m->wide, m->maxw,
-                                m->tiles, m->bias_tiles, static_cast<const uint16_t *>(X), batch,
-                                ls, loss ? m->y : nullptr, m->g0, m->g1));
+    MISOHIP_TRY(launch_mlp_grad(ctx->stream, m->net, m->wide, m->maxw,
+                                static_cast<const uint16_t *>(X), batch, ls,
+                                loss ? m->y : nullptr, m->g0, m->g1));
     int nb = 0;
     if (loss) MISOHIP_TRY(launch_mlp_loss(ctx->stream, m->y, T, m->loss_part, n, &nb));
     if (loss) {
@@ -230,7 +221,7 @@ int misohip_mlp_adam(misohip_ctx *ctx, misohip_mlp *m, float lr, float beta1, fl
   m->t += 1;
   const float c1 = 1.f - std::pow(beta1, (float)m->t), c2 = 1.f - std::pow(beta2, (float)m->t);
   const MlpAdam p = {lr, beta1, beta2, eps, c1, c2, weight_decay};
-  MISOHIP_TRY(launch_mlp_adam(ctx->stream, m->d_layer, m->n_layers, m->tiles, p));
+  MISOHIP_TRY(launch_mlp_adam(ctx->stream, m->net, p));
   return MISOHIP_OK;
 }
 
