@@ -459,28 +459,43 @@ __global__ __launch_bounds__(256) void rt_transpose_xy_kernel(const double *__re
 // Every ray's field x-fastest (blockIdx.z = ray): 32 x 32 tiles of a plane,
 // through LDS where the ray is kept y-fastest.  Bound by HBM (each value read
 // and written once); a clone followed by a transpose of each y-fastest ray
-// wrote those rays twice.
+// wrote those rays twice.  The others are copied 16 bytes a lane (by eights,
+// through the same tiles: cold solve of 211 x 150 x 187 7.27 ms for 7.10, slab
+// solve of 384^2 x 27 3.02 for 2.96).
 __global__ __launch_bounds__(256) void rt_xfast_kernel(const double *__restrict__ I,
                                                        double *__restrict__ out, int It, int Jt,
                                                        int tiles_i, unsigned tr, long ray_stride) {
   __shared__ double tile[32][33];
   const int ti = blockIdx.x % tiles_i, tj = blockIdx.x / tiles_i, l = threadIdx.x & 31;
   const long plane = ray_stride * blockIdx.z + (long)It * Jt * blockIdx.y;
-  const bool y = (tr >> blockIdx.z) & 1u;  // uniform over the block
-  if (y) {
-    for (int r = threadIdx.x >> 5; r < 32; r += 8) {
-      const int j = tj * 32 + l, i = ti * 32 + r;
-      if (i < It && j < Jt) tile[r][l] = I[plane + (long)i * Jt + j];
+  if (!((tr >> blockIdx.z) & 1u)) {  // uniform over the block: a copy, 1024 values a block
+    typedef double d2 __attribute__((ext_vector_type(2), aligned(8)));
+    const int n = It * Jt, c0 = blockIdx.x * 1024 + 2 * threadIdx.x;
+    const double *src = I + plane + c0;
+    double *dst = out + plane + c0;
+    if (c0 + 513 < n) {
+      const d2 a = *reinterpret_cast<const d2 *>(src), b = *reinterpret_cast<const d2 *>(src + 512);
+      *reinterpret_cast<d2 *>(dst) = a;
+      *reinterpret_cast<d2 *>(dst + 512) = b;
+    } else {
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const int q = (m & 1) + 512 * (m >> 1);
+        if (c0 + q < n) dst[q] = src[q];
+      }
     }
-    __syncthreads();
+    return;
   }
 #pragma unroll
   for (int m = 0; m < 4; ++m) {
+    const int r = (threadIdx.x >> 5) + 8 * m, j = tj * 32 + l, i = ti * 32 + r;
+    if (i < It && j < Jt) tile[r][l] = I[plane + (long)i * Jt + j];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
     const int r = (threadIdx.x >> 5) + 8 * m, i = ti * 32 + l, j = tj * 32 + r;
-    if (i < It && j < Jt) {
-      const long c = plane + (long)j * It + i;
-      out[c] = y ? tile[l][r] : I[c];
-    }
+    if (i < It && j < Jt) out[plane + (long)j * It + i] = tile[l][r];
   }
 }
 
