@@ -210,9 +210,12 @@ __device__ __forceinline__ int batch_find(const int *__restrict__ start, int n, 
 // per block (batch_rk_ywalk_kernel; the batch's block counts use these).
 constexpr int RK_YWALK_OUT = 60;
 constexpr int RK_YWALK_ROWS = 16;
-// a single x-y run walks y only when that makes at least this many waves
-// (eight per CU); smaller runs keep the one-plane kernel
-constexpr int RK_YWALK_MIN_WAVES = 2048;
+// A single x-y run walks y only when that makes at least this many waves, about
+// 2000^2: the one-plane kernel reads every cell at all its stencil points, and
+// is the faster one while the run's fields come from the last-level cache (FP32
+// stage of 1600 x 1500 66 us, the walk 79; FP64 of 1600 x 1590 170 and 174;
+// 2400^2 203 and 171, 363 and 348; 4096^2 599 and 446, 1079 and 976).
+constexpr int RK_YWALK_MIN_WAVES = 4096;
 
 template <typename R>
 hipError_t launch_batch_rk(hipStream_t, const BatchInst<R> *, const BatchDyn<R> *, const int *,

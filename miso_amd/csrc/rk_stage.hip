@@ -929,8 +929,8 @@ static hipError_t launch_rk_t(hipStream_t st, const Fld<const R> &o, const Fld<c
   const long yw_waves = (long)((ni + RK_YWALK_OUT - 1) / RK_YWALK_OUT) *
                         ((nj + RK_YWALK_ROWS - 1) / RK_YWALK_ROWS);
   if (HX && HY && !HZ && sc.variant >= 4 && sc.variant <= 6 && yw_waves >= RK_YWALK_MIN_WAVES) {
-    // an x-y run large enough to fill the chip with y-walk waves (a smaller
-    // one runs the one-plane kernel below: 256^2 is 80 waves)
+    // an x-y run too large for the last-level cache (a smaller one runs the
+    // one-plane kernel below)
     if (sh.mi < 2 || sh.mj < 2) return hipErrorInvalidValue;
     const long nb = (yw_waves + 3) / 4;
     if (nb > 2147483647L) return hipErrorInvalidValue;

@@ -49,3 +49,31 @@ def test_3d_runs_in_the_shortest_chunks(ctx, sizes, periodic):
     assert np.array_equal(dts, ref_dts), (dts, ref_dts)
     sl = (slice(None),) + (slice(2, -2),) * 3  # the oracle's 3D edges keep what was there
     assert_bitwise(out[sl], ref[sl], f"{sizes} {periodic}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("sizes", [(61, 32790, 1), (61, 32700, 1)])
+def test_long_strips_on_both_sides_of_the_y_walk(ctx, dtype, sizes):
+    """A strip of 61 cells in x, long enough in y for the walking RK stage (4100
+    waves) and just not (4088): the bits of the one-plane kernel."""
+    from miso_amd import mhd
+    from miso_amd.autotune import get_tiles, set_tiles
+    t0 = get_tiles(ctx)
+    default = (t0.rk_pencil_bx, t0.rk_pencil_by, t0.sweep_chunk, t0.rk_variant, t0.rk_zchunk,
+               t0.av_fuse_xy, t0.av_xy_chunk)
+    g = mhd.Grid(*sizes, 2, dtype=dtype, device="cuda:0")
+    q0 = random_state((g.i_total, g.j_total, g.k_total), 4, dtype, amp=0.05)
+    bc = mhd.BoundaryCondition((1, 0, 1), SIGNS)
+    out = []
+    for variant in (0, 5):
+        set_tiles(ctx, 2, 8, 256, variant, 256, 1, 64)
+        try:
+            m = mhd.MHD(mhd.Config({"mhd": {"cfl_number": 0.4}}), g, ctx, gm=5.0 / 3.0)
+            m.apply_initial_condition(q0, bc)
+            dts = m.integrator.run(bc, m.qq, 2)
+            out.append((list(dts), m.qq.to_host(ctx)))
+        finally:
+            set_tiles(ctx, *default)
+    assert out[0][0] == out[1][0]
+    assert_bitwise(out[1][1], out[0][1], str(sizes))
