@@ -9,7 +9,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <cmath>
+#include "split_rounds.hpp"
 
 namespace misohip {
 
@@ -158,34 +158,6 @@ __device__ __forceinline__ int wrap_coord(int x, int total, int m, bool on) {
   if (!on) return x;
   const int n = total - 2 * m;
   return x < m ? x + n : (x >= total - m ? x - n : x);
-}
-
-// Chunks of a march or walk over n cells, none longer than `most`, in a
-// launch of per_chunk blocks each: of all counts the one with the least
-// rounds x length, where `slots` blocks run at a time and each costs `start`
-// cells more than it covers (its first window is loaded, and its first slopes
-// formed, anew).  The last round of a launch is then nearly full, and a small
-// grid is spread over the chip as far as the repeated cells allow.  Past
-// `even` rounds the blocks no longer end together: half a round is lost at the
-// end, and nothing is gained by more chunks (the FP32 z walk of 512^3, 2.7
-// rounds of 256 planes: 3.1 ms; 4 of 171: 3.3).  Every chunk starts from the
-// fields, so the results do not depend on the split.
-inline void split_rounds(int n, long per_chunk, int most, long slots, double start, double even,
-                         int &chunk, int &nchunks) {
-  const int least = most < 1 ? 1 : most;
-  double best = 0.0, rounds = 0.0;
-  nchunks = 0;
-  for (int m = (n + least - 1) / least; m <= n && rounds <= even; ++m) {
-    const int c = (n + m - 1) / m;
-    if ((n + c - 1) / c != m) continue;  // the same length as fewer chunks'
-    const double full = (double)per_chunk * m / slots;
-    const double cost = (full <= even ? std::ceil(full) : full + 0.5) * (c + start);
-    if (nchunks && cost > 0.98 * best) continue;
-    best = cost;
-    rounds = full;
-    chunk = c;
-    nchunks = m;
-  }
 }
 
 // Blocks of the z-march kernel: (nbx, nby) columns of 64 x TY cells, each cut

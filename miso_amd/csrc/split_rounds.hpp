@@ -1,0 +1,45 @@
+// How a march or walk is cut into chunks (host code, no HIP).
+#pragma once
+
+#include <cmath>
+
+namespace misohip {
+
+// Chunks of a march or walk over n cells, none longer than `most`, in a
+// launch of per_chunk blocks each: of all counts the one with the least
+// rounds x length, where `slots` blocks run at a time and each costs `start`
+// cells more than it covers (its first window is loaded, and its first slopes
+// formed, anew).  The last round of a launch is then nearly full, and a small
+// grid is spread over the chip as far as the repeated cells allow.  Past
+// `even` rounds the blocks no longer end together: half a round is lost at the
+// end, and nothing is gained by more chunks (the FP32 z walk of 512^3, 2.7
+// rounds of 256 planes: 3.1 ms; 4 of 171: 3.3).  Every chunk starts from the
+// fields, so the results do not depend on the split.
+//   Only counts with a length of their own are looked at, and none once even a
+// full last round could not win: m chunks cost at least the rounds they need
+// times the cells they walk, per_chunk / slots x (n + m start).  This runs at
+// every launch: 0.3 us for 256 cells, 1.7 for 100000 (every count up to n: 1.3
+// and 450).
+inline void split_rounds(int n, long per_chunk, int most, long slots, double start, double even,
+                         int &chunk, int &nchunks) {
+  const int least = most < 1 ? 1 : most;
+  const double load = (double)per_chunk / slots;
+  double best = 0.0, rounds = 0.0;
+  nchunks = 0;
+  for (int m = (n + least - 1) / least; m <= n && rounds <= even;) {
+    if (nchunks && load * (n + m * start) > best) break;
+    const int c = (n + m - 1) / m;
+    const double full = (double)per_chunk * m / slots;
+    const double cost = (full <= even ? std::ceil(full) : full + 0.5) * (c + start);
+    if (!nchunks || cost <= 0.98 * best) {
+      best = cost;
+      rounds = full;
+      chunk = c;
+      nchunks = m;
+    }
+    if (c == 1) break;
+    m = (n + c - 2) / (c - 1);  // the fewest chunks shorter than these
+  }
+}
+
+}  // namespace misohip

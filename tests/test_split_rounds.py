@@ -1,0 +1,30 @@
+"""The cut of marches and walks into chunks (miso_amd/csrc/split_rounds.hpp),
+on the CPU by tests/cpp/test_split_rounds.cpp: the choice of a scan of every
+count, at a cost that no launch notices.  It runs at every launch; scanning
+every count took 140 us for a strip of 32790 rows and 440 for 100000."""
+import ctypes
+import os
+
+import pytest
+
+LIB = os.path.join(os.path.dirname(__file__), "cpp", "_build", "libsplit_rounds_check.so")
+pytestmark = pytest.mark.skipif(not os.path.exists(LIB),
+                                reason="tests/cpp not built (run __graft_entry__.build())")
+
+
+def test_choice_is_that_of_a_full_scan():
+    lib = ctypes.CDLL(LIB)
+    msg, calls = ctypes.create_string_buffer(512), ctypes.c_int(0)
+    rc = lib.split_rounds_check(msg, 512, ctypes.byref(calls))
+    assert rc == 0, msg.value.decode()
+    assert calls.value > 50000, calls.value
+
+
+@pytest.mark.parametrize("n,per_chunk,slots", [(256, 1, 256), (32790, 1, 256), (100000, 1, 768),
+                                               (16384, 61, 768), (100000, 4000, 256)])
+def test_a_call_costs_far_less_than_a_launch(n, per_chunk, slots):
+    lib = ctypes.CDLL(LIB)
+    lib.split_rounds_time.restype = ctypes.c_double
+    lib.split_rounds_time.argtypes = [ctypes.c_int, ctypes.c_long, ctypes.c_int, ctypes.c_long]
+    us = lib.split_rounds_time(n, per_chunk, 256, slots)
+    assert us < 25.0, us
