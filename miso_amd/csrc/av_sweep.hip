@@ -864,6 +864,24 @@ constexpr double WALK_START = 4.0;
 constexpr int XY_SLOTS = 256;
 constexpr double XY_START = 5.0;
 
+// blocks of a y (dir 1) or z (dir 2) walk: nbx by nbo of four waves for each of
+// nchunks chunks
+struct WalkSplit {
+  int nbx, nbo, chunk, nchunks;
+};
+template <typename R> static WalkSplit walk_split(const Shape &sh, int dir, int most) {
+  const int ni = sh.It - 2 * sh.mi;
+  const int n_dir = dir == 1 ? sh.Jt - 2 * sh.mj : sh.Kt - 2 * sh.mk;
+  const int n_oth = dir == 1 ? sh.Kt - 2 * sh.mk : sh.Jt - 2 * sh.mj;
+  const int wx = walk_waves_x(n_oth);
+  WalkSplit w;
+  w.nbx = ((ni + 63) / 64 + wx - 1) / wx;
+  w.nbo = (n_oth + 4 / wx - 1) / (4 / wx);
+  split_rounds(n_dir, (long)w.nbx * w.nbo, walk_limit(ni, most, sizeof(R) == 8),
+               WALK_SLOTS<R>, WALK_START, 2.0, w.chunk, w.nchunks);
+  return w;
+}
+
 template <typename R, int DIR>
 static hipError_t launch_av_t(hipStream_t st, const Fld<const R> &q, const Fld<R> &r, R *cc_store,
                               const R *cc_in, const R *dd, const Shape &sh, const AvScalars &sc) {
@@ -887,14 +905,8 @@ template <typename R, int DIR, bool DEGEN = false>
 static hipError_t launch_walk_t(hipStream_t st, const Fld<const R> &q, const Fld<R> &r,
                                 const R *cc_in, const R *dd, const Shape &sh,
                                 const AvScalars &sc, const R *dz_arr = nullptr) {
-  const int n_dir = DIR == 1 ? sh.Jt - 2 * sh.mj : sh.Kt - 2 * sh.mk;
-  const int n_oth = DIR == 1 ? sh.Kt - 2 * sh.mk : sh.Jt - 2 * sh.mj;
-  const int wx = walk_waves_x(n_oth);
-  const int nbx = ((sh.It - 2 * sh.mi + 63) / 64 + wx - 1) / wx;
-  const int nbo = (n_oth + 4 / wx - 1) / (4 / wx);
-  int chunk, nchunks;  // even walk lengths
-  split_rounds(n_dir, (long)nbx * nbo, sc.chunk, WALK_SLOTS<R>, WALK_START, 2.0, chunk,
-               nchunks);
+  const WalkSplit w = walk_split<R>(sh, DIR, sc.chunk);
+  const int nbx = w.nbx, nbo = w.nbo, chunk = w.chunk, nchunks = w.nchunks;
   if (sc.nparts && (sc.part0 < 0 || sc.nparts < 0 || sc.part0 + sc.nparts > nchunks))
     return hipErrorInvalidValue;
   const long nbl = (long)(sc.nparts ? sc.nparts : nchunks) * nbx * nbo;
@@ -952,14 +964,8 @@ template <typename R, int DIR, bool DEGEN>
 static hipError_t launch_walk_cfl_t(hipStream_t st, const Fld<const R> &q, const Fld<R> &r,
                                     const R *cc_in, const R *dd, const Shape &sh,
                                     const AvScalars &sc, const R *dz_arr, const CflFuse<R> &cf) {
-  const int n_dir = DIR == 1 ? sh.Jt - 2 * sh.mj : sh.Kt - 2 * sh.mk;
-  const int n_oth = DIR == 1 ? sh.Kt - 2 * sh.mk : sh.Jt - 2 * sh.mj;
-  const int wx = walk_waves_x(n_oth);
-  const int nbx = ((sh.It - 2 * sh.mi + 63) / 64 + wx - 1) / wx;
-  const int nbo = (n_oth + 4 / wx - 1) / (4 / wx);
-  int chunk, nchunks;  // even walk lengths
-  split_rounds(n_dir, (long)nbx * nbo, sc.chunk, WALK_SLOTS<R>, WALK_START, 2.0, chunk,
-               nchunks);
+  const WalkSplit w = walk_split<R>(sh, DIR, sc.chunk);
+  const int nbx = w.nbx, nbo = w.nbo, chunk = w.chunk, nchunks = w.nchunks;
   if (sc.nparts && (sc.part0 < 0 || sc.nparts < 0 || sc.part0 + sc.nparts > nchunks))
     return hipErrorInvalidValue;
   const long nbl = (long)(sc.nparts ? sc.nparts : nchunks) * nbx * nbo;
@@ -1092,13 +1098,9 @@ hipError_t launch_batch_av(hipStream_t st, int dir, int mode, const BatchInst<R>
 
 template <typename R>
 void av_walk_split(const Shape &sh, int dir, int chunk_req, int *chunk, int *nchunks) {
-  const int n_dir = dir == 1 ? sh.Jt - 2 * sh.mj : sh.Kt - 2 * sh.mk;
-  const int n_oth = dir == 1 ? sh.Kt - 2 * sh.mk : sh.Jt - 2 * sh.mj;
-  const int wx = walk_waves_x(n_oth);
-  const int nbx = ((sh.It - 2 * sh.mi + 63) / 64 + wx - 1) / wx;
-  const int nbo = (n_oth + 4 / wx - 1) / (4 / wx);
-  split_rounds(n_dir, (long)nbx * nbo, chunk_req, WALK_SLOTS<R>, WALK_START, 2.0, *chunk,
-               *nchunks);
+  const WalkSplit w = walk_split<R>(sh, dir, chunk_req);
+  *chunk = w.chunk;
+  *nchunks = w.nchunks;
 }
 template void av_walk_split<double>(const Shape &, int, int, int *, int *);
 template void av_walk_split<float>(const Shape &, int, int, int *, int *);

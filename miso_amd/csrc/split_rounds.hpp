@@ -42,4 +42,20 @@ inline void split_rounds(int n, long per_chunk, int most, long slots, double sta
   }
 }
 
+// Longest walk of the y and z sweeps whose last 64-cell segment along x holds
+// `ni` cells or the rest of them.  A wave of at most eight lanes takes 4.8 us a
+// plane of a long walk where one of twelve or more takes 1.5 to 2.7 (512 x 512
+// rows, 256 planes, FP64; the cause was not found), and less in short ones: z
+// sweep of 4 x 512 x 512 1240 us in walks of 256, 830 of 64, 740 of 16 (FP32
+// 450, 345, 285); of 12 x 512 x 512 382, 382, 439.  Beside whole segments the
+// narrow one is the last to end in FP64: 72 x 512 x 512 2220 us in walks of
+// 256, 958 of 128, 934 of 64; 65 x 200 x 600 395, 395, 409 (FP32, 72 x 512 x
+// 512: 538, 547, 534; 260^3: 446, 489, 441).
+constexpr int WALK_NARROW = 8, WALK_NARROW_ALONE = 16, WALK_NARROW_LAST = 128;
+inline int walk_limit(int ni, int most, bool f64) {
+  if ((ni - 1) % 64 + 1 > WALK_NARROW || (ni > 64 && !f64)) return most;
+  const int limit = ni > 64 ? WALK_NARROW_LAST : WALK_NARROW_ALONE;
+  return most < limit ? most : limit;
+}
+
 }  // namespace misohip

@@ -72,3 +72,8 @@ extern "C" double split_rounds_time(int n, long per_chunk, int most, long slots)
   }
   return best;
 }
+
+// the longest walk of a y or z sweep over rows of ni cells
+extern "C" int walk_limit_of(int ni, int most, int f64) {
+  return misohip::walk_limit(ni, most, f64 != 0);
+}

@@ -28,3 +28,13 @@ def test_a_call_costs_far_less_than_a_launch(n, per_chunk, slots):
     lib.split_rounds_time.argtypes = [ctypes.c_int, ctypes.c_long, ctypes.c_int, ctypes.c_long]
     us = lib.split_rounds_time(n, per_chunk, 256, slots)
     assert us < 25.0, us
+
+
+@pytest.mark.parametrize("ni,most,f64,want", [
+    (1, 256, 1, 16), (8, 256, 1, 16), (8, 256, 0, 16), (8, 4, 1, 4), (9, 256, 1, 256),
+    (64, 256, 1, 256), (65, 256, 1, 128), (72, 256, 1, 128), (72, 64, 1, 64), (72, 256, 0, 256),
+    (73, 256, 1, 256), (512, 4096, 1, 4096)])
+def test_narrow_rows_walk_short(ni, most, f64, want):
+    """A last segment of at most eight cells: 72 x 512 x 512's z sweep in FP64
+    takes 2220 us in walks of 256 planes and 958 in walks of 128."""
+    assert ctypes.CDLL(LIB).walk_limit_of(ni, most, f64) == want
