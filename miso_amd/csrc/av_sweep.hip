@@ -853,16 +853,12 @@ __global__ __launch_bounds__(256) __attribute__((
 
 // Blocks that run at a time, and the rows a chunk costs more than it covers
 // (split_rounds): the y and z walks hold one FP64 wave per SIMD (256 registers
-// and a few more) or three FP32 ones; the x-y walk holds more, but is bound by
-// VALU issue, so that what counts is how evenly its blocks fall on the CUs.
-// Walks halved until the launch had 2^18 threads, as before, at 64^3 and 205 x
-// 131 x 93 in FP64: x-y 61 -> 49 and 229 -> 198 us, z with its CFL 27 -> 21
-// and 163 -> 122 (512 blocks: 24 and 132), y of 256^2 16 -> 8; FP32 of 181 x
-// 97 x 260: z 102 -> 92 (512 blocks: 102).
+// and a few more) or three FP32 ones.  Walks halved until the launch had 2^18
+// threads, as before, at 64^3 and 205 x 131 x 93 in FP64: z with its CFL 27 ->
+// 21 and 163 -> 122 us (512 blocks: 24 and 132), y of 256^2 16 -> 8; FP32 of
+// 181 x 97 x 260: z 102 -> 92 (512 blocks: 102).
 template <typename R> constexpr int WALK_SLOTS = sizeof(R) == 8 ? 256 : 768;
 constexpr double WALK_START = 4.0;
-constexpr int XY_SLOTS = 256;
-constexpr double XY_START = 5.0;
 
 // blocks of a y (dir 1) or z (dir 2) walk: nbx by nbo of four waves for each of
 // nchunks chunks
@@ -996,10 +992,9 @@ hipError_t launch_av_sweep_xy(hipStream_t st, const Fld<const R> &q, const Fld<R
   const int nj = sh.Jt - 2 * sh.mj;
   if (!sh.is || !sh.js || !sh.ks || nj < 2 || sh.mj < 2) return hipErrorInvalidValue;
   const int nseg = (sh.It - 2 * sh.mi + 59) / 60;
-  int chunk, nchunks;  // even walk lengths
-  split_rounds(nj, (nseg * (sh.Kt - 2L * sh.mk + 2) + 3) / 4, sc.chunk, XY_SLOTS, XY_START, 4.0, chunk,
-               nchunks);
   const int npl = sh.Kt - 2 * sh.mk + 2;  // interior planes and the two z ring planes
+  int chunk, nchunks;  // even walk lengths
+  split_xy(nj, nseg, npl, sc.nparts, sc.chunk, chunk, nchunks);
   if (sc.nparts && (sc.nparts < 0 || sc.nparts > npl || sc.part0 < sh.mk - 1 ||
                     sc.part0 > sh.Kt - sh.mk))
     return hipErrorInvalidValue;

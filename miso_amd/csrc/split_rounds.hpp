@@ -58,4 +58,23 @@ inline int walk_limit(int ni, int most, bool f64) {
   return most < limit ? most : limit;
 }
 
+// The x-y walk over nj rows: nseg waves for each of npl planes, four a block.
+// More than one of its blocks fits a CU, but it is bound by VALU issue, so that
+// what counts is how evenly they fall on the CUs.  Against walks halved until
+// the launch had 2^18 threads, at 64^3 and 205 x 131 x 93 in FP64: 61 -> 49 and
+// 229 -> 198 us.
+//   A launch of nparts planes, one slab of the overlapped walks, is cut by its
+// own blocks where those of the whole walk's cut would leave CUs idle (overlapped
+// FP32 step of 128^3 1237 -> 685 us, of 96^3 1211 -> 536, FP64 of 64^3 878 ->
+// 492; 256^3, whose slabs fill the chip, 5.61 ms either way).
+constexpr int XY_SLOTS = 256;
+constexpr double XY_START = 5.0;
+inline void split_xy(int nj, int nseg, int npl, int nparts, int most, int &chunk, int &nchunks) {
+  auto cut = [&](int planes) {
+    split_rounds(nj, ((long)nseg * planes + 3) / 4, most, XY_SLOTS, XY_START, 4.0, chunk, nchunks);
+  };
+  cut(npl);
+  if (nparts && ((long)nseg * nchunks * nparts + 3) / 4 < XY_SLOTS) cut(nparts);
+}
+
 }  // namespace misohip

@@ -77,3 +77,8 @@ extern "C" double split_rounds_time(int n, long per_chunk, int most, long slots)
 extern "C" int walk_limit_of(int ni, int most, int f64) {
   return misohip::walk_limit(ni, most, f64 != 0);
 }
+
+// rows and chunks of the x-y walk
+extern "C" void split_xy_of(int nj, int nseg, int npl, int nparts, int most, int *out) {
+  misohip::split_xy(nj, nseg, npl, nparts, most, out[0], out[1]);
+}

@@ -38,3 +38,21 @@ def test_narrow_rows_walk_short(ni, most, f64, want):
     """A last segment of at most eight cells: 72 x 512 x 512's z sweep in FP64
     takes 2220 us in walks of 256 planes and 958 in walks of 128."""
     assert ctypes.CDLL(LIB).walk_limit_of(ni, most, f64) == want
+
+
+@pytest.mark.parametrize("nj,nseg,npl,nparts", [(128, 3, 130, 11), (96, 2, 98, 8), (64, 2, 66, 4),
+                                                (300, 1, 92, 6)])
+def test_slabs_of_the_xy_walk_fill_the_chip(nj, nseg, npl, nparts):
+    """A slab of the overlapped walks has a few planes: the whole walk's cut
+    would make 22 to 90 blocks of it, for 256 CUs."""
+    lib, out = ctypes.CDLL(LIB), (ctypes.c_int * 2)()
+    lib.split_xy_of(nj, nseg, npl, nparts, 64, out)
+    chunk, n = out
+    assert chunk * n >= nj and (n - 1) * chunk < nj
+    waves = nseg * nparts
+    assert (waves * n + 3) // 4 >= 128 or chunk == 1
+    # slabs of a large box keep the whole walk's cut
+    lib.split_xy_of(512, 9, 514, 32, 64, out)
+    whole = tuple(out)
+    lib.split_xy_of(512, 9, 514, 0, 64, out)
+    assert tuple(out) == whole
