@@ -326,9 +326,10 @@ int update_t(misohip_ctx *ctx, const misohip_grid *g, const misohip_params *p,
   if (fuse_xy && ctx->tile.rk_variant >= 4 && ctx->tile.rk_variant <= 6)
     for (int a = 0; a < 3; ++a)
       if (bc->periodic[a] == 1) wrap |= 1 << a;
-  // In an x-y run with periodic and mirrored axes every pass stores the ghost
-  // cells with their sources instead, and no fill runs.
-  const GhostImg img = ctx->bc_fn ? GhostImg{} : ghost_img(sh, b);
+  // In an x-y run with periodic and mirrored axes and not too many rows every
+  // pass stores the ghost cells with their sources instead, and no fill runs.
+  const GhostImg img =
+      ctx->bc_fn ? GhostImg{} : ghost_img(sh, b, ctx->tile.rk_variant, sizeof(R) == 8);
   // stage 1 reads qq as both orgn and argm; later stages ping-pong between
   // the two workspace field sets.
   const misohip_fields *argm = qq;

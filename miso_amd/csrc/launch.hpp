@@ -51,11 +51,41 @@ struct BcDev {
   const void *fixed[9];
 };
 
-// the ghost cells of an x-y run that its passes can store themselves
-inline GhostImg ghost_img(const Shape &sh, const BcDev &b) {
+// The batched RK stage of runs with x and y axes and no z axis walks y:
+// each wave owns RK_YWALK_OUT x outputs over RK_YWALK_ROWS rows, four waves
+// per block (batch_rk_ywalk_kernel; the batch's block counts use these).
+constexpr int RK_YWALK_OUT = 60;
+constexpr int RK_YWALK_ROWS = 16;
+// A single x-y run walks y only when that makes at least this many waves, about
+// 2000^2: the one-plane kernel reads every cell at all its stencil points, and
+// is the faster one while the run's fields come from the last-level cache (FP32
+// stage of 1600 x 1500 66 us, the walk 79; FP64 of 1600 x 1590 170 and 174;
+// 2400^2 203 and 171, 363 and 348; 4096^2 599 and 446, 1079 and 976).
+constexpr int RK_YWALK_MIN_WAVES = 4096;
+
+inline bool rk_walks_y(const Shape &sh, int variant) {
+  const int ni = sh.It - 2 * sh.mi, nj = sh.Jt - 2 * sh.mj;
+  return sh.is && sh.js && !sh.ks && variant >= 4 && variant <= 6 &&
+         (long)((ni + RK_YWALK_OUT - 1) / RK_YWALK_OUT) *
+                 ((nj + RK_YWALK_ROWS - 1) / RK_YWALK_ROWS) >= RK_YWALK_MIN_WAVES;
+}
+
+// The ghost cells of an x-y run that its passes can store themselves, where
+// that costs less than the fills: those of the x faces are a few scattered
+// stores of an end lane in every row, which the wave waits for.  They pay up to
+// a number of rows, and in FP64 only beside the one-plane RK stage.  A step with
+// and without: FP64 of 512 x 4096 766 and 810 us, 61 x 8192 273 and 261, 61 x
+// 16384 487 and 434; FP32 of 61 x 16384 233 and 246, of 4 x 16384 285 and 298.
+// With the walking stage FP64 of 1000 x 4096 1485 and 1403, 2048^2 1412 and
+// 1403, 61 x 32790 1746 and 1443; FP32 of 2048^2 743 and 749, 1000 x 4096 740
+// and 739, 4096^2 2563 and 2532, 61 x 32790 721 and 625.
+inline GhostImg ghost_img(const Shape &sh, const BcDev &b, int variant, bool f64) {
   GhostImg m;
+  const bool walk = rk_walks_y(sh, variant);
+  const int rows = f64 ? (walk ? 0 : 6144) : (walk ? 3072 : 20480);
   m.on = sh.is && sh.js && !sh.ks && b.periodic[0] < 2 && b.periodic[1] < 2 &&
-         sh.It >= 3 * sh.mi && sh.Jt >= 3 * sh.mj;  // every image is a ghost cell
+         sh.It >= 3 * sh.mi && sh.Jt >= 3 * sh.mj &&  // every image is a ghost cell
+         sh.Jt - 2 * sh.mj <= rows;
   for (int a = 0; a < 2; ++a) {
     m.periodic[a] = b.periodic[a];
     for (int f = 0; f < 9; ++f)
@@ -204,18 +234,6 @@ __device__ __forceinline__ int batch_find(const int *__restrict__ start, int n, 
   }
   return lo;
 }
-
-// The batched RK stage of runs with x and y axes and no z axis walks y:
-// each wave owns RK_YWALK_OUT x outputs over RK_YWALK_ROWS rows, four waves
-// per block (batch_rk_ywalk_kernel; the batch's block counts use these).
-constexpr int RK_YWALK_OUT = 60;
-constexpr int RK_YWALK_ROWS = 16;
-// A single x-y run walks y only when that makes at least this many waves, about
-// 2000^2: the one-plane kernel reads every cell at all its stencil points, and
-// is the faster one while the run's fields come from the last-level cache (FP32
-// stage of 1600 x 1500 66 us, the walk 79; FP64 of 1600 x 1590 170 and 174;
-// 2400^2 203 and 171, 363 and 348; 4096^2 599 and 446, 1079 and 976).
-constexpr int RK_YWALK_MIN_WAVES = 4096;
 
 template <typename R>
 hipError_t launch_batch_rk(hipStream_t, const BatchInst<R> *, const BatchDyn<R> *, const int *,

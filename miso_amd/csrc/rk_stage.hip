@@ -926,13 +926,12 @@ static hipError_t launch_rk_t(hipStream_t st, const Fld<const R> &o, const Fld<c
                          a, r, dxi, dyi, dzi, sh, sc, mc);
     return hipGetLastError();
   }
-  const long yw_waves = (long)((ni + RK_YWALK_OUT - 1) / RK_YWALK_OUT) *
-                        ((nj + RK_YWALK_ROWS - 1) / RK_YWALK_ROWS);
-  if (HX && HY && !HZ && sc.variant >= 4 && sc.variant <= 6 && yw_waves >= RK_YWALK_MIN_WAVES) {
+  if (HX && HY && !HZ && rk_walks_y(sh, sc.variant)) {
     // an x-y run too large for the last-level cache (a smaller one runs the
     // one-plane kernel below)
     if (sh.mi < 2 || sh.mj < 2) return hipErrorInvalidValue;
-    const long nb = (yw_waves + 3) / 4;
+    const long nb = ((long)((ni + RK_YWALK_OUT - 1) / RK_YWALK_OUT) *
+                         ((nj + RK_YWALK_ROWS - 1) / RK_YWALK_ROWS) + 3) / 4;
     if (nb > 2147483647L) return hipErrorInvalidValue;
     hipLaunchKernelGGL((rk_stage_kernel_ywalk<R>), dim3((unsigned)nb), dim3(256), 0, st, o, a, r,
                        dxi, dyi, sh, sc, (int)nb);

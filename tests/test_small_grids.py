@@ -77,3 +77,49 @@ def test_long_strips_on_both_sides_of_the_y_walk(ctx, dtype, sizes):
             set_tiles(ctx, *default)
     assert out[0][0] == out[1][0]
     assert_bitwise(out[1][1], out[0][1], str(sizes))
+
+
+def _fills(ctx, fn):
+    """Ghost fills launched by fn()."""
+    import ctypes as C
+
+    from miso_amd import hip
+    hip.call("misohip_profile_enable", ctx.handle, 1)
+    try:
+        fn()
+        ms, n = (C.c_double * 8)(), (C.c_int * 8)()
+        hip.call("misohip_profile_read", ctx.handle, ms, n, 8)
+    finally:
+        hip.call("misohip_profile_enable", ctx.handle, 0)
+    return n[4]
+
+
+# the passes store the ghost cells up to a number of rows, by type and by the RK
+# stage's kernel: beyond, that costs more than the fills
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,sizes,fills", [
+    (np.float64, (5, 6144, 1), 0), (np.float64, (5, 6145, 1), 12),
+    (np.float32, (5, 20480, 1), 0), (np.float32, (5, 20481, 1), 12),
+    (np.float64, (2000, 1920, 1), 0), (np.float64, (2000, 1936, 1), 12),
+    (np.float32, (1300, 3072, 1), 0), (np.float32, (1300, 3073, 1), 12),
+])
+def test_ghost_fills_where_images_cost_more(ctx, dtype, sizes, fills):
+    import torch
+    from miso_amd import mhd
+    g = mhd.Grid(*sizes, 2, dtype=dtype, device="cuda:0")
+    m = mhd.MHD(mhd.Config({"mhd": {"cfl_number": 0.4}}), g, ctx, gm=5.0 / 3.0)
+    bc = mhd.BoundaryCondition((1, 0, 1), SIGNS)
+    m.apply_initial_condition(random_state((g.i_total, g.j_total, g.k_total), 4, dtype, amp=0.05),
+                              bc)
+    assert _fills(ctx, lambda: m.integrator.run(bc, m.qq, 2)) == fills
+    q = m.qq.data.clone()
+    m.integrator.apply_boundary_condition(bc, m.qq)
+    assert torch.isfinite(q).all() and torch.equal(q, m.qq.data)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", [(5, 6144, 1), (5, 6145, 1)])
+def test_strips_on_both_sides_of_the_images(ctx, sizes):
+    out, ref, dts, ref_dts = _both(ctx, sizes, (1, 0, 1), 2, True)
+    assert np.array_equal(dts, ref_dts), (dts, ref_dts)
+    assert_bitwise(out, ref, str(sizes))

@@ -44,7 +44,7 @@ def test_narrow_rows_walk_short(ni, most, f64, want):
                                                 (300, 1, 92, 6)])
 def test_slabs_of_the_xy_walk_fill_the_chip(nj, nseg, npl, nparts):
     """A slab of the overlapped walks has a few planes: the whole walk's cut
-    would make 22 to 90 blocks of it, for 256 CUs."""
+    would make 14 to 42 blocks of it, for 256 CUs."""
     lib, out = ctypes.CDLL(LIB), (ctypes.c_int * 2)()
     lib.split_xy_of(nj, nseg, npl, nparts, 64, out)
     chunk, n = out
