@@ -222,44 +222,51 @@ __global__ __launch_bounds__(64 * W) void rt_sweep_tile_kernel(
     lds_barrier();
     x.ih = edge[p & 1][w ? w - 1 : 0][lane];
   };
-  RtTilePlane<R> x0, x1, x2;
-  load(x0, p0 - 1, off, col);
-  load(x1, p0, off_i, col_i);
-  exchange(x0, p0 - 1);
   unsigned best = 0u;
-  auto step = [&](const RtTilePlane<R> &b4, RtTilePlane<R> &x, RtTilePlane<R> &nx, int p) {
-    load(nx, min(p + 1, pend - 1), off_i, col_i);
-    double I01 = b4.ih, K01 = b4.kh, S01 = b4.sh;
-    double I11 = lane_up(I01), K11 = lane_up(K01), S11 = lane_up(S01);
-    double now[R];
+  if (vw < Q.nc) {
+    RtTilePlane<R> x0, x1, x2;
+    load(x0, p0 - 1, off, col);
+    load(x1, p0, off_i, col_i);
+    exchange(x0, p0 - 1);
+    auto step = [&](const RtTilePlane<R> &b4, RtTilePlane<R> &x, RtTilePlane<R> &nx, int p) {
+      load(nx, min(p + 1, pend - 1), off_i, col_i);
+      double I01 = b4.ih, K01 = b4.kh, S01 = b4.sh;
+      double I11 = lane_up(I01), K11 = lane_up(K01), S11 = lane_up(S01);
+      double now[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const double I00 = b4.i[r], K00 = b4.k[r], S00 = b4.s[r];
-      const double I10 = lane_up(I00), K10 = lane_up(K00), S10 = lane_up(S00);
-      now[r] = rt_node<true>(Q, I00, I10, I01, I11, S00, S10, S01, S11, K00, K10, K01, K11,
-                             x.k[r], x.s[r]);
-      I01 = I00; K01 = K00; S01 = S00;
-      I11 = I10; K11 = K10; S11 = S10;
+      for (int r = 0; r < R; ++r) {
+        const double I00 = b4.i[r], K00 = b4.k[r], S00 = b4.s[r];
+        const double I10 = lane_up(I00), K10 = lane_up(K00), S10 = lane_up(S00);
+        now[r] = rt_node<true>(Q, I00, I10, I01, I11, S00, S10, S01, S11, K00, K10, K01, K11,
+                               x.k[r], x.s[r]);
+        I01 = I00; K01 = K00; S01 = S00;
+        I11 = I10; K11 = K10; S11 = S10;
+      }
+      if (own) {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          if (vw + r >= v_own && vw + r < Q.nc) {
+            best = max(best, rt_change(now[r], x.i[r]));
+            *at(Ir + (off[r] + p * Q.da), col) = now[r];
+          }
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r) x.i[r] = bound || vw + r < 0 ? x.i[r] : now[r];
+      exchange(x, p);
+    };
+    for (int p = p0;;) {
+      step(x0, x1, x2, p);
+      if (++p >= pend) break;
+      step(x1, x2, x0, p);
+      if (++p >= pend) break;
+      step(x2, x0, x1, p);
+      if (++p >= pend) break;
     }
-    if (own) {
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-        if (vw + r >= v_own && vw + r < Q.nc) {
-          best = max(best, rt_change(now[r], x.i[r]));
-          *at(Ir + (off[r] + p * Q.da), col) = now[r];
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r) x.i[r] = bound || vw + r < 0 ? x.i[r] : now[r];
-    exchange(x, p);
-  };
-  for (int p = p0;;) {
-    step(x0, x1, x2, p);
-    if (++p >= pend) break;
-    step(x1, x2, x0, p);
-    if (++p >= pend) break;
-    step(x2, x0, x1, p);
-    if (++p >= pend) break;
+  } else {
+    // rows past the ray's end: no stored node depends on them, and their loads
+    // would be most of a thin ray's (384^2 x 27, three iterations: 4.86 -> 4.53
+    // ms; x 20: 4.72 -> 4.30)
+    for (int p = p0 - 1; p < pend; ++p) lds_barrier();
   }
   rt_block_max(best, part);
 }
