@@ -314,10 +314,9 @@ int misohip_update_noalloc(misohip_ctx *ctx, const misohip_grid *g, misohip_dtyp
  * on x and on y) keeps its field of rint y-fastest, index
  * ((k * i_total + i) * j_total + j), so the planes it sweeps are contiguous;
  * misohip_rt_ray_layout names those rays.  0: every ray x-fastest.
- * sweep_planes 2..16: a ray with two real transverse axes advances
- * min(sweep_planes, 8) planes per launch; 0 or 1: one launch per plane for
- * every ray.  Results
- * are the same bits under every setting of both. */
+ * sweep_planes 2..16: a ray with two real transverse axes advances several
+ * planes per launch, as many as suit the box; 0 or 1: one launch per plane for
+ * every ray.  Results are the same bits under every setting of both. */
 typedef struct misohip_rt_config {
   int num_rays;
   int periodic[3];

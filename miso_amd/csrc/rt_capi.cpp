@@ -215,14 +215,14 @@ int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_c
     kap_y = ctx->rt_kap_y;
     src_y = ctx->rt_src_y;
   }
-  // Rays with two real transverse axes advance P planes per launch, patch by
-  // patch (rt_sweep_tile_kernel); the others one plane per launch.
-  const int P = std::min(rt->sweep_planes, RT_TILE_PLANES);
+  // Rays with two real transverse axes advance several planes per launch, patch
+  // by patch (rt_sweep_tile_kernel); the others one plane per launch.
   std::vector<RtRay> trays;
   std::vector<int> plane_rays;
   for (int n = 0; n < su.nrays; ++n) {
     const RtRay &R = su.rays.r[n];
-    if (P >= 2 && R.sb != 0 && R.sc != 0 && R.ua == R.da && (R.nb + 2L) * R.db < 1L << 29)
+    if (rt->sweep_planes >= 2 && R.sb != 0 && R.sc != 0 && R.ua == R.da &&
+        (R.nb + 2L) * R.db < 1L << 29)
       trays.push_back(R);
     else
       plane_rays.push_back(n);
@@ -238,7 +238,8 @@ int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_c
   });
   struct Chain {
     RtRays rays;
-    int n = 0, planes = 0, rows = RT_ROWS_SMALL;
+    int n = 0, planes = 0, rows = RT_ROWS_SMALL, P = RT_TILE_PLANES;
+    int max_nc = 0;
     long blocks = 0;  // workgroups of a launch in patches of RT_ROWS rows
   };
   std::vector<Chain> axes;
@@ -249,23 +250,27 @@ int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_c
     Chain &ch = axes.back();
     ch.rays.r[ch.n++] = R;
     ch.planes = std::max(ch.planes, R.nplanes);
-    ch.blocks += (long)rt_patches(R.nb, 64, P) * rt_patches(R.nc, RT_ROWS, P);
+    ch.max_nc = std::max(ch.max_nc, R.nc);
+    ch.blocks += (long)rt_patches(R.nb, 64, RT_TILE_PLANES) *
+                 rt_patches(R.nc, RT_ROWS, RT_TILE_PLANES);
   }
-  // chains of few workgroups take shorter patches and share their launches
+  // chains of few workgroups take shorter patches, and share their launches
+  // where these are alike
   std::vector<Chain> chains;
-  int few = -1;
   for (Chain &ch : axes) {
-    if (ch.blocks >= RT_FEW) {
-      ch.rows = RT_ROWS;
-    } else if (few < 0) {
-      few = (int)chains.size();
-    } else {
-      Chain &to = chains[few];
-      for (int r = 0; r < ch.n; ++r) to.rays.r[to.n++] = ch.rays.r[r];
-      to.planes = std::max(to.planes, ch.planes);
+    const bool full = ch.blocks >= RT_FEW;
+    if (full) ch.rows = RT_ROWS;
+    else if (ch.max_nc < ch.rows) ch.P = RT_TILE_PLANES_THIN;
+    Chain *to = nullptr;
+    if (!full)
+      for (Chain &c : chains)
+        if (c.rows == ch.rows && c.P == ch.P) to = &c;
+    if (!to) {
+      chains.push_back(ch);
       continue;
     }
-    chains.push_back(ch);
+    for (int r = 0; r < ch.n; ++r) to->rays.r[to->n++] = ch.rays.r[r];
+    to->planes = std::max(to->planes, ch.planes);
   }
   // Sweep phases: plane ranges over which the set of rays that still have
   // planes is constant; each phase launches only those rays, sized for
@@ -335,17 +340,18 @@ int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_c
       if (nside > 0) MISOHIP_TRY(hipEventRecord(ctx->rt_fork, ctx->stream));
       for (int i = 0; i < nside; ++i)
         MISOHIP_TRY(hipStreamWaitEvent(ctx->rt_side[i], ctx->rt_fork, 0));
-      int left = (int)chains.size();
-      for (int p0 = 0; left; p0 += P) {
-        left = 0;
+      bool left = !chains.empty();
+      for (int l = 0; left; ++l) {
+        left = false;
         for (size_t c = 0; c < chains.size(); ++c) {
           const Chain &ch = chains[c];
+          const int p0 = l * ch.P;
           if (p0 >= ch.planes) continue;
           const int i = (int)c % (nside + 1);
           MISOHIP_TRY(launch_rt_sweep_tiles(i ? ctx->rt_side[i - 1] : ctx->stream, I, kap, src,
-                                            kap_y, src_y, ch.rays, ch.n, p0, P, ch.rows,
+                                            kap_y, src_y, ch.rays, ch.n, p0, ch.P, ch.rows,
                                             su.ray_stride, parts));
-          if (p0 + P < ch.planes) ++left;
+          if (p0 + ch.P < ch.planes) left = true;
         }
       }
       for (const Phase &ph : phases)

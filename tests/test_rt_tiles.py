@@ -112,3 +112,62 @@ def test_patches_equal_the_plane_sweep_on_the_gpu(ctx, sizes, planes):
         assert res == out[0][0]
         assert torch.equal(I, out[0][1])
         assert torch.equal(q, out[0][2])
+
+
+# the two heights of a patch with the planes each takes per launch; sixteen
+# planes only where a short patch holds a ray's whole c axis
+@pytest.mark.parametrize("dims", [(8, 8, 8), (68, 6, 36), (70, 38, 12), (36, 70, 21), (22, 150, 9)])
+@pytest.mark.parametrize("rows,P", [(32, 8), (20, 8), (20, 16)])
+def test_patch_heights_give_the_plane_sweep(monkeypatch, dims, rows, P):
+    import sys
+    monkeypatch.setattr(sys.modules[__name__], "ROWS", rows)
+    rng = np.random.default_rng(2)
+    n = dims[0] * dims[1] * dims[2]
+    K, S, I0 = rng.random(n), rng.random(n), rng.random(n)
+    cases = 0
+    for dom, t, tr in ((0, (1, -1, 1), True), (1, (-1, 1, -1), False), (2, (1, 1, -1), False)):
+        R = _ray(dims, 2, dom, t, tr)
+        if P > 8 and R["nc"] >= rows:
+            continue
+        want, got = I0.copy(), I0.copy()
+        _plane_sweep(R, want, K, S)
+        _patched_sweep(R, got, K, S, P, n)
+        assert np.array_equal(want, got)
+        cases += 1
+    assert cases > 0
+
+
+def _equal_to_plane_sweep(ctx, sizes, rays, kinds, max_iters):
+    import torch
+
+    from miso_amd import mhd
+    from miso_amd.rt import RT
+    g = mhd.Grid(*sizes, 2, bounds=((0, 1), (0, 1), (0, 1)), device="cuda:0")
+    gen = torch.Generator(device="cuda:0").manual_seed(7)
+    shp = (g.k_total, g.j_total, g.i_total)
+    kap, S = (torch.rand(shp, generator=gen, device="cuda:0", dtype=torch.float64)
+              for _ in range(2))
+    out = []
+    for pl, yf in ((0, True),) + kinds:
+        rt = RT(g, rays)
+        rt.abs_coeff.copy_(20.0 * kap ** 3)
+        rt.src_func.copy_(1 + 0.3 * S)
+        kw = dict(periodic=(True, True, False), face_kind=(0, 0, 0, 0, 1, 2), tolerance=1e-9,
+                  max_iters=max_iters, sweep_planes=pl, x_rays_yfast=yf)
+        res = rt.solve(ctx, **kw)
+        q = rt.qrad(ctx, **kw).clone()
+        out.append((res, rt.intensities().clone(), q))
+        del rt
+    for res, I, q in out[1:]:
+        assert res == out[0][0]
+        assert torch.equal(I, out[0][1])
+        assert torch.equal(q, out[0][2])
+
+
+# boxes of few nodes along one axis: sixteen planes a launch, in patches wider
+# and narrower than the box, and of one ray
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes,rays", [((300, 40, 2), 24), ((131, 70, 19), 24), ((131, 70, 18), 24),
+                                        ((70, 16, 16), 24), ((16, 150, 12), 24), ((90, 2, 35), 1)])
+def test_thin_boxes_equal_the_plane_sweep(ctx, sizes, rays):
+    _equal_to_plane_sweep(ctx, sizes, rays, ((16, True), (2, True)), 6)
