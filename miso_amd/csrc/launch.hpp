@@ -154,6 +154,30 @@ __host__ __device__ inline int rt_patches(int n, int size, int P) {
 __host__ __device__ inline int rt_patch_first(int a, int size, int P) {
   return a == 0 ? -1 : size - 1 + (a - 1) * (size - P) - P;
 }
+// The cones of x rays kept x-fastest (rt_sweep_multi_kernel): RT_MULTI_PLANES
+// planes per launch, RT_MULTI_COLS columns of a plane to a workgroup, up to
+// RT_MULTI_ROWS rows with the boundary.
+constexpr int RT_MULTI_COLS = 32, RT_MULTI_PLANES = 16, RT_MULTI_ROWS = 33;
+// How a ray advances where several planes per launch are allowed.  One with a
+// degenerate axis, or a plane too large for a patch's 32-bit addresses: plane
+// by plane.  One whose neighbouring nodes are neighbours in memory: in patches.
+// The others, x rays kept x-fastest: in cones where these hold the c axis; in
+// patches where launches count or the fields exceed the caches; plane by plane
+// between (three iterations in patches and by planes: 48^3 0.67 and 1.04 ms,
+// 64^3 1.39 and 1.42, 80^3 2.38 and 2.11, 96^3 3.6 and 2.97, 128^3 5.9 and 5.9,
+// 500 x 30 x 40 4.3 and 8.6, 384^2 x 33 20.4 and 29.0, 211 x 150 x 187 13.5 and
+// 19.7; in patches and in cones: 20^3 0.22 and 0.33, 32^3 0.34 and
+// 0.47, 100^2 x 15 1.33 and 0.84).
+enum RtWay { RT_BY_PLANES, RT_IN_PATCHES, RT_IN_CONES };
+inline RtWay rt_way(const RtRay &R) {
+  if (R.sb == 0 || R.sc == 0 || R.ua != R.da || (R.nb + 2L) * R.db >= 1L << 29)
+    return RT_BY_PLANES;
+  if (R.db == 1) return RT_IN_PATCHES;
+  const long plane = (long)R.nb * R.nc, nodes = plane * R.nplanes;
+  if (nodes < 65536) return RT_IN_PATCHES;
+  if (R.nc < RT_MULTI_ROWS) return RT_IN_CONES;
+  return plane >= 5000 && nodes <= 1300000 ? RT_BY_PLANES : RT_IN_PATCHES;
+}
 // the patches of a launch, by groups of `same` rays with the same planes:
 // group g has patches start[g] .. start[g + 1] - 1, per_xcd go to each XCD
 struct RtPatches {
@@ -163,6 +187,8 @@ struct RtPatches {
 hipError_t launch_rt_sweep_tiles(hipStream_t, double *, const double *, const double *,
                                  const double *, const double *, const RtRays &, int, int, int,
                                  int, long, unsigned *);
+hipError_t launch_rt_sweep_multi(hipStream_t, double *, const double *, const double *,
+                                 const RtRays &, int, int, long, int, unsigned *);
 hipError_t launch_rt_xfast(hipStream_t, const double *, double *, int, int, int, int, unsigned);
 hipError_t launch_rt_incoming(hipStream_t, double *, const double *, const double *,
                               const RtIncoming &, long, int, unsigned *);

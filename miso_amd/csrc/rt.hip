@@ -112,6 +112,138 @@ __global__ __launch_bounds__(256) void rt_sweep_plane_kernel(double *__restrict_
   rt_block_max(best, part);
 }
 
+// Planes p0 .. p0 + P - 1 of every ray of `rays` in one launch, for rays with
+// neighbouring nodes of a plane in different cache lines (x rays kept x-fastest)
+// and a short c axis (nc < RT_MULTI_ROWS).  Such a sweep is bound by the lines
+// that its loads touch, so no node is loaded twice where it can be helped: a
+// workgroup owns the RT_MULTI_COLS columns u in [U0, U0 + W) of a ray over the
+// whole c range (u, v as in the patches below), and computes plane by plane the
+// cone u in [U0 - P, U0 + W) of nodes that its last plane depends on; the plane
+// is kept in LDS, column u = -1 and row v = -1 (the upwind boundary nodes, which
+// the sweep never writes) are read from memory.  Every node is computed by
+// rt_node from the same values as in rt_sweep_plane_kernel, so the results are
+// the same bits; cone nodes outside the owned columns are recomputed, not
+// stored, and the cone's stale edge (u below U0 - P + s + 1 at step s) never
+// reaches them.  Patches load a row and eight columns more for each that they
+// own: three iterations of 384^2 x 27 10.5 ms for 15.5, of 1024^2 x 3 11.1 for
+// 24.2, of 300 x 300 x 2 1.2 for 3.1.
+constexpr int RT_MULTI_THREADS = 1024;
+
+__global__ __launch_bounds__(RT_MULTI_THREADS) void rt_sweep_multi_kernel(double *__restrict__ I,
+                                                             const double *__restrict__ kap,
+                                                             const double *__restrict__ S,
+                                                             RtRays rays, int p0, int P,
+                                                             long ray_stride, unsigned *part) {
+  constexpr int W = RT_MULTI_COLS, X = RT_MULTI_COLS + RT_MULTI_PLANES, ROWS = RT_MULTI_ROWS;
+  constexpr int NT = RT_MULTI_THREADS, CPT = (X * ROWS + NT - 1) / NT;
+  __shared__ double Il[ROWS][X], Kl[ROWS][X], Sl[ROWS][X];
+  const RtRay &R = rays.r[blockIdx.y];
+  const int U0 = blockIdx.x * W;
+  // uniform over the workgroup
+  if (p0 >= R.nplanes || U0 >= R.nb || R.nc + 1 > ROWS || P < 1 || P > RT_MULTI_PLANES) return;
+  double *Ir = I + ray_stride * R.id;
+  const int ext = W + P, ncell = ext * (R.nc + 1);
+  const int pend = min(p0 + P, R.nplanes);
+  // per cell: memory index at plane 0, role (0 none, 1 boundary, read every
+  // plane; 2 computed; 3 computed and owned, its value before the sweep read
+  // for the change; 4 the cone's far edge e = 0,
+  // read for the plane before p0 only: never valid after it, and its node
+  // may be written by another workgroup meanwhile), LDS position
+  int off[CPT], role[CPT], ce[CPT], cr[CPT];
+#pragma unroll
+  for (int q = 0; q < CPT; ++q) {
+    const int idx = threadIdx.x + q * NT;
+    const int e = idx % ext, r = idx / ext;
+    const int u = U0 - P + e, v = r - 1;
+    ce[q] = e;
+    cr[q] = r;
+    role[q] = 0;
+    off[q] = 0;
+    if (idx >= ncell || u < -1 || u >= R.nb) continue;
+    const int ib = R.sb > 0 ? u : R.nb - 1 - u;
+    const int ic = R.sc > 0 ? v : R.nc - 1 - v;
+    off[q] = R.start + ib * R.db + ic * R.dc;
+    if (u == -1 || v == -1) role[q] = 1;
+    else if (e == 0) role[q] = 4;
+    else role[q] = (u >= U0 && u < U0 + W) ? 3 : 2;
+  }
+  // the plane before p0
+#pragma unroll
+  for (int q = 0; q < CPT; ++q)
+    if (role[q]) {
+      const int c = off[q] + (p0 - 1) * R.da;
+      Il[cr[q]][ce[q]] = Ir[c];
+      Kl[cr[q]][ce[q]] = kap[c];
+      Sl[cr[q]][ce[q]] = S[c];
+    }
+  // kappa, S and the boundary (role 1) or before-sweep (role 3) intensity of
+  // a plane's cells; loads run two planes ahead of the computation
+  auto load = [&](int p, double *k, double *s, double *b) {
+#pragma unroll
+    for (int q = 0; q < CPT; ++q) {
+      k[q] = s[q] = b[q] = 0.0;
+      if (p < pend && role[q] && role[q] < 4) {
+        const int c = off[q] + p * R.da;
+        k[q] = kap[c];
+        s[q] = S[c];
+        if (role[q] == 1 || role[q] == 3) b[q] = Ir[c];
+      }
+    }
+  };
+  double kc[CPT], sc[CPT], bnd[CPT], k1[CPT], s1[CPT], b1[CPT];
+  load(p0, kc, sc, bnd);
+  load(p0 + 1, k1, s1, b1);
+  __syncthreads();
+  unsigned best = 0u;
+  for (int p = p0; p < pend; ++p) {
+    double kn[CPT], sn[CPT], bn[CPT];
+    load(p + 2, kn, sn, bn);
+    double in[CPT];
+#pragma unroll
+    for (int q = 0; q < CPT; ++q) {
+      in[q] = bnd[q];
+      if (role[q] == 2 || role[q] == 3) {
+        const int r = cr[q], e = ce[q];
+        in[q] = rt_node<false>(R, Il[r][e], Il[r][e - 1], Il[r - 1][e], Il[r - 1][e - 1], Sl[r][e],
+                        Sl[r][e - 1], Sl[r - 1][e], Sl[r - 1][e - 1], Kl[r][e], Kl[r][e - 1],
+                        Kl[r - 1][e], Kl[r - 1][e - 1], kc[q], sc[q]);
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < CPT; ++q)
+      if (role[q] && role[q] < 4) {
+        Il[cr[q]][ce[q]] = in[q];
+        Kl[cr[q]][ce[q]] = kc[q];
+        Sl[cr[q]][ce[q]] = sc[q];
+        if (role[q] == 3) {
+          best = max(best, rt_change(in[q], bnd[q]));
+          Ir[off[q] + p * R.da] = in[q];
+        }
+      }
+#pragma unroll
+    for (int q = 0; q < CPT; ++q) {
+      kc[q] = k1[q];
+      sc[q] = s1[q];
+      bnd[q] = b1[q];
+      k1[q] = kn[q];
+      s1[q] = sn[q];
+      b1[q] = bn[q];
+    }
+    __syncthreads();
+  }
+  rt_block_max(best, part);
+}
+
+hipError_t launch_rt_sweep_multi(hipStream_t st, double *I, const double *kap, const double *S,
+                                 const RtRays &rays, int nrays, int p0, long ray_stride,
+                                 int max_nb, unsigned *part) {
+  dim3 grid((max_nb + RT_MULTI_COLS - 1) / RT_MULTI_COLS, nrays);
+  hipLaunchKernelGGL(rt_sweep_multi_kernel, grid, dim3(RT_MULTI_THREADS), 0, st, I, kap, S, rays,
+                     p0, RT_MULTI_PLANES, ray_stride, part);
+  return hipGetLastError();
+}
+
 // Planes p0 .. p0 + P - 1 of every ray of `rays` in one launch.  Node
 // coordinates are mirrored so that upwind is always one step back: u = ib
 // (sb > 0) or nb - 1 - ib, likewise v.  A workgroup takes a patch of 64

@@ -215,14 +215,14 @@ int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_c
     kap_y = ctx->rt_kap_y;
     src_y = ctx->rt_src_y;
   }
-  // Rays with two real transverse axes advance several planes per launch, patch
-  // by patch (rt_sweep_tile_kernel); the others one plane per launch.
+  // Rays with two real transverse axes advance several planes per launch, in
+  // patches (rt_sweep_tile_kernel) or cones (rt_sweep_multi_kernel); the others
+  // one plane per launch.
   std::vector<RtRay> trays;
   std::vector<int> plane_rays;
   for (int n = 0; n < su.nrays; ++n) {
     const RtRay &R = su.rays.r[n];
-    if (rt->sweep_planes >= 2 && R.sb != 0 && R.sc != 0 && R.ua == R.da &&
-        (R.nb + 2L) * R.db < 1L << 29)
+    if (rt->sweep_planes >= 2 && rt_way(R) != RT_BY_PLANES)
       trays.push_back(R);
     else
       plane_rays.push_back(n);
@@ -239,7 +239,8 @@ int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_c
   struct Chain {
     RtRays rays;
     int n = 0, planes = 0, rows = RT_ROWS_SMALL, P = RT_TILE_PLANES;
-    int max_nc = 0;
+    int max_nb = 0, max_nc = 0;
+    bool cones = false;
     long blocks = 0;  // workgroups of a launch in patches of RT_ROWS rows
   };
   std::vector<Chain> axes;
@@ -250,7 +251,9 @@ int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_c
     Chain &ch = axes.back();
     ch.rays.r[ch.n++] = R;
     ch.planes = std::max(ch.planes, R.nplanes);
+    ch.max_nb = std::max(ch.max_nb, R.nb);
     ch.max_nc = std::max(ch.max_nc, R.nc);
+    ch.cones = rt_way(R) == RT_IN_CONES;  // one way for the rays of an axis
     ch.blocks += (long)rt_patches(R.nb, 64, RT_TILE_PLANES) *
                  rt_patches(R.nc, RT_ROWS, RT_TILE_PLANES);
   }
@@ -259,12 +262,13 @@ int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_c
   std::vector<Chain> chains;
   for (Chain &ch : axes) {
     const bool full = ch.blocks >= RT_FEW;
-    if (full) ch.rows = RT_ROWS;
+    if (ch.cones) ch.P = RT_MULTI_PLANES;
+    else if (full) ch.rows = RT_ROWS;
     else if (ch.max_nc < ch.rows) ch.P = RT_TILE_PLANES_THIN;
     Chain *to = nullptr;
-    if (!full)
+    if (!full && !ch.cones)
       for (Chain &c : chains)
-        if (c.rows == ch.rows && c.P == ch.P) to = &c;
+        if (!c.cones && c.rows == ch.rows && c.P == ch.P) to = &c;
     if (!to) {
       chains.push_back(ch);
       continue;
@@ -348,9 +352,13 @@ int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_c
           const int p0 = l * ch.P;
           if (p0 >= ch.planes) continue;
           const int i = (int)c % (nside + 1);
-          MISOHIP_TRY(launch_rt_sweep_tiles(i ? ctx->rt_side[i - 1] : ctx->stream, I, kap, src,
-                                            kap_y, src_y, ch.rays, ch.n, p0, ch.P, ch.rows,
-                                            su.ray_stride, parts));
+          hipStream_t st = i ? ctx->rt_side[i - 1] : ctx->stream;
+          if (ch.cones)
+            MISOHIP_TRY(launch_rt_sweep_multi(st, I, kap, src, ch.rays, ch.n, p0, su.ray_stride,
+                                              ch.max_nb, parts));
+          else
+            MISOHIP_TRY(launch_rt_sweep_tiles(st, I, kap, src, kap_y, src_y, ch.rays, ch.n, p0,
+                                              ch.P, ch.rows, su.ray_stride, parts));
           if (p0 + ch.P < ch.planes) left = true;
         }
       }

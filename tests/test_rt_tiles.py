@@ -171,3 +171,12 @@ def _equal_to_plane_sweep(ctx, sizes, rays, kinds, max_iters):
                                         ((70, 16, 16), 24), ((16, 150, 12), 24), ((90, 2, 35), 1)])
 def test_thin_boxes_equal_the_plane_sweep(ctx, sizes, rays):
     _equal_to_plane_sweep(ctx, sizes, rays, ((16, True), (2, True)), 6)
+
+
+# every ray x-fastest: x rays in cones (up to 32 nodes along z, planes of one and
+# of several workgroups), by planes and in patches
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", [(70, 31, 32), (73, 32, 31), (170, 70, 3), (20, 33, 33),
+                                   (20, 20, 20), (70, 75, 72), (110, 112, 115)])
+def test_one_layout_equals_the_plane_sweep(ctx, sizes):
+    _equal_to_plane_sweep(ctx, sizes, 24, ((16, False), (4, False), (0, False)), 4)
