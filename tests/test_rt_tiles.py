@@ -180,3 +180,11 @@ def test_thin_boxes_equal_the_plane_sweep(ctx, sizes, rays):
                                    (20, 20, 20), (70, 75, 72), (110, 112, 115)])
 def test_one_layout_equals_the_plane_sweep(ctx, sizes):
     _equal_to_plane_sweep(ctx, sizes, 24, ((16, False), (4, False), (0, False)), 4)
+
+
+# axes of at least 128 workgroups: patches of 32 rows, an axis' rays in launches
+# and on a stream of their own; boxes with all, two and one of the axes so
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", [(128, 128, 128), (150, 131, 187), (70, 260, 250), (384, 384, 27)])
+def test_full_launches_equal_the_plane_sweep(ctx, sizes):
+    _equal_to_plane_sweep(ctx, sizes, 24, ((16, True),), 3)
