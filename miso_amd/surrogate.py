@@ -34,11 +34,12 @@ def interior_columns(field, grid):
 
 
 def _rows(x):
-    """(N, W) as the column kernels read it: row-major, FP32 or FP64."""
+    """x as the column kernels read it: (N, W) row-major, FP32 or FP64, the
+    axes after the first as one."""
     import torch
     if x.dtype not in (torch.float32, torch.float64):
         x = x.double()
-    x = x.contiguous()
+    x = x.flatten(1).contiguous()
     return x, hip.F64 if x.dtype == torch.float64 else hip.F32
 
 
@@ -48,9 +49,10 @@ def _stream(x):
 
 
 def _moments(x, rows):
-    """FP64 mean, standard deviation (n - 1) and mean magnitude of x[rows] by
-    column."""
+    """FP64 mean, standard deviation (n - 1) and mean magnitude of x[rows] over
+    the rows, each in the shape of a row."""
     import torch
+    row = x.shape[1:]
     x, dt = _rows(x)
     out = [torch.empty(x.shape[1], dtype=torch.float64, device=x.device) for _ in range(3)]
     work = torch.empty(2 * hip.MOMENT_SHARES * x.shape[1], dtype=torch.float64, device=x.device)
@@ -59,14 +61,14 @@ def _moments(x, rows):
                  C.c_void_p(rows.data_ptr()), rows.shape[0], x.shape[1],
                  *(C.c_void_p(t.data_ptr()) for t in out), C.c_void_p(work.data_ptr()),
                  _stream(x))
-    return out
+    return [t.reshape(row) for t in out]
 
 
 def _normalized(x, mean, sd, dtype):
     """(x - mean) / sd, formed in FP64, as bf16 or FP32."""
     import torch
-    x, dt = _rows(x)
     out = torch.empty(x.shape, dtype=dtype, device=x.device)
+    x, dt = _rows(x)
     with torch.cuda.device(x.device):
         hip.call("misohip_column_normalize", dt, C.c_void_p(x.data_ptr()), x.shape[0], x.shape[1],
                  C.c_void_p(mean.data_ptr()), C.c_void_p(sd.data_ptr()),

@@ -159,3 +159,31 @@ def test_training_data_moments_and_scaling(dtype, n, width, chosen):
     assert torch.equal(surrogate._normalized(x, mean, sd, torch.float32), want.float())
     odd = torch.cat([x[:1], x])[1:]  # rows from an odd offset on
     assert torch.equal(surrogate._normalized(odd, mean, sd, torch.float32), want.float())
+
+
+@pytest.mark.gpu
+def test_training_data_with_the_features_as_an_axis(ctx):
+    """Raw features as (N, features, nz): each row's values in the order of
+    (N, features nz), and the same weights."""
+    import torch
+    from miso_amd import surrogate
+    nz, n = 32, 160
+    g = torch.Generator().manual_seed(3)
+    feats = (torch.randn((n, 4, nz), generator=g) * 0.1 + 1).to("cuda:0")
+    targets = torch.randn((n, nz), generator=g, dtype=torch.float64).to("cuda:0")
+    got = []
+    for f in (feats.reshape(n, 4 * nz), feats):
+        s = surrogate.ColumnSurrogate(ctx, nz, hidden=32, features=4, max_batch=64, seed=5)
+        last, val = s.fit(f, targets, epochs=2, batch=32)
+        w = []
+        for layer, (i, o) in enumerate(zip(s.sizes[:-1], s.sizes[1:])):
+            a = np.zeros((o, i), np.float32)
+            from miso_amd import hip
+            hip.call("misohip_mlp_get_layer", ctx.handle, s.h, layer, 0, a.ctypes.data_as(C.c_void_p))
+            w.append(a)
+        got.append((last, val, w, [a.ravel() for a in s.norm]))
+        s.close()
+    assert got[0][:2] == got[1][:2] and np.isfinite(got[0][1])
+    for k in (2, 3):
+        for a, b in zip(got[0][k], got[1][k]):
+            assert np.array_equal(a, b)
