@@ -418,7 +418,8 @@ int misohip_mlp_qrad(misohip_ctx *ctx, misohip_mlp *m, const misohip_grid *g, co
  * column, in FP64: mean, standard deviation (n - 1), mean magnitude; work is
  * scratch of 2 x MISOHIP_MOMENT_SHARES x width doubles.  Normalize: out =
  * (x - mean) / sd of the first n rows, formed in FP64, as FP32 or bf16; width
- * a multiple of 4, out on a 16-byte boundary. */
+ * a multiple of 4, out on a 16-byte boundary.  Without rows (n = 0; x, rows and
+ * out may be null) the moments are NaN and nothing is scaled. */
 #define MISOHIP_MOMENT_SHARES 64
 int misohip_column_moments(misohip_dtype dt, const void *x, const long long *rows, long n,
                            int width, double *mean, double *sd, double *mean_abs, double *work,

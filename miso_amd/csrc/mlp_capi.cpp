@@ -276,7 +276,7 @@ int misohip_mlp_qrad(misohip_ctx *ctx, misohip_mlp *m, const misohip_grid *g, co
 int misohip_column_moments(misohip_dtype dt, const void *x, const long long *rows, long n,
                            int width, double *mean, double *sd, double *mean_abs, double *work,
                            void *stream) {
-  if (!x || !rows || !mean || !sd || !mean_abs || !work || n < 0 || width < 1)
+  if (n < 0 || width < 1 || (n > 0 && (!x || !rows)) || !mean || !sd || !mean_abs || !work)
     return MISOHIP_E_ARG;
   if (dt != MISOHIP_F64 && dt != MISOHIP_F32) return MISOHIP_E_DTYPE;
   MISOHIP_TRY(launch_moments(static_cast<hipStream_t>(stream), x, dt == MISOHIP_F64, rows, n,
@@ -287,7 +287,8 @@ int misohip_column_moments(misohip_dtype dt, const void *x, const long long *row
 int misohip_column_normalize(misohip_dtype dt, const void *x, long n, int width,
                              const double *mean, const double *sd, int bf16, void *out,
                              void *stream) {
-  if (!x || !mean || !sd || !out || n < 0 || width < 4 || width % 4) return MISOHIP_E_ARG;
+  if (n < 0 || width < 4 || width % 4 || (n > 0 && (!x || !out)) || !mean || !sd)
+    return MISOHIP_E_ARG;
   if (dt != MISOHIP_F64 && dt != MISOHIP_F32) return MISOHIP_E_DTYPE;
   if ((double)n * width / 1024.0 >= 4294967295.0) return MISOHIP_E_RANGE;
   if (n == 0) return MISOHIP_OK;

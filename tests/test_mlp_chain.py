@@ -187,3 +187,24 @@ def test_training_data_with_the_features_as_an_axis(ctx):
     for k in (2, 3):
         for a, b in zip(got[0][k], got[1][k]):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.gpu
+def test_fit_of_no_rows(ctx):
+    """No training data: NaN moments, no step, the weights as they were."""
+    import torch
+    from miso_amd import hip, surrogate
+    nz = 32
+    s = surrogate.ColumnSurrogate(ctx, nz, hidden=32, max_batch=64, seed=5)
+
+    def weights():
+        a = np.zeros((32, 3 * nz), np.float32)
+        hip.call("misohip_mlp_get_layer", ctx.handle, s.h, 0, 0, a.ctypes.data_as(C.c_void_p))
+        return a
+    before = weights()
+    assert s.fit(torch.empty((0, 3 * nz), device="cuda:0"),
+                 torch.empty((0, nz), dtype=torch.float64, device="cuda:0"), epochs=2,
+                 batch=32) == (0.0, None)
+    assert len(s.history) == 2 and all(np.isnan(a).all() for a in s.norm)
+    assert np.array_equal(weights(), before)
+    s.close()
