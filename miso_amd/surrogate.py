@@ -174,6 +174,11 @@ class ColumnSurrogate:
         (train MSE of the last epoch, validation relative L2 of Q_rad)."""
         import torch
         n = feats.shape[0]
+        # the kernels take row numbers and pointers as they are
+        if targets.shape[0] < n:
+            raise IndexError(f"{targets.shape[0]} target rows for {n} feature rows")
+        if targets.device != feats.device:
+            raise RuntimeError(f"features on {feats.device}, targets on {targets.device}")
         g = torch.Generator(device="cpu").manual_seed(seed)
         perm = torch.randperm(n, generator=g).to(feats.device)
         nval = max(batch, int(n * val_frac)) if n > 2 * batch else 0

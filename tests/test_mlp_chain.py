@@ -208,3 +208,19 @@ def test_fit_of_no_rows(ctx):
     assert len(s.history) == 2 and all(np.isnan(a).all() for a in s.norm)
     assert np.array_equal(weights(), before)
     s.close()
+
+
+@pytest.mark.parametrize("feats,targets,error", [
+    (dict(size=(100, 96)), dict(size=(99, 32)), IndexError),
+    (dict(size=(100, 96)), dict(size=(0, 32)), IndexError),
+    (dict(size=(100, 96)), dict(size=(100, 32), device="meta"), RuntimeError),
+])
+def test_fit_refuses_targets_it_would_read_past(feats, targets, error):
+    """Fewer targets than feature rows, or targets elsewhere: refused before any
+    kernel gets their pointers."""
+    import torch
+    from miso_amd.surrogate import ColumnSurrogate
+    s = ColumnSurrogate.__new__(ColumnSurrogate)
+    s.h = None
+    with pytest.raises(error, match="target"):
+        s.fit(torch.zeros(**feats), torch.zeros(**targets))
