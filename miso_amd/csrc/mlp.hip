@@ -59,10 +59,16 @@ constexpr int MLP_X_TALL = 128;
 // takes NS = 16 NT columns through all layers.  A layer is D = W a: the
 // weights are the A operand, from their packed copies (L2 holds all of them),
 // the activations the B operand, rows of one column in one of two buffers in
-// LDS (WIDE: in the workgroup's part of g0, g1, where two of them do not fit);
+// LDS (WIDE: in the columns' part of g0, g1, where two of them do not fit);
 // lanes are columns in D, so that a lane holds four consecutive outputs of
 // one column.  X passes through LDS in chunks of xw features (all but the last
 // a multiple of 32 PD: the k-steps in flight keep their places).
+//   WIDE: `phase` alone, a layer forward or (nl, nl + 1, ..) back, its input by
+// way of LDS as X, its outputs spread over the launch's rows of workgroups: with
+// all layers in a workgroup, which fetched its fragments from g0, g1 as it came
+// to them, a batch of 32 through 1536-2048-2048-2048-384 took 521 us, this 54
+// (128 x 128 tiles of a launch per layer 190; 16384 columns 2269, 668, 1053; a
+// training step's gradients at a batch of 32 972, 114, 490).
 //   A wave takes cnt <= RT row tiles of 16 outputs at a time and keeps PD
 // k-steps of their weights in flight; the first PD of the next layer are
 // loaded before the barrier that ends a layer.
@@ -87,7 +93,7 @@ template <int NT, int WAVES, int RT, int PD, bool TRAIN, bool WIDE>
 __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
     MlpNet net, const uint16_t *__restrict__ X, int M,
     float *__restrict__ Y, MlpLoss ls, MlpField fo, uint16_t *g0, uint16_t *g1, int bw, int xoff,
-    int xw) {
+    int xw, int phase) {
   constexpr int NS = 16 * NT, NTHR = 64 * WAVES;
   static_assert(RT <= 3, "product()");
   static_assert(NT > 1 || RT == 1, "one row tile a wave");
@@ -99,10 +105,13 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
   const int s0 = blockIdx.x * NS;
   const int pitch = bw + 8, xpitch = xw + 8;  // odd multiples of 16 bytes: no bank conflicts
   // the input layer writes the first buffer (X may be staged in the second)
-  uint16_t *nxt = WIDE ? g0 + (long)s0 * pitch : lds;
-  uint16_t *cur = WIDE ? g1 + (long)s0 * pitch : lds + NS * pitch;
+  uint16_t *nxt = WIDE ? (phase & 1 ? g1 : g0) + (long)s0 * pitch : lds;
+  uint16_t *cur = WIDE ? (phase & 1 ? g0 : g1) + (long)s0 * pitch : lds + NS * pitch;
   uint16_t *xbuf = lds + xoff;
-  const int n_in = net.n_in, nl = net.nl;
+  const int nl = net.nl;
+  // what passes through xbuf, by columns: X, in a layer of its own its input
+  const uint16_t *src = WIDE && phase ? cur : X + (long)s0 * net.n_in;
+  const int ld = WIDE && phase ? pitch : net.n_in;
 
   bf16x8 a[PD][RT];
   f32x4 acc[RT][NT];
@@ -138,9 +147,9 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
           make_uint4(v[0], v[1], v[2], v[3]);
     }
   };
-  // features [f0, f0 + cw) of the workgroup's columns into xbuf
-  auto stage = [&](int f0) {
-    const int cw = min(xw, n_in - f0), per = cw >> 3, n = NS * per;
+  // features [f0, f0 + cw) of K of the workgroup's columns into xbuf
+  auto stage = [&](int K, int f0) {
+    const int cw = min(xw, K - f0), per = cw >> 3, n = NS * per;
     chain_barrier<WIDE>();
     for (int t = tid; t < n; t += 4 * NTHR) {
       uint4 v[4];
@@ -149,7 +158,7 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
         const int q = t + e * NTHR, r = q / per, c = q - r * per;
         v[e] = make_uint4(0, 0, 0, 0);
         if (q < n && s0 + r < M)
-          v[e] = *reinterpret_cast<const uint4 *>(X + (long)(s0 + r) * n_in + f0 + 8 * c);
+          v[e] = *reinterpret_cast<const uint4 *>(src + (long)r * ld + f0 + 8 * c);
       }
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -164,13 +173,12 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
   // flight while the chunk before is multiplied
   constexpr int XW = MLP_X_TALL, XE = NT > 1 ? NS * XW / 8 / NTHR : 1;
   uint4 xr[XE];
-  auto fetch = [&](int f0) {
+  auto fetch = [&](int K, int f0) {
 #pragma unroll
     for (int e = 0; e < XE; ++e) {
       const int q = tid + e * NTHR, r = q / (XW / 8), f = f0 + 8 * (q % (XW / 8));
       xr[e] = make_uint4(0, 0, 0, 0);
-      if (s0 + r < M && f < n_in)
-        xr[e] = *reinterpret_cast<const uint4 *>(X + (long)(s0 + r) * n_in + f);
+      if (s0 + r < M && f < K) xr[e] = *reinterpret_cast<const uint4 *>(src + (long)r * ld + f);
     }
   };
   auto put = [&](uint16_t *xb) {
@@ -180,7 +188,8 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
       *reinterpret_cast<uint4 *>(xb + q / (XW / 8) * xpitch + 8 * (q % (XW / 8))) = xr[e];
     }
   };
-  // acc = W b over all k for `cnt` row tiles; input: b is X, chunk by chunk
+  // acc = W b over all k for `cnt` row tiles; input: b by way of xbuf, chunk by
+  // chunk; keep: b is X, for the weight gradients
   auto gemm = [&](auto cnt_, const uint16_t *wp, int KT, int OT, int base, const uint16_t *b,
                   bool input, bool keep) {
     constexpr int cnt = decltype(cnt_)::value;
@@ -225,18 +234,18 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
     if (!input) {
       steps(b + col * pitch + kq * 8, 16 * pitch, 0, KT);
     } else if constexpr (NT > 1) {
-      fetch(0);
+      fetch(32 * KT, 0);
       if (base) chain_barrier<WIDE>();
       put(xbuf);
       for (int k0 = 0, h = 0; k0 < KT; k0 += XW / 32, h ^= 1) {
         chain_barrier<WIDE>();
-        if (k0 + XW / 32 < KT) fetch(k0 * 32 + XW);
+        if (k0 + XW / 32 < KT) fetch(32 * KT, k0 * 32 + XW);
         steps(xbuf + (h * NS + col) * xpitch + kq * 8, 16 * xpitch, k0, min(XW / 32, KT - k0));
         if (k0 + XW / 32 < KT) put(xbuf + (h ^ 1) * NS * xpitch);
       }
     } else {
       for (int k0 = 0; k0 < KT; k0 += xw >> 5) {
-        const int cw = stage(k0 * 32);
+        const int cw = stage(32 * KT, k0 * 32);
         if (TRAIN && keep) pack(xbuf, xpitch, cw, net.aT, k0 * 32);
         steps(xbuf + col * xpitch + kq * 8, 16 * xpitch, k0, cw >> 5);
       }
@@ -300,17 +309,26 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
     }
   };
 
+  // the outputs of this workgroup among O, packed
+  auto pack_rows = [&](int O, uint16_t *dst) {
+    if (!WIDE) return pack(nxt, pitch, O, dst, 0);
+    for (int f = blockIdx.y * WAVES * 16; f < O; f += gridDim.y * WAVES * 16)
+      pack(nxt + f, pitch, min(WAVES * 16, O - f), dst, f);
+  };
+
   auto load4 = [](const float *q) { return *reinterpret_cast<const f32x4u *>(q); };
+  // WIDE: a row of workgroups per pass over the layer's outputs
+  const int row = WIDE ? blockIdx.y : 0, rows = WIDE ? gridDim.y : 1;
   // ---- forward
-  preload(net.wp, n_in / 32, net.out(0) / 16, 0, tiles_of(net.out(0) / 16));
-  for (int l = 0; l < nl; ++l) {
+  if (!WIDE) preload(net.wp, net.n_in / 32, net.out(0) / 16, 0, tiles_of(net.out(0) / 16));
+  for (int l = WIDE ? phase : 0; l < (WIDE ? min(phase + 1, nl) : nl); ++l) {
     const bool last = l == nl - 1;
     const int KT = net.in(l) / 32, O = net.out(l), OT = O / 16, cnt = tiles_of(OT);
     const uint16_t *wp = net.wp + net.w_at(l);
     const float *b = net.b + net.b_at(l);
-    for (int base = 0; base < OT; base += WAVES * cnt) {
-      if (base) preload(wp, KT, OT, base, cnt);
-      product(cnt, wp, KT, OT, base, cur, l == 0, base == 0);
+    for (int base = row * WAVES * cnt; base < OT; base += rows * WAVES * cnt) {
+      if (WIDE || base) preload(wp, KT, OT, base, cnt);
+      product(cnt, wp, KT, OT, base, cur, WIDE || l == 0, l == 0 && base == 0);
 #pragma unroll
       for (int r = 0; r < RT; ++r) {
         const int tile = base + wave * cnt + r;
@@ -345,14 +363,14 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
         }
       }
     }
-    if (!last)
+    if (!WIDE && !last)
       preload(net.wp + net.w_at(l + 1), O / 32, net.out(l + 1) / 16, 0,
               tiles_of(net.out(l + 1) / 16));
-    else if (TRAIN)
+    else if (!WIDE && TRAIN)
       preload(net.wtp + net.w_at(l), O / 32, net.in(l) / 16, 0, tiles_of(net.in(l) / 16));
-    if (!last || TRAIN) {
+    if (TRAIN || (!WIDE && !last)) {
       chain_barrier<WIDE>();
-      if (TRAIN) pack(nxt, pitch, O, last ? net.dT + net.d_at(l) : net.aT + net.a_at(l + 1), 0);
+      if (TRAIN) pack_rows(O, last ? net.dT + net.d_at(l) : net.aT + net.a_at(l + 1));
       uint16_t *swap = cur;
       cur = nxt;
       nxt = swap;
@@ -360,12 +378,13 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
   }
   if constexpr (TRAIN) {
     // ---- back: the gradient of layer l's input, times silu' of layer l - 1
-    for (int l = nl - 1; l > 0; --l) {
+    const int from = !WIDE ? nl - 1 : phase < nl ? 0 : 2 * nl - 1 - phase;
+    for (int l = from; l > (WIDE ? max(from - 1, 0) : 0); --l) {
       const int KT = net.out(l) / 32, I = net.in(l), OT = I / 16, cnt = tiles_of(OT);
       const uint16_t *wp = net.wtp + net.w_at(l);
-      for (int base = 0; base < OT; base += WAVES * cnt) {
-        if (base) preload(wp, KT, OT, base, cnt);
-        product(cnt, wp, KT, OT, base, cur, false, false);
+      for (int base = row * WAVES * cnt; base < OT; base += rows * WAVES * cnt) {
+        if (WIDE || base) preload(wp, KT, OT, base, cnt);
+        product(cnt, wp, KT, OT, base, cur, WIDE, false);
         const int tile = base + wave;
         if (tile < OT) {
           const f32x4 x = *reinterpret_cast<const f32x4 *>(
@@ -379,11 +398,11 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
           *reinterpret_cast<uint2 *>(nxt + col * pitch + tile * 16 + 4 * kq) = f2bf4(g);
         }
       }
-      if (l > 1)
+      if (!WIDE && l > 1)
         preload(net.wtp + net.w_at(l - 1), I / 32, net.in(l - 1) / 16, 0,
                 tiles_of(net.in(l - 1) / 16));
       chain_barrier<WIDE>();
-      pack(nxt, pitch, I, net.dT + net.d_at(l - 1), 0);
+      pack_rows(I, net.dT + net.d_at(l - 1));
       uint16_t *swap = cur;
       cur = nxt;
       nxt = swap;
@@ -775,6 +794,17 @@ namespace {
 
 // columns from which inference takes 64 to a workgroup: fewer leave CUs idle
 constexpr int MLP_TALL = 8192;
+// A layer of its own (WIDE) takes 64 columns to a workgroup where that still
+// makes this many of them, 16 otherwise (1536-2048-2048-2048-384, 2048 columns:
+// 118 and 162 us; 1024: 110 and 92; 1536-1024-1024-1024-384, 4096: 88 and 125,
+// 2048: 81 and 68).
+constexpr int MLP_LAYER_TALL = 192;
+// Hidden widths above this go by layers in inference also where LDS would hold
+// them: a small batch has a few workgroups, and each would read all weights
+// (1536-1536-1536-1536-384, one column: 42 us for 160, 16384: 387 for 613).
+// Training, 16 columns a workgroup, stays in one launch (batch of 4096: 428 us
+// for 616).
+constexpr int MLP_LAYERS = 1024;
 constexpr int LDS_BYTES = 160 * 1024;
 // features of X that a 16-column workgroup stages at a time
 int x_width(int n_in) { return n_in < 2048 ? n_in : 2048; }
@@ -784,58 +814,80 @@ size_t chain_lds(int ns, int bw, int xw) {
   return sizeof(uint16_t) * ns * ((bw ? 2 * (bw + 8) : 0) + (xw ? xw + 8 : 0));
 }
 
+// workgroups per tile of columns for a layer of its own: `per` row tiles each
+int wide_rows(const MlpNet &net, int phase, int per) {
+  const int O = phase < net.nl ? net.out(phase) : net.in(2 * net.nl - 1 - phase);
+  return (O / 16 + per - 1) / per;
+}
+
 template <int NT, int WAVES, int RT, int PD, bool TRAIN, bool WIDE>
 hipError_t chain(hipStream_t st, const MlpNet &net, const uint16_t *X, int M, float *Y,
                  const MlpLoss &ls, const MlpField &fo, uint16_t *g0, uint16_t *g1, int bw,
-                 int xoff, int xw, size_t bytes) {
+                 int xoff, int xw, size_t bytes, int phase = 0) {
   auto k = mlp_chain_kernel<NT, WAVES, RT, PD, TRAIN, WIDE>;
   if (bytes > 65536) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(k, dim3((M + 16 * NT - 1) / (16 * NT)), dim3(64 * WAVES), bytes, st, net,
-                     X, M, Y, ls, fo, g0, g1, bw, xoff, xw);
+  const dim3 grid((M + 16 * NT - 1) / (16 * NT),
+                  WIDE ? wide_rows(net, phase, WAVES * RT) : 1);
+  hipLaunchKernelGGL(k, grid, dim3(64 * WAVES), bytes, st, net, X, M, Y, ls, fo, g0, g1, bw, xoff,
+                     xw, phase);
   return hipGetLastError();
 }
 
 }  // namespace
 
-bool mlp_is_wide(int n_in, int maxw) {
-  return chain_lds(16, maxw, x_width(n_in)) + 1024 > (size_t)LDS_BYTES;
+bool mlp_is_wide(int n_in, int width) {
+  return chain_lds(16, width, x_width(n_in)) + 1024 > (size_t)LDS_BYTES;
+}
+bool mlp_by_layers(int n_in, int n_hidden) {
+  return n_hidden > MLP_LAYERS || mlp_is_wide(n_in, n_hidden);
 }
 
-hipError_t launch_mlp_forward(hipStream_t st, const MlpNet &net, bool wide, int maxw,
-                              const uint16_t *X, int M, float *Y, const MlpField &fo,
-                              uint16_t *g0, uint16_t *g1) {
+hipError_t launch_mlp_forward(hipStream_t st, const MlpNet &net, int maxw, const uint16_t *X,
+                              int M, float *Y, const MlpField &fo, uint16_t *g0, uint16_t *g1) {
   const int n_in = net.n_in, n_hidden = net.n_hidden;
   const MlpLoss none{};
+  constexpr int NT = 4, NS = 16 * NT;
+  if (mlp_by_layers(n_in, n_hidden)) {
+    const int xw = x_width(std::max(n_in, n_hidden));
+    hipError_t e = hipSuccess;
+    for (int p = 0; p < net.nl && e == hipSuccess; ++p)
+      e = (long)((M + NS - 1) / NS) * wide_rows(net, p, 16) >= MLP_LAYER_TALL
+              ? chain<NT, 8, 2, 2, false, true>(st, net, X, M, Y, none, fo, g0, g1, maxw, 0,
+                                                MLP_X_TALL,
+                                                sizeof(uint16_t) * NS * 2 * (MLP_X_TALL + 8), p)
+              : chain<1, 16, 1, 4, false, true>(st, net, X, M, Y, none, fo, g0, g1, maxw, 0, xw,
+                                                chain_lds(16, 0, xw), p);
+    return e;
+  }
   // X passes through the place of the second buffer, two chunks of it (the
   // input layer writes the first buffer)
-  constexpr int NT = 4, NS = 16 * NT;
   const size_t tall = sizeof(uint16_t) * NS *
                       (n_hidden + 8 + std::max(n_hidden + 8, 2 * (MLP_X_TALL + 8)));
   if (M >= MLP_TALL && tall <= (size_t)LDS_BYTES)
     return chain<NT, 8, 2, 2, false, false>(st, net, X, M, Y, none, fo, g0, g1, n_hidden,
                                             NS * (n_hidden + 8), MLP_X_TALL, tall);
   const int xw = x_width(n_in);
-  if (wide)
-    return chain<1, 16, 1, 4, false, true>(st, net, X, M, Y, none, fo, g0, g1, maxw, 0, xw,
-                                           chain_lds(16, 0, xw));
-  return chain<1, 16, 1, 4, false, false>(st, net, X, M, Y, none, fo, g0, g1, maxw,
-                                          32 * (maxw + 8), xw, chain_lds(16, maxw, xw));
+  return chain<1, 16, 1, 4, false, false>(st, net, X, M, Y, none, fo, g0, g1, n_hidden,
+                                          32 * (n_hidden + 8), xw, chain_lds(16, n_hidden, xw));
 }
 
 hipError_t launch_mlp_grad(hipStream_t st, const MlpNet &net, bool wide, int maxw,
                            const uint16_t *X, int M, const MlpLoss &ls, float *Y, uint16_t *g0,
                            uint16_t *g1) {
   const MlpField none{};
-  const int xw = x_width(net.n_in);
-  hipError_t e =
-      wide ? chain<1, 16, 1, 4, true, true>(st, net, X, M, Y, ls, none, g0, g1, maxw, 0, xw,
-                                            chain_lds(16, 0, xw))
-           : chain<1, 16, 1, 4, true, false>(st, net, X, M, Y, ls, none, g0, g1, maxw,
-                                             32 * (maxw + 8), xw, chain_lds(16, maxw, xw));
+  const int xw = x_width(wide ? std::max(net.n_in, maxw) : net.n_in);
+  hipError_t e = hipSuccess;
+  if (wide)
+    for (int p = 0; p < 2 * net.nl - 1 && e == hipSuccess; ++p)
+      e = chain<1, 16, 1, 4, true, true>(st, net, X, M, Y, ls, none, g0, g1, maxw, 0, xw,
+                                         chain_lds(16, 0, xw), p);
+  else
+    e = chain<1, 16, 1, 4, true, false>(st, net, X, M, Y, ls, none, g0, g1, maxw, 32 * (maxw + 8),
+                                        xw, chain_lds(16, maxw, xw));
   if (e != hipSuccess) return e;
   int splits = 16;  // equal sums of whole k-steps
   while (M % (32 * splits)) --splits;

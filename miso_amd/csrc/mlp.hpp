@@ -58,11 +58,13 @@ struct MlpField {
   int col0;  // the interior column (i fastest) of the first one
 };
 
-// two activation buffers of 16 columns and widths up to maxw exceed the LDS
-bool mlp_is_wide(int n_in, int maxw);
-hipError_t launch_mlp_forward(hipStream_t, const MlpNet &, bool wide, int maxw,
-                              const uint16_t *X, int M, float *Y, const MlpField &, uint16_t *g0,
-                              uint16_t *g1);
+// two activation buffers of 16 columns and widths up to `width` exceed the LDS
+bool mlp_is_wide(int n_in, int width);
+// inference goes layer by layer, by way of g0 and g1
+bool mlp_by_layers(int n_in, int n_hidden);
+// g0, g1: rows of maxw + 8 for M columns, rounded up to whole 64s
+hipError_t launch_mlp_forward(hipStream_t, const MlpNet &, int maxw, const uint16_t *X, int M,
+                              float *Y, const MlpField &, uint16_t *g0, uint16_t *g1);
 // Y may be null
 hipError_t launch_mlp_grad(hipStream_t, const MlpNet &, bool wide, int maxw, const uint16_t *X,
                            int M, const MlpLoss &, float *Y, uint16_t *g0, uint16_t *g1);

@@ -15,7 +15,8 @@ struct misohip_mlp {
   int n_in, n_hidden, n_out, n_layers;  // n_layers = hidden layers + output layer
   int max_batch;
   int maxw;    // the widest activation
-  bool wide;   // activations in g0, g1 instead of LDS
+  bool wide;   // training: activations in g0, g1 instead of LDS
+  bool by_layers;  // inference: the same
   long t;  // Adam step
   MlpNet net;
   uint16_t *g0 = nullptr, *g1 = nullptr;
@@ -40,8 +41,7 @@ template <typename T> hipError_t alloc(misohip_mlp *m, T **p, size_t n) {
 
 int forward(misohip_ctx *ctx, misohip_mlp *m, const uint16_t *X, int batch, float *Y,
             const MlpField &field) {
-  MISOHIP_TRY(launch_mlp_forward(ctx->stream, m->net, m->wide, m->maxw, X, batch, Y, field, m->g0,
-                                 m->g1));
+  MISOHIP_TRY(launch_mlp_forward(ctx->stream, m->net, m->maxw, X, batch, Y, field, m->g0, m->g1));
   return MISOHIP_OK;
 }
 
@@ -80,6 +80,7 @@ int misohip_mlp_create(misohip_ctx *ctx, int n_in, int n_hidden, int n_hidden_la
   m->t = 0;
   m->maxw = n_hidden > n_out ? n_hidden : n_out;
   m->wide = mlp_is_wide(n_in, m->maxw);
+  m->by_layers = mlp_by_layers(n_in, n_hidden);
   hipError_t e = hipSuccess;
   MlpNet &net = m->net;
   net.n_in = n_in;
@@ -99,9 +100,10 @@ int misohip_mlp_create(misohip_ctx *ctx, int n_in, int n_hidden, int n_hidden_la
   if (e == hipSuccess) e = alloc(m, &net.aT, (size_t)net.a_at(m->n_layers));
   if (e == hipSuccess)
     e = alloc(m, &net.dT, (size_t)net.d_at(m->n_layers - 1) + (size_t)max_batch * n_out);
-  if (m->wide) {
-    if (e == hipSuccess) e = alloc(m, &m->g0, (size_t)max_batch * (m->maxw + 8));
-    if (e == hipSuccess) e = alloc(m, &m->g1, (size_t)max_batch * (m->maxw + 8));
+  if (m->wide || m->by_layers) {
+    const size_t rows = (size_t)(max_batch + 63) / 64 * 64;  // whole tiles of columns
+    if (e == hipSuccess) e = alloc(m, &m->g0, rows * (m->maxw + 8));
+    if (e == hipSuccess) e = alloc(m, &m->g1, rows * (m->maxw + 8));
   }
   if (e == hipSuccess) e = alloc(m, &m->loss_part, (size_t)max_batch * n_out / 256 + 1);
   if (e == hipSuccess) e = alloc(m, &m->y, (size_t)max_batch * n_out);
@@ -262,7 +264,7 @@ int misohip_mlp_qrad(misohip_ctx *ctx, misohip_mlp *m, const misohip_grid *g, co
   f.qrad = static_cast<double *>(qrad);
   f.sh = shape_of(g);
   // activations in LDS: any number of columns; else as many as g0, g1 hold
-  const int step = m->wide ? m->max_batch : ncol;
+  const int step = m->by_layers ? m->max_batch : ncol;
   for (int c0 = 0; c0 < ncol; c0 += step) {
     const int nb = ncol - c0 < step ? ncol - c0 : step;
     f.col0 = c0;

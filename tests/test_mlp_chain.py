@@ -224,3 +224,37 @@ def test_fit_refuses_targets_it_would_read_past(feats, targets, error):
     s.h = None
     with pytest.raises(error, match="target"):
         s.fit(torch.zeros(**feats), torch.zeros(**targets))
+
+
+# hidden layers above 1024 in inference, and above what LDS holds in training: a
+# launch per layer, 16 or 64 columns to a workgroup by their number, one or more
+# rows of workgroups over the outputs; inputs in two chunks
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes", [[64, 1056, 1056, 96], [32, 1600, 1600, 32], [2080, 2112, 160]])
+@pytest.mark.parametrize("batch", [1, 17, 1100, 2081])
+def test_forward_by_layers(ctx, sizes, batch):
+    import torch
+    net, Ws, bs = _net(ctx, sizes, 2112, 13)
+    X = MO.to_bf16(np.random.default_rng(14).standard_normal((batch, sizes[0])))
+    Y = torch.full((batch + 1, sizes[-1]), 7.0, dtype=torch.float32, device="cuda:0")
+    net.hip.call("misohip_mlp_forward", ctx.handle, net.h, _ptr(_bf16_dev(X)), batch, _ptr(Y))
+    torch.cuda.synchronize()
+    ref, _, _ = MO.forward([MO.to_bf16(w) for w in Ws], bs, X)
+    got = Y.cpu().numpy()
+    assert np.abs(got[:batch] - ref).max() <= 2e-3 * np.abs(ref).max()
+    assert (got[batch] == 7.0).all()
+    net.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sizes,batch", [([32, 1600, 32], 32), ([2080, 2112, 2112, 96], 96),
+                                         ([32, 64, 2080], 64)])
+def test_gradients_by_layers(ctx, sizes, batch):
+    import torch
+    net, Ws, bs = _net(ctx, sizes, batch, 11)
+    rng = np.random.default_rng(12)
+    X = MO.to_bf16(rng.standard_normal((batch, sizes[0])))
+    T = rng.standard_normal((batch, sizes[-1])).astype(np.float32).astype(np.float64)
+    _check_grads(net, Ws, bs, X, T,
+                 _grad(net, ctx, _bf16_dev(X), torch.from_numpy(T.astype(np.float32)).to("cuda:0")))
+    net.close()
