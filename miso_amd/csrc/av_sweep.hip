@@ -874,7 +874,8 @@ template <typename R> static WalkSplit walk_split(const Shape &sh, int dir, int 
   w.nbx = ((ni + 63) / 64 + wx - 1) / wx;
   w.nbo = (n_oth + 4 / wx - 1) / (4 / wx);
   split_rounds(n_dir, (long)w.nbx * w.nbo, walk_limit(ni, most, sizeof(R) == 8),
-               WALK_SLOTS<R>, WALK_START, 2.0, w.chunk, w.nchunks);
+               WALK_SLOTS<R> * (ni <= WALK_NARROW ? WALK_NARROW_SLOTS : 1), WALK_START, 2.0, w.chunk,
+               w.nchunks);
   return w;
 }
 
