@@ -278,7 +278,7 @@ template <int R> struct RtTilePlane {
   double ih, kh, sh;        // the row above them
 };
 
-template <int R, int W>
+template <int R, int W, bool THIN>
 __global__ __launch_bounds__(64 * W) void rt_sweep_tile_kernel(
     double *__restrict__ I, const double *__restrict__ kap_x, const double *__restrict__ S_x,
     const double *__restrict__ kap_y, const double *__restrict__ S_y, RtRays rays, RtPatches pt,
@@ -355,7 +355,7 @@ __global__ __launch_bounds__(64 * W) void rt_sweep_tile_kernel(
     x.ih = edge[p & 1][w ? w - 1 : 0][lane];
   };
   unsigned best = 0u;
-  if (vw < Q.nc) {
+  if (!THIN || vw < Q.nc) {
     RtTilePlane<R> x0, x1, x2;
     load(x0, p0 - 1, off, col);
     load(x1, p0, off_i, col_i);
@@ -395,9 +395,9 @@ __global__ __launch_bounds__(64 * W) void rt_sweep_tile_kernel(
       if (++p >= pend) break;
     }
   } else {
-    // rows past the ray's end: no stored node depends on them, and their loads
-    // would be most of a thin ray's (384^2 x 27, three iterations: 4.86 -> 4.53
-    // ms; x 20: 4.72 -> 4.30)
+    // THIN: rows past the ray's end: no stored node depends on them, and their
+    // loads would be most of a thin ray's (elsewhere the branch costs more than
+    // the few rows that it saves: slab solve of 384^2 x 27 2.95 -> 2.97 ms)
     for (int p = p0 - 1; p < pend; ++p) lds_barrier();
   }
   rt_block_max(best, part);
@@ -431,12 +431,16 @@ hipError_t launch_rt_sweep_tiles(hipStream_t st, double *I, const double *kap, c
   if (!pt.start[pt.groups]) return hipSuccess;
   pt.per_xcd = (pt.start[pt.groups] + 7) / 8;
   const dim3 grid(8 * pt.per_xcd * pt.same);
-  if (rows == RT_ROWS_SMALL)
-    hipLaunchKernelGGL((rt_sweep_tile_kernel<RT_R_SMALL, RT_ROWS_SMALL / RT_R_SMALL>), grid,
+  if (rows == RT_ROWS_SMALL && P == RT_TILE_PLANES_THIN)
+    hipLaunchKernelGGL((rt_sweep_tile_kernel<RT_R_SMALL, RT_ROWS_SMALL / RT_R_SMALL, true>), grid,
+                       dim3(64 * RT_ROWS_SMALL / RT_R_SMALL), 0, st, I, kap, S, kap_y, S_y, rays,
+                       pt, p0, P, ray_stride, part);
+  else if (rows == RT_ROWS_SMALL)
+    hipLaunchKernelGGL((rt_sweep_tile_kernel<RT_R_SMALL, RT_ROWS_SMALL / RT_R_SMALL, false>), grid,
                        dim3(64 * RT_ROWS_SMALL / RT_R_SMALL), 0, st, I, kap, S, kap_y, S_y, rays,
                        pt, p0, P, ray_stride, part);
   else
-    hipLaunchKernelGGL((rt_sweep_tile_kernel<RT_R, RT_ROWS / RT_R>), grid,
+    hipLaunchKernelGGL((rt_sweep_tile_kernel<RT_R, RT_ROWS / RT_R, false>), grid,
                        dim3(64 * RT_ROWS / RT_R), 0, st, I, kap, S, kap_y, S_y, rays, pt, p0, P,
                        ray_stride, part);
   return hipGetLastError();
