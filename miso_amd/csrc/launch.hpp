@@ -129,21 +129,21 @@ hipError_t launch_rt_sweep_plane(hipStream_t, double *, const double *, const do
                                  const double *, const double *, const RtRays &, int, int, long,
                                  int, unsigned *);
 hipError_t launch_rt_transpose_xy(hipStream_t, const double *, double *, int, int, int);
-// The patched sweep: RT_TILE_PLANES planes per launch (4, 6, 8 and 10:
-// 17.4, 17.0, 17.0, 17.3 ms for a radiative step of 256^3 and 9.2, 8.6, 8.3,
-// 8.5 ms for a cold solve of 211 x 150 x 187; three iterations of that solve in
-// two planes a launch 5.8 ms, in eight 3.9), or RT_TILE_PLANES_THIN
-// where an axis' launch has few workgroups and its rays so few nodes along c
-// that a short patch holds them and nothing but columns repeats (three
+// The patched sweep: RT_TILE_PLANES planes per launch (4, 6, 8 and 10: 17.4,
+// 17.0, 17.0, 17.3 ms for a radiative step of 256^3 and 9.2, 8.6, 8.3, 8.5 ms
+// for a cold solve of 211 x 150 x 187; three iterations of that solve in two
+// planes a launch 5.8 ms, in eight 3.9), or RT_TILE_PLANES_THIN where a short
+// patch holds the c axis of an axis' rays and nothing but columns repeats (three
 // iterations in 8 and 16 planes: 300 x 300 x 2 1.90 and 0.97 ms, 384^2 x 6 2.52
-// and 1.44, 1024 x 16 x 16 6.0 and 5.1); in patches of 64 x
-// RT_ROWS nodes (48 rows: 17.0 ms for 16.0 and 8.2 for 7.6; 36 of three a wave
-// 16.8 and 8.3); of 64 x RT_ROWS_SMALL where an axis' launch would have fewer
-// than RT_FEW workgroups, so that a thin slab's x and y rays, two patches
-// high, reach the CUs that whole patches leave idle (slab solve of 384^2 x
-// 27: 4.44 -> 3.56 ms; 16 rows, three patches high, 3.68; at 256^3, where the
-// chip is full either way, the short patches' repeated rows make 19.1 ms of
-// 17.0; a limit of 256 sends a 211 x 150 x 187 box there: 8.1 ms for 7.6).
+// and 1.44, 1024 x 16 x 16 6.0 and 5.1, 1500 x 300 x 7 12.7 and 5.5, 900 x 800 x
+// 18 11.3 and 10.7).  Patches have 64 x RT_ROWS nodes (48 rows: 17.0 ms for 16.0
+// and 8.2 for 7.6; 36 of three a wave 16.8 and 8.3), or 64 x RT_ROWS_SMALL for
+// thin rays and where an axis' launch would have fewer than RT_FEW workgroups,
+// so that a thin slab's x and y rays, two patches high, reach the CUs that whole
+// patches leave idle (slab solve of 384^2 x 27: 4.44 -> 3.56 ms; 16 rows, three
+// patches high, 3.68; at 256^3, where the chip is full either way, the short
+// patches' repeated rows make 19.1 ms of 17.0; a limit of 256 sends a 211 x 150 x
+// 187 box there: 8.1 ms for 7.6).
 // The first patch of an axis starts on the upwind boundary and owns size - 1
 // nodes, the others start P nodes before the size - P they own.
 constexpr int RT_TILE_PLANES = 8, RT_TILE_PLANES_THIN = 16;

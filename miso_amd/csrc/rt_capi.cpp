@@ -257,14 +257,14 @@ int misohip_rt_solve(misohip_ctx *ctx, const misohip_grid *g, const misohip_rt_c
     ch.blocks += (long)rt_patches(R.nb, 64, RT_TILE_PLANES) *
                  rt_patches(R.nc, RT_ROWS, RT_TILE_PLANES);
   }
-  // chains of few workgroups take shorter patches, and share their launches
-  // where these are alike
+  // chains of thin rays and of few workgroups take shorter patches, and the
+  // latter share their launches where these are alike
   std::vector<Chain> chains;
   for (Chain &ch : axes) {
     const bool full = ch.blocks >= RT_FEW;
     if (ch.cones) ch.P = RT_MULTI_PLANES;
-    else if (full) ch.rows = RT_ROWS;
     else if (ch.max_nc < ch.rows) ch.P = RT_TILE_PLANES_THIN;
+    else if (full) ch.rows = RT_ROWS;
     Chain *to = nullptr;
     if (!full && !ch.cones)
       for (Chain &c : chains)

@@ -168,7 +168,8 @@ def _equal_to_plane_sweep(ctx, sizes, rays, kinds, max_iters):
 # and narrower than the box, and of one ray
 @pytest.mark.gpu
 @pytest.mark.parametrize("sizes,rays", [((300, 40, 2), 24), ((131, 70, 19), 24), ((131, 70, 18), 24),
-                                        ((70, 16, 16), 24), ((16, 150, 12), 24), ((90, 2, 35), 1)])
+                                        ((70, 16, 16), 24), ((16, 150, 12), 24), ((90, 2, 35), 1),
+                                        ((1100, 900, 3), 24)])
 def test_thin_boxes_equal_the_plane_sweep(ctx, sizes, rays):
     _equal_to_plane_sweep(ctx, sizes, rays, ((16, True), (2, True)), 6)
 
