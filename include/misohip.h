@@ -169,11 +169,11 @@ typedef struct misohip_work {
 } misohip_work;
 
 /* Context: device ordinal and the HIP stream every call is ordered on
- * (NULL = the null stream).  Creates no stream at creation; the first
- * misohip_rt_solve with rays along more than one sweep axis creates two more
- * (default priority) for the multi-plane sweeps, forked from and joined back
- * to the context's stream with events inside each iteration, and
- * misohip_destroy frees it. */
+ * (NULL = the null stream).  Creates no stream at creation; a
+ * misohip_rt_solve whose sweep axes take launches of their own creates one or
+ * two more (default priority) for all but the first of them, forked from and
+ * joined back to the context's stream with events inside each iteration, and
+ * misohip_destroy frees them. */
 int misohip_create(int device, void *stream, misohip_ctx **out);
 int misohip_destroy(misohip_ctx *ctx);
 int misohip_set_stream(misohip_ctx *ctx, void *stream);

@@ -76,19 +76,22 @@ constexpr int MLP_X_TALL = 128;
 // X and the activations (aT), the pre-activation gradients (dT); and the
 // hidden layers' pre-activations in FP32, which the lane that wrote them
 // reads again.
-// Bound by the weights' way from L2 into the CU (64 bytes a clock): 1.24 MB
-// forward and 0.46 back for 1536-256-256-256-384.
 // NT = 1 (16 waves) spreads a batch of 1024 over 64 CUs; NT = 4 (eight waves,
 // two workgroups a CU) reads the weights a quarter as often, for large
 // batches of inference (NT = 2: 736 us for 635 at 147456 columns; four waves
 // of twice the row tiles 680; three row tiles a wave spill: 994; features of
 // X by 256, one workgroup a CU: 850).
-// At that size and a batch of 1024 a training step's chain takes 34 us, where
-// a launch per layer, product and elementwise step (128 x 128 tiles: 16
-// workgroups) took 232; 147456 columns of inference, their Q_rad field
-// included, 640 us for 957 (without
-// its 1.1 GB of Y, corrections and Q_rad it would take 363).  Every sum is
-// taken in the order of k, 32 at a time, as those took it: the same bits.
+// A training step's chain at a batch of 1024 and 1536-256-256-256-384 is bound
+// by latency: seven layers of 4 to 5 us (first weights, code that runs a few
+// times, the barrier; waves wait in 55 % of their cycles), with 117 MB from L2
+// in 34 us a third of what the 64 CUs could take, and VALU issue at 8 %.  A
+// launch per layer, product and elementwise step (128 x 128 tiles: 16
+// workgroups) took 232.  147456 columns of inference, their Q_rad field
+// included, are bound by HBM: 2.2 GB in 622 us, 957 before (without its 1.1 GB
+// of Y, corrections and Q_rad it would take 363).  Sums go in the order of k, 32
+// to an instruction; the 32 x 32 x 16 products before, 16 to an instruction,
+// gave the same bits at every size compared (outputs, gradients and weights of
+// hidden widths 32 to 4096 at batches of 1 to 16384).
 template <int NT, int WAVES, int RT, int PD, bool TRAIN, bool WIDE>
 __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
     MlpNet net, const uint16_t *__restrict__ X, int M,
@@ -416,10 +419,10 @@ __global__ __launch_bounds__(64 * WAVES, 4) void mlp_chain_kernel(
 // (a sixteenth of the batch where that divides), so that no chain of
 // additions grows with the batch, and these sums are added in order; a bias
 // is 16 sums, of every 16th column each, added in order.
-// Bound by the operands' way from L2 (64 bytes a clock and CU): 80 MB at a
-// batch of 1024 and 1536-256-256-256-384: 8.2 us, where a launch per layer
-// that transposed through LDS, its partial sums in memory and column sums by
-// four workgroups took 134.
+// Bound by latency, with a wave for two SIMDs in three (644): 82 MB from L2 in
+// 8.2 us at a batch of 1024 and 1536-256-256-256-384, a quarter of 64 bytes a
+// clock and CU, where a launch per layer that transposed through LDS, its
+// partial sums in memory and column sums by four workgroups took 134.
 __global__ __launch_bounds__(64) void mlp_wgrad_kernel(MlpNet net, int SB, int per,
                                                        int tiles) {
   const int lane = threadIdx.x, row = lane & 15, kq = lane >> 4;

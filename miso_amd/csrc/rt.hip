@@ -255,8 +255,11 @@ hipError_t launch_rt_sweep_multi(hipStream_t st, double *I, const double *kap, c
 // writes it) or, in the patches after the first, P columns and rows of the
 // neighbouring patch, computed again: step s leaves the first s of them
 // stale, so the columns and rows from P on are right after P planes, and
-// only those are stored.  No workgroup reads what another one of the launch
-// writes.
+// only those are stored.  No workgroup uses what another one of the launch
+// writes: the plane before p0 is not written, and of the planes after it a
+// patch uses the old intensities of owned and boundary nodes alone (patches
+// with a boundary on one side load those of the overlap on the other as well,
+// while the neighbour stores there, and drop them).
 // Three register sets hold the plane before, the current plane's kappa, S
 // and old intensities, and the next plane's, in flight meanwhile.
 // The four rays that go the same way along the planes read the same kappa
@@ -265,11 +268,13 @@ hipError_t launch_rt_sweep_multi(hipStream_t st, double *I, const double *kap, c
 // are neighbours.
 // rt_node forms each value from the same operands as rt_sweep_plane_kernel:
 // the same bits.
-// Bound by VALU issue (84 instructions a node and 1.4 x the nodes, for the
-// repeated columns and rows) and, at the large sizes, HBM: a launch per plane
-// read the plane before again, kappa and S once per ray, and moved 41 bytes
-// a node and ray; this 26.  At 256^3 an iteration's sweeps take 3.0 ms of
-// 5.2, radiative step 23.4 -> 17.0 ms, cold solve of 211 x 150 x 187 14.2 ->
+// No rate bounds it alone: at 256^3, where an iteration's sweeps take 3.0 ms
+// of 5.2, VALU issue is at half of its rate (84 instructions for each of 1.72 x
+// the nodes, for the repeated columns and rows; 1.55 to 1.75 along the axes of
+// 211 x 150 x 187) and 4.1 TB/s pass the L2, 30 bytes a node and ray; the rest is
+// the latency of a plane's FP64 chain, with four waves a SIMD to cover it.  A
+// launch per plane read the plane before again, and kappa and S once per ray.
+// Radiative step of 256^3 23.4 -> 17.0 ms, cold solve of 211 x 150 x 187 14.2 ->
 // 8.2 ms.  (Tiles marched in wavefront order, which repeat nothing, read
 // kappa and S once per ray and start and end with an idle chip: 19.4 and
 // 10.6 ms.)
